@@ -787,15 +787,29 @@ int build_tables(nyxpm_ctx* c) {
             s.coff = c->boxes[b].cell_off;
             s.nblk = std::min(s.nblk, kReduceBlocks);
             vr.push_back(s);
-            // z-marching residual: kResTX x kResTY columns, chunks of up to 64 planes
-            const Level& L = c->boxes[b].lev[0];
-            CellSeg z = mk(b, 0, 1);
-            z.coff = c->boxes[b].cell_off;
-            const int nbx = (L.n[0] + kResTX - 1) / kResTX, nby = (L.n[1] + kResTY - 1) / kResTY;
-            z.zchunk = std::min(64, L.n[2]);
-            z.nblk = nbx * nby * ((L.n[2] + z.zchunk - 1) / z.zchunk);
-            vz.push_back(z);
         }
+        // z-marching residual: kResTX x kResTY columns in chunks of 64 planes, halved
+        // down to 4 while the launch has fewer than two blocks per CU (a block of 64
+        // planes is a serial chain of ~25-60 us: at 32^3 two blocks took 25 us, 16 of
+        // 4 planes take 7; a chunk re-reads two planes, so 512^3, with 2048 blocks
+        // already, keeps 64)
+        auto res_pieces = [&](int zc) {
+            vz.clear();
+            long long blocks = 0;
+            for (int b = 0; b < nbox; ++b) {
+                const Level& L = c->boxes[b].lev[0];
+                CellSeg z = mk(b, 0, 1);
+                z.coff = c->boxes[b].cell_off;
+                const int nbx = (L.n[0] + kResTX - 1) / kResTX, nby = (L.n[1] + kResTY - 1) / kResTY;
+                z.zchunk = std::min(zc, L.n[2]);
+                z.nblk = nbx * nby * ((L.n[2] + z.zchunk - 1) / z.zchunk);
+                blocks += z.nblk;
+                vz.push_back(z);
+            }
+            return blocks;
+        };
+        int rzc = 64;
+        while (res_pieces(rzc) < 512 && rzc > 4) rzc /= 2;
         c->t_res = add_table(vr);
         c->t_resz = add_table(vz);
     }
