@@ -1037,37 +1037,227 @@ __global__ void __launch_bounds__(kBlock) k_bottom(const CellSeg* segs, int nseg
 
 // The coarse end of a V-cycle in one workgroup per box: every level from the
 // first one with at most kCoarseCells cells (segs[first[b]], "top") down to the
-// bottom (segs[first[b+1]-1]), and back up.  Corrections e of all these levels
-// and residuals r of the levels below the top live in LDS; the top's r is read
-// from the pool and the top's final e is written to the pool (buffer e), where
-// the prolongation of the next finer level finds it.  Per cell the arithmetic is
-// that of k_fill, k_gsrb_half, k_resid_restrict, k_bottom and k_prolong, in the
-// same order, so the result equals those launches bit for bit; what it saves is
-// ~30 latency-bound launches per cycle.
+// bottom (segs[first[b+1]-1]), and back up.  Per cell the arithmetic is that of
+// k_fill, k_gsrb_half, k_resid_restrict, k_bottom and k_prolong, in the same
+// order, so the result equals those launches bit for bit; what it saves is ~30
+// latency-bound launches per cycle.
+//
+// One workgroup is a serial chain of ~35 steps, each a few LDS reads, a
+// dependent update and a barrier, so the kernel is bound by the latency of a
+// step.  A level's cells belong to threads as pairs of x-adjacent cells (pair q =
+// cells 2q, 2q+1, one red and one black), whose e and r stay in registers for the
+// whole cycle and whose neighbour addresses are computed once; LDS holds one e
+// array per colour, indexed by pair, only to pass values between threads (an
+// update reads five consecutive-lane words: the sixth neighbour is the pair's
+// other cell).  The residual is formed by the cells' owners, passed through the
+// same arrays and summed by the coarse cells' owners.  Measured in a solve's
+// V-cycles, 16^3 top: 36 -> 15 us FP64, 35 -> 13 us FP32 against a version that kept
+// e and r in LDS and derived every index by division.
+//
+// At most three smoothing levels fit below kCoarseCells (each coarsening divides
+// the cells by 8 and the bottom has at least 8): at most kCoarseCells / 2 pairs on
+// the top (two per thread), kCoarseCells / 16 and kCoarseCells / 128 below.
 constexpr int kCoarseCells = 4096;
 constexpr int kCoarseThreads = 1024;
+constexpr int kBottomStage = 1024;  // bottom cells up to which G is staged in LDS
 
-template <typename T>
-__device__ __forceinline__ void coarse_half(const CellSeg& sg, T* E, const T* R, int colour) {
-    const int nx = sg.n[0], ny = sg.n[1], nz = sg.n[2];
-    const int hx = nx >> 1;
-    const int nh = hx * ny * nz;
-    const T dhx = T(sg.dh[0]), dhy = T(sg.dh[1]), dhz = T(sg.dh[2]);
-    const T gamma = T(sg.gamma), inv_gamma = T(sg.inv_gamma);
-    for (int q = threadIdx.x; q < nh; q += blockDim.x) {
-        const int ih = q % hx;
-        const int t = q / hx;
-        const int j = t % ny, k = t / ny;
-        const int i = 2 * ih + ((j + k + colour) & 1);
-        int im = i == 0 ? nx - 1 : i - 1, ip = i == nx - 1 ? 0 : i + 1;
-        int jm = j == 0 ? ny - 1 : j - 1, jp = j == ny - 1 ? 0 : j + 1;
-        int km = k == 0 ? nz - 1 : k - 1, kp = k == nz - 1 ? 0 : k + 1;
-        const int c = (k * ny + j) * nx + i;
-        E[c] = gs_update(E[c], R[c], E[(k * ny + j) * nx + im] + E[(k * ny + j) * nx + ip],
-                         E[(k * ny + jm) * nx + i] + E[(k * ny + jp) * nx + i],
-                         E[(km * ny + j) * nx + i] + E[(kp * ny + j) * nx + i], gamma, inv_gamma, dhx, dhy, dhz);
+// q / d for 0 <= q < 4096, inv = 1 / d in FP32: (q + 1/2) / d lies at least 1 / (2d)
+// from an integer, the product's error is below 1e-3 / d.  (A 32-bit integer
+// division is ~25 instructions, each 16 cycles with 16 waves on one CU.)
+__device__ __forceinline__ int small_div(int q, float inv) { return (int)(((float)q + 0.5f) * inv); }
+
+// One smoothing level as its threads hold it (NP pairs per thread).
+template <typename T, int NP>
+struct CoarseLevel {
+    int np = 0;                        // pairs of the level
+    int hx = 0, ny = 0;                // pairs per row, rows per plane
+    float ihx, iny;                    // 1/hx, 1/ny
+    T *sr = nullptr, *sb = nullptr;    // LDS: red and black e by pair
+    T dhx, dhy, dhz, gamma, inv_gamma;
+    int xm[NP], xp[NP], ym[NP], yp[NP], zm[NP], zp[NP];  // neighbour pairs
+    int par[NP];                       // parent cell: index in the coarse level
+    bool c[NP];                        // the red cell is the pair's second
+    T er[NP], eb[NP], fr[NP], fb[NP];  // e and r of the red and the black cell
+
+    __device__ __forceinline__ void setup(const CellSeg& sg, T* lds) {
+        const int nx = sg.n[0], nz = sg.n[2];
+        ny = sg.n[1];
+        hx = nx >> 1;
+        np = hx * ny * nz;
+        sr = lds;
+        sb = lds + np;
+        dhx = T(sg.dh[0]);
+        dhy = T(sg.dh[1]);
+        dhz = T(sg.dh[2]);
+        gamma = T(sg.gamma);
+        inv_gamma = T(sg.inv_gamma);
+        ihx = 1.0f / (float)hx;
+        iny = 1.0f / (float)ny;
+#pragma unroll
+        for (int u = 0; u < NP; ++u) {
+            if (!has(u)) continue;
+            const int q = pair(u);
+            int m, j, k;
+            coords(q, m, j, k);
+            const int pl = hx * ny;
+            xm[u] = m == 0 ? q + hx - 1 : q - 1;
+            xp[u] = m == hx - 1 ? q - (hx - 1) : q + 1;
+            ym[u] = j == 0 ? q + (ny - 1) * hx : q - hx;
+            yp[u] = j == ny - 1 ? q - (ny - 1) * hx : q + hx;
+            zm[u] = k == 0 ? q + (nz - 1) * pl : q - pl;
+            zp[u] = k == nz - 1 ? q - (nz - 1) * pl : q + pl;
+            c[u] = (j + k) & 1;
+            par[u] = ((k >> 1) * (ny >> 1) + (j >> 1)) * hx + m;
+            er[u] = eb[u] = fr[u] = fb[u] = T(0);
+        }
     }
-}
+    // pair q = (k * ny + j) * hx + m
+    __device__ __forceinline__ void coords(int q, int& m, int& j, int& k) const {
+        const int t = small_div(q, ihx);
+        m = q - t * hx;
+        k = small_div(t, iny);
+        j = t - k * ny;
+    }
+    __device__ __forceinline__ bool has(int u) const { return (int)threadIdx.x + u * kCoarseThreads < np; }
+    __device__ __forceinline__ int pair(int u) const { return (int)threadIdx.x + u * kCoarseThreads; }
+    // r of the pair's first and second cell
+    __device__ __forceinline__ void set_r(int u, T a, T b) {
+        fr[u] = c[u] ? b : a;
+        fb[u] = c[u] ? a : b;
+    }
+    __device__ __forceinline__ void load_r(const T* R) {
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (has(u)) set_r(u, R[2 * pair(u)], R[2 * pair(u) + 1]);
+    }
+    __device__ __forceinline__ void load_e(const T* E) {
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (has(u)) {
+                const T a = E[2 * pair(u)], b = E[2 * pair(u) + 1];
+                er[u] = c[u] ? b : a;
+                eb[u] = c[u] ? a : b;
+            }
+    }
+    __device__ __forceinline__ void store_e(T* E) const {
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (has(u)) {
+                E[2 * pair(u)] = c[u] ? eb[u] : er[u];
+                E[2 * pair(u) + 1] = c[u] ? er[u] : eb[u];
+            }
+    }
+    __device__ __forceinline__ void publish() const {
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (has(u)) {
+                sr[pair(u)] = er[u];
+                sb[pair(u)] = eb[u];
+            }
+        __syncthreads();
+    }
+    // one red-black sweep from the published values (from_zero: e is zero and was
+    // not published: the red step uses literal zeros)
+    __device__ __forceinline__ void sweep(bool from_zero) {
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (has(u)) {
+                T sx = T(0) + T(0), sy = sx, sz = sx;
+                if (!from_zero) {
+                    sx = eb[u] + sb[c[u] ? xp[u] : xm[u]];
+                    sy = sb[ym[u]] + sb[yp[u]];
+                    sz = sb[zm[u]] + sb[zp[u]];
+                }
+                er[u] = gs_update(er[u], fr[u], sx, sy, sz, gamma, inv_gamma, dhx, dhy, dhz);
+                sr[pair(u)] = er[u];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (has(u)) {
+                eb[u] = gs_update(eb[u], fb[u], er[u] + sr[c[u] ? xm[u] : xp[u]], sr[ym[u]] + sr[yp[u]],
+                                  sr[zm[u]] + sr[zp[u]], gamma, inv_gamma, dhx, dhy, dhz);
+                sb[pair(u)] = eb[u];
+            }
+        __syncthreads();
+    }
+    // the residual r - L e (lap7's arithmetic) of every cell into the LDS arrays,
+    // first cells in sr, second cells in sb (e itself stays in the registers)
+    __device__ __forceinline__ void publish_residual() {
+        T ra[NP], rb[NP];
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (has(u)) {
+                const T a = c[u] ? eb[u] : er[u], b = c[u] ? er[u] : eb[u];
+                const T fa = c[u] ? fb[u] : fr[u], f2 = c[u] ? fr[u] : fb[u];
+                const T* oa = c[u] ? sr : sb;  // the colour of a's neighbours
+                const T* ob = c[u] ? sb : sr;
+                const T ax = dhx * (oa[xm[u]] - T(2) * a + b), bx = dhx * (a - T(2) * b + ob[xp[u]]);
+                const T ay = dhy * (oa[ym[u]] - T(2) * a + oa[yp[u]]), by = dhy * (ob[ym[u]] - T(2) * b + ob[yp[u]]);
+                const T az = dhz * (oa[zm[u]] - T(2) * a + oa[zp[u]]), bz = dhz * (ob[zm[u]] - T(2) * b + ob[zp[u]]);
+                ra[u] = fa - (ax + ay + az);
+                rb[u] = f2 - (bx + by + bz);
+            }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (has(u)) {
+                sr[pair(u)] = ra[u];
+                sb[pair(u)] = rb[u];
+            }
+        __syncthreads();
+    }
+    // restriction of the published residual to coarse cell (I, J, K): the 8
+    // children summed k, j, i
+    __device__ __forceinline__ T restricted(int I, int J, int K) const {
+        T acc = T(0);
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk)
+#pragma unroll
+            for (int jj = 0; jj < 2; ++jj) {
+                const int p = ((2 * K + kk) * ny + 2 * J + jj) * hx + I;
+                acc += sr[p];
+                acc += sb[p];
+            }
+        return T(0.125) * acc;
+    }
+    // r of this level from the finer level's published residual
+    template <int NF>
+    __device__ __forceinline__ void restrict_from(const CoarseLevel<T, NF>& f) {
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (has(u)) {
+                int m, j, k;
+                coords(pair(u), m, j, k);
+                set_r(u, f.restricted(2 * m, j, k), f.restricted(2 * m + 1, j, k));
+            }
+    }
+    // down: sweeps from zero (or from e as loaded), the residual published
+    __device__ __forceinline__ void down(int nu1, bool zero) {
+        if (!zero) publish();
+        for (int it = 0; it < nu1; ++it) sweep(zero && it == 0);
+        publish_residual();
+    }
+    // up: e += the parent cell's value, sweeps
+    template <class F>
+    __device__ __forceinline__ void up(int nu2, F parent) {
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (has(u)) {
+                const T cv = parent(par[u]);
+                er[u] = er[u] + cv;
+                eb[u] = eb[u] + cv;
+            }
+        publish();
+        for (int it = 0; it < nu2; ++it) sweep(false);
+    }
+    // e of a cell of this level as published
+    __device__ __forceinline__ T cell(int q) const {
+        int m, j, k;
+        coords(q >> 1, m, j, k);
+        return ((q + j + k) & 1 ? sb : sr)[q >> 1];
+    }
+};
 
 template <typename T>
 __global__ void __launch_bounds__(kCoarseThreads) k_coarse_vcycle(const CellSeg* segs, const int* first,
@@ -1076,116 +1266,96 @@ __global__ void __launch_bounds__(kCoarseThreads) k_coarse_vcycle(const CellSeg*
                                                                   const double* __restrict__ G, int nu1, int nu2,
                                                                   int keep_top) {
     extern __shared__ double coarse_smem[];
-    T* lds = reinterpret_cast<T*>(coarse_smem);
     const int l0 = first[blockIdx.x], l1 = first[blockIdx.x + 1];
-    if (!active[segs[l0].box]) return;
-    const int nl = l1 - l0;
-    auto ncell = [&](int l) { return segs[l].n[0] * segs[l].n[1] * segs[l].n[2]; };
-    // LDS: e of levels l0..l1-1, then r of levels l0+1..l1-1
-    auto eoff = [&](int l) {
-        int o = 0;
-        for (int q = l0; q < l; ++q) o += ncell(q);
-        return o;
-    };
-    auto roff = [&](int l) {
-        int o = eoff(l1);
-        for (int q = l0 + 1; q < l; ++q) o += ncell(q);
-        return o;
-    };
-    auto rptr = [&](int l) -> const T* { return l == l0 ? r + segs[l0].off : lds + roff(l); };
-    const int tid = threadIdx.x, nth = blockDim.x;
+    const CellSeg& top = segs[l0];
+    if (!active[top.box]) return;
+    const int ns = l1 - 1 - l0;  // smoothing levels (0: the bottom alone)
+    const CellSeg& bs = segs[l1 - 1];
+    const int nbx = bs.n[0], nby = bs.n[1], nbz = bs.n[2];
+    const int nb = nbx * nby * nbz;
+    const int tid = threadIdx.x;
+    // LDS: the bottom's r (FP64), its G where staged, its e, then the levels' arrays
+    double* rb = coarse_smem;
+    const bool stage = nb <= kBottomStage;
+    double* gl = rb + nb;
+    T* ebot = reinterpret_cast<T*>(gl + (stage ? nb : 0));
+    T* lds = ebot + nb;
+    const double* Gb = G + bs.coff;
+    CoarseLevel<T, 2> L0;
+    CoarseLevel<T, 1> L1, L2;
+    if (ns > 0) {
+        L0.setup(top, lds);
+        L0.load_r(r + top.off);
+    }
+    if (stage && tid < nb) gl[tid] = Gb[tid];
+    if (ns > 1) L1.setup(segs[l0 + 1], lds + 2 * L0.np);
+    if (ns > 2) L2.setup(segs[l0 + 2], lds + 2 * L0.np + 2 * L1.np);
     // down: zero guess (keep_top: on the box's own level, the e of the previous
     // V-cycle of the same refinement step), nu1 red-black sweeps, residual
     // restricted to the next level
-    for (int l = l0; l + 1 < l1; ++l) {
-        const CellSeg& sg = segs[l];
-        T* E = lds + eoff(l);
-        const T* R = rptr(l);
-        const int nc = ncell(l);
-        const bool keep = keep_top && l == l0 && sg.lev == 0;
-        const T* Eg = e + sg.off;
-        for (int q = tid; q < nc; q += nth) E[q] = keep ? Eg[q] : T(0);
-        __syncthreads();
-        for (int it = 0; it < nu1; ++it)
-            for (int col = 0; col < 2; ++col) {
-                coarse_half(sg, E, R, col);
-                __syncthreads();
-            }
-        const int nx = sg.n[0], ny = sg.n[1], nz = sg.n[2];
-        const int cx = nx >> 1, cy = ny >> 1, cz = nz >> 1;
-        const T dhx = T(sg.dh[0]), dhy = T(sg.dh[1]), dhz = T(sg.dh[2]);
-        T* Rc = lds + roff(l + 1);
-        for (int q = tid; q < cx * cy * cz; q += nth) {
-            const int I = q % cx;
-            const int t = q / cx;
-            const int J = t % cy, K = t / cy;
-            T acc = T(0);
-            for (int kk = 0; kk < 2; ++kk)
-                for (int jj = 0; jj < 2; ++jj)
-                    for (int ii = 0; ii < 2; ++ii) {
-                        const int i = 2 * I + ii, j = 2 * J + jj, k = 2 * K + kk;
-                        T rc = R[(k * ny + j) * nx + i] - lap7(E, i, j, k, nx, ny, nz, dhx, dhy, dhz);
-                        acc += rc;
-                    }
-            Rc[q] = T(0.125) * acc;
-        }
-        __syncthreads();
+    if (ns > 0) {
+        const bool keep = keep_top && top.lev == 0;
+        if (keep) L0.load_e(e + top.off);
+        L0.down(nu1, !keep);
+    }
+    if (ns > 1) {
+        L1.restrict_from(L0);
+        L1.down(nu1, true);
+    }
+    if (ns > 2) {
+        L2.restrict_from(L1);
+        L2.down(nu1, true);
     }
     // bottom: e = G * r (periodic convolution, natural order), FP64 in both
     // precisions as in k_bottom
+    for (int q = tid; q < nb; q += kCoarseThreads) {
+        const int I = q % nbx, t = q / nbx;
+        const int J = t % nby, K = t / nby;
+        rb[q] = (double)(ns == 0   ? r[bs.off + q]
+                         : ns == 1 ? L0.restricted(I, J, K)
+                         : ns == 2 ? L1.restricted(I, J, K)
+                                   : L2.restricted(I, J, K));
+    }
+    __syncthreads();
     {
-        const int lb = l1 - 1;
-        const CellSeg& sg = segs[lb];
-        const int nx = sg.n[0], ny = sg.n[1], nz = sg.n[2];
-        const int nc = nx * ny * nz;
-        const T* R = rptr(lb);
-        const double* Gb = G + sg.coff;
-        T* E = lds + eoff(lb);
-        for (int c = tid; c < nc; c += nth) {
-            const int cx = c % nx, cy = (c / nx) % ny, cz = c / (nx * ny);
+        const double* g = stage ? gl : Gb;
+        for (int q = tid; q < nb; q += kCoarseThreads) {
+            const int cx = q % nbx, t = q / nbx;
+            const int cy = t % nby, cz = t / nby;
             double acc = 0.0;
-            for (int qz = 0; qz < nz; ++qz) {
-                int dz = cz - qz; dz = dz < 0 ? dz + nz : dz;
-                for (int qy = 0; qy < ny; ++qy) {
-                    int dy = cy - qy; dy = dy < 0 ? dy + ny : dy;
-                    for (int qx = 0; qx < nx; ++qx) {
-                        int dxx = cx - qx; dxx = dxx < 0 ? dxx + nx : dxx;
-                        acc += Gb[(dz * ny + dy) * nx + dxx] * (double)R[(qz * ny + qy) * nx + qx];
+            for (int qz = 0; qz < nbz; ++qz) {
+                int dz = cz - qz; dz = dz < 0 ? dz + nbz : dz;
+                for (int qy = 0; qy < nby; ++qy) {
+                    int dy = cy - qy; dy = dy < 0 ? dy + nby : dy;
+                    const double* gr = g + (dz * nby + dy) * nbx;
+                    const double* rr = rb + (qz * nby + qy) * nbx;
+                    for (int qx = 0; qx < nbx; ++qx) {
+                        int dxx = cx - qx; dxx = dxx < 0 ? dxx + nbx : dxx;
+                        acc += gr[dxx] * rr[qx];
                     }
                 }
             }
-            E[c] = T(acc);
+            if (ns == 0)
+                e[bs.off + q] = T(acc);
+            else
+                ebot[q] = T(acc);
         }
-        __syncthreads();
     }
+    if (ns == 0) return;
+    __syncthreads();
     // up: piecewise-constant prolongation, nu2 red-black sweeps
-    for (int l = l1 - 2; l >= l0; --l) {
-        const CellSeg& sg = segs[l];
-        T* E = lds + eoff(l);
-        const T* Ec = lds + eoff(l + 1);
-        const int nx = sg.n[0], ny = sg.n[1], nz = sg.n[2];
-        const int nc = nx * ny * nz;
-        for (int q = tid; q < nc; q += nth) {
-            const int i = q % nx;
-            const int t = q / nx;
-            const int j = t % ny, k = t / ny;
-            E[q] = E[q] + Ec[((k >> 1) * (ny >> 1) + (j >> 1)) * (nx >> 1) + (i >> 1)];
-        }
-        __syncthreads();
-        const T* R = rptr(l);
-        for (int it = 0; it < nu2; ++it)
-            for (int col = 0; col < 2; ++col) {
-                coarse_half(sg, E, R, col);
-                __syncthreads();
-            }
+    auto bottom = [&](int q) { return ebot[q]; };
+    if (ns > 2) {
+        L2.up(nu2, bottom);
+        L1.up(nu2, [&](int q) { return L2.cell(q); });
+    } else if (ns > 1) {
+        L1.up(nu2, bottom);
     }
-    {
-        T* Eg = e + segs[l0].off;
-        const T* E = lds + eoff(l0);
-        const int nc = ncell(l0);
-        for (int q = tid; q < nc; q += nth) Eg[q] = E[q];
-    }
-    (void)nl;
+    if (ns > 1)
+        L0.up(nu2, [&](int q) { return L1.cell(q); });
+    else
+        L0.up(nu2, bottom);
+    L0.store_e(e + top.off);
 }
 
 // Level-0 residual r = f - L phi (FP64), stored as T.  A block owns a TX x TY
@@ -1332,18 +1502,23 @@ __global__ void __launch_bounds__(kBlock) k_update0(const CellSeg* segs, int nse
 //         active = |r0| > target (or fixed_iters > 0)
 //   iter: iters++, active = |r| > target && iters < limit
 // state: [0] resnorm0 [1] rhsnorm [2] final [3] target
-__global__ void k_check(int nbox, int init, int fixed_iters, int max_iter, double rel_tol,
-                        double abs_tol, int* active, int* iters, int* failed,
-                        unsigned long long* nr, unsigned long long* nf, double* state, int inc) {
-    const int b = blockIdx.x * blockDim.x + threadIdx.x;
-    if (b >= nbox) return;
-    unsigned long long br = 0ull, bf = 0ull;
-    for (int q = 0; q < kNormSlots; ++q) {
-        br = max(br, nr[b * kNormSlots + q]);
-        bf = max(bf, nf[b * kNormSlots + q]);
-        nr[b * kNormSlots + q] = 0ull;
-        nf[b * kNormSlots + q] = 0ull;
+// One wave per box: its lanes take the norm slots (one lane reading them in turn
+// was a chain of 64 loads, 5 us a launch).
+__global__ void __launch_bounds__(kWave) k_check(int init, int fixed_iters, int max_iter, double rel_tol,
+                                                 double abs_tol, int* active, int* iters, int* failed,
+                                                 unsigned long long* nr, unsigned long long* nf, double* state,
+                                                 int inc) {
+    static_assert(kNormSlots == kWave, "one lane per norm slot");
+    const int b = blockIdx.x;
+    const int slot = b * kNormSlots + threadIdx.x;
+    unsigned long long br = nr[slot], bf = nf[slot];
+    nr[slot] = 0ull;
+    nf[slot] = 0ull;
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        br = max(br, (unsigned long long)__shfl_xor((long long)br, o));
+        bf = max(bf, (unsigned long long)__shfl_xor((long long)bf, o));
     }
+    if (threadIdx.x != 0) return;
     if (init) {
         const double r0 = __longlong_as_double((long long)br);
         const double fn = __longlong_as_double((long long)bf);

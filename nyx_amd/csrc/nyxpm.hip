@@ -756,15 +756,20 @@ int build_tables(nyxpm_ctx* c) {
         for (int b = 0; b < nbox; ++b) {
             const Box& B = c->boxes[b];
             firsts.push_back((int)vcc.size());
-            long long cells = 0;
+            long long cells = 0;  // e of every level
             for (int l = B.dc; l < B.nlev; ++l) {
                 CellSeg s = mk(b, l, 1);
                 if (l == B.nlev - 1) s.coff = B.G_off;
                 vcc.push_back(s);
-                cells += B.lev[l].nc * (l == B.dc ? 1 : 2);  // e of every level, r below the top
+                cells += B.lev[l].nc;
             }
+            // the bottom's r and, where staged, G in FP64 (a bottom without levels
+            // above it keeps no e)
+            const long long nb = B.lev[B.nlev - 1].nc;
+            const long long fp64 = nb * (nb <= kBottomStage ? 2 : 1);
+            if (B.dc == B.nlev - 1) cells = 0;
             for (int pr = 0; pr < 2; ++pr)
-                c->cc_lds[pr] = std::max(c->cc_lds[pr], (size_t)cells * (pr == 0 ? 8 : 4));
+                c->cc_lds[pr] = std::max(c->cc_lds[pr], (size_t)(fp64 * 8 + cells * (pr == 0 ? 8 : 4)));
         }
         firsts.push_back((int)vcc.size());
         c->t_cc = add_table(vcc);
@@ -1491,8 +1496,8 @@ int update(nyxpm_ctx* c) {
 // inc: the V-cycles run since the previous check (added to the per-box count)
 int check(nyxpm_ctx* c, bool init, int fixed_iters, double rel, double abs_tol, int inc = 1) {
     const int nbox = (int)c->boxes.size();
-    hipLaunchKernelGGL(k_check, dim3(nblocks(nbox, 64)), dim3(64), 0, c->stream, nbox, init ? 1 : 0, fixed_iters,
-                       c->max_iter, rel, abs_tol, c->active, c->iters, c->failed, c->nr, c->nf, c->state, inc);
+    hipLaunchKernelGGL(k_check, dim3(nbox), dim3(kWave), 0, c->stream, init ? 1 : 0, fixed_iters, c->max_iter, rel,
+                       abs_tol, c->active, c->iters, c->failed, c->nr, c->nf, c->state, inc);
     LAUNCHCK(c);
     return NYXPM_OK;
 }

@@ -29,3 +29,45 @@ def test_residual_chunks_bitwise(nyx, orc, n):
     assert it == it2 == 2
     assert np.array_equal(phi, ref)
     assert np.array_equal(norms[:3], st[:3])
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("n", [
+    (16, 16, 16),    # three smoothing levels over a 2^3 bottom, the whole cycle in one workgroup
+    (12, 20, 16),    # two levels, 3 x 5 x 4 bottom
+    (4, 16, 64),     # 2 x 8 x 32 bottom, pairs whose x-neighbours are themselves
+    (10, 14, 6),     # one level, 5 x 7 x 3 bottom
+    (9, 5, 7),       # a bottom alone
+    (14, 12, 13),    # a bottom too large to be staged (2184 cells)
+    (36, 40, 48),    # finer levels above a 9 x 10 x 12 workgroup level
+])
+def test_coarse_workgroup_equals_per_level(nyx, orc, n, precision):
+    # the one-workgroup coarse cycle against one launch per level and step, bit for
+    # bit, from zero, and in FP64 against the oracle (a bottom alone: to rounding,
+    # the library's and the oracle's Green's functions come from two compilers)
+    f = mean_free(n, 33)
+    hi = [v / 32 for v in n]
+    out = []
+    for coarse in ("workgroup", "per_level"):
+        with ctx1(nyx, n, hi=hi, precision=precision, coarse=coarse) as c:
+            out.append(c.solve_poisson(f, fixed_iters=3)[0])
+    assert np.array_equal(out[0], out[1])
+    if precision == "fp64":
+        ref, _, _, _ = orc.mg_solve(n, [1.0 / 32] * 3, f, fixed_iters=3)
+        if any(v % 2 for v in n):
+            assert np.abs(out[0] - ref).max() <= 1e-12 * np.abs(ref).max()
+        else:
+            assert np.array_equal(out[0], ref)
+
+
+def test_coarse_workgroup_keeps_the_correction(nyx):
+    # grouped FP32 cycles continue from the previous correction also where the
+    # whole V-cycle runs in the workgroup (a converged mixed solve, no fixed count)
+    n = (16, 16, 16)
+    f = mean_free(n, 34)
+    out = []
+    for coarse in ("workgroup", "per_level"):
+        with ctx1(nyx, n, precision="mixed", coarse=coarse) as c:
+            out.append(c.solve_poisson(f)[:2])
+    assert out[0][1] == out[1][1]
+    assert np.array_equal(out[0][0], out[1][0])
