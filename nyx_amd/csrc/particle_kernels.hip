@@ -225,9 +225,12 @@ __global__ void __launch_bounds__(kBlock) k_scan_down(const int* __restrict__ co
     if (blockIdx.x == 0 && threadIdx.x == 0) start[n] = bsum[gridDim.x];
 }
 
+// One particle buffer: arrays of one allocation that starts at x (`bytes` long, 0
+// for a buffer not allocated).
 struct PartPtrs {
     double *x, *y, *z, *vx, *vy, *vz, *m;
     int* id;
+    size_t bytes;
 };
 
 // Move every particle to its tile's slot range (order inside a tile is
@@ -1611,6 +1614,92 @@ __global__ void __launch_bounds__(kBlock) k_unsort(long long p0, long long span,
     const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
     if (q >= span || isnan(x[p0 + q])) return;
     out[id[p0 + q]] = in[p0 + q];
+}
+
+// Destinations of a download: x y z vx vy vz in upload order (null: not wanted).
+struct UnsortOut {
+    double* p[6];
+};
+
+// All components of a box's particles to their destinations in upload order, one
+// thread per slot: what the caches hold of the scattered 8-byte writes merges into
+// whole lines while the output is small.
+__global__ void __launch_bounds__(kBlock) k_unsort_all(long long p0, long long span, PartPtrs A, UnsortOut out) {
+    const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
+    if (q >= span) return;
+    const long long p = p0 + q;
+    const double px = A.x[p];
+    if (isnan(px)) return;
+    const int d = A.id[p];
+    if (out.p[0]) out.p[0][d] = px;
+    if (out.p[1]) out.p[1][d] = A.y[p];
+    if (out.p[2]) out.p[2][d] = A.z[p];
+    if (out.p[3]) out.p[3][d] = A.vx[p];
+    if (out.p[4]) out.p[4][d] = A.vy[p];
+    if (out.p[5]) out.p[5][d] = A.vz[p];
+}
+
+// The same in two passes for outputs the caches do not hold: k_pack_records writes
+// each particle's six components as one 64-byte record at its upload index (whole
+// lines instead of six scattered 8-byte writes, each of which costs a line), and
+// k_unpack_records spreads the records over the component arrays in order.  Both
+// go through LDS so that four lanes move a record as 16-byte pieces.
+// Bound by HBM: 60 + 64 B and 64 + 48 B per particle.
+// Measured: see kUnsortDirect.
+constexpr int kRecDoubles = 8;    // doubles per record
+constexpr int kRecStride = 10;    // its stride in LDS (16-byte aligned, spread over the banks)
+__global__ void __launch_bounds__(kBlock) k_pack_records(long long p0, long long span, PartPtrs A,
+                                                         double* __restrict__ rec) {
+    __shared__ __align__(16) double sh[kBlock * kRecStride];
+    __shared__ int sid[kBlock];
+    const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
+    const long long p = p0 + q;
+    int id = -1;
+    if (q < span) {
+        const double px = A.x[p];
+        if (!isnan(px)) {
+            id = A.id[p];
+            double2* s = reinterpret_cast<double2*>(sh + threadIdx.x * kRecStride);
+            s[0] = make_double2(px, A.y[p]);
+            s[1] = make_double2(A.z[p], A.vx[p]);
+            s[2] = make_double2(A.vy[p], A.vz[p]);
+            s[3] = make_double2(0.0, 0.0);
+        }
+    }
+    sid[threadIdx.x] = id;
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        const int r = it * (kBlock / 4) + threadIdx.x / 4, c = threadIdx.x & 3;
+        const int d = sid[r];
+        if (d >= 0)
+            reinterpret_cast<double2*>(rec + (size_t)d * kRecDoubles)[c] =
+                reinterpret_cast<const double2*>(sh + r * kRecStride)[c];
+    }
+}
+
+__global__ void __launch_bounds__(kBlock) k_unpack_records(long long np, const double* __restrict__ rec,
+                                                           UnsortOut out) {
+    __shared__ __align__(16) double sh[kBlock * kRecStride];
+    const long long base = (long long)blockIdx.x * kBlock;
+#pragma unroll
+    for (int it = 0; it < 4; ++it) {
+        const int r = it * (kBlock / 4) + threadIdx.x / 4, c = threadIdx.x & 3;
+        if (base + r < np && c < 3)
+            reinterpret_cast<double2*>(sh + r * kRecStride)[c] =
+                reinterpret_cast<const double2*>(rec + (size_t)(base + r) * kRecDoubles)[c];
+    }
+    __syncthreads();
+    const long long d = base + threadIdx.x;
+    if (d >= np) return;
+    const double2* s = reinterpret_cast<const double2*>(sh + threadIdx.x * kRecStride);
+    const double2 a = s[0], b = s[1], c = s[2];
+    if (out.p[0]) out.p[0][d] = a.x;
+    if (out.p[1]) out.p[1][d] = a.y;
+    if (out.p[2]) out.p[2][d] = b.x;
+    if (out.p[3]) out.p[3][d] = b.y;
+    if (out.p[4]) out.p[4][d] = c.x;
+    if (out.p[5]) out.p[5][d] = c.y;
 }
 
 __global__ void __launch_bounds__(kBlock) k_iota(long long p0, long long np, int* __restrict__ id) {

@@ -71,3 +71,45 @@ def test_coarse_workgroup_keeps_the_correction(nyx):
             out.append(c.solve_poisson(f)[:2])
     assert out[0][1] == out[1][1]
     assert np.array_equal(out[0][0], out[1][0])
+
+
+@pytest.mark.parametrize("npart", [1, 300, 2 ** 18, 2 ** 18 + 77])
+@pytest.mark.parametrize("slack", [0.0, -1.0])
+def test_device_download_equals_host_download(nyx, npart, slack):
+    # downloads into device arrays (directly, or through records above 2^18
+    # particles where the idle buffer holds them) against the host path, for the
+    # second box of a batch, whole and with components left out, also between a
+    # kick-drift and its re-sort (moves waiting in the idle buffer), whose list must
+    # survive
+    import torch
+    r = np.random.default_rng(41)
+    geoms = [nyx.BoxGeom((16, 16, 16)), nyx.BoxGeom((48, 32, 32), (0, 0, 0), (1.5, 1, 1))]
+    with nyx.PMContext(geoms, resort_slack=slack) as c, nyx.PMContext(geoms, resort_slack=slack) as c2:
+        pos = [r.random(npart) * (1.5 if d == 0 else 1.0) for d in range(3)]
+        vel = [r.standard_normal(npart) for _ in range(3)]
+        small = [r.random(500) for _ in range(3)]
+        for q in (c, c2):
+            q.upload(0, small, [np.zeros(500)] * 3, m=r.random(500))
+            q.upload(1, pos, vel, m_const=1.0 / npart)
+            q.pm_init()
+        out = torch.full((6, npart), -7.0, dtype=torch.float64, device="cuda")
+        addr = [out[k].data_ptr() for k in range(6)]
+
+        def check(use):
+            out.fill_(-7.0)
+            torch.cuda.synchronize()
+            c.download_device([a if k in use else None for k, a in enumerate(addr)], box=1)
+            p, v = c.download(1)
+            got = out.cpu().numpy()
+            for k, ref in enumerate(list(p) + list(v)):
+                assert np.array_equal(got[k], ref if k in use else np.full(npart, -7.0))
+
+        check(range(6))
+        c.assign_density(want=False)
+        check(range(6))
+        for q in (c, c2):
+            q.move_kick_drift(1e-3)
+        check((1, 3, 4))
+        check(range(6))
+        assert np.array_equal(c.assign_density(1), c2.assign_density(1))
+        check((0, 5))
