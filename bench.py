@@ -493,7 +493,7 @@ def main():
 
     def smoother_roof(stt, sz):
         """The finest level's smoothing sweep: a full red+black sweep per pass
-        (sweep.d0), or two per pass (sweep2.d0, FP32 levels): then `achieved` is
+        (sweep.d0), or two per pass (sweep2.d0, sweep2_u.d0): then `achieved` is
         the pass's compulsory bytes (e, r in, e out once for both sweeps) per
         time and `per_sweep_equivalent` the bytes of the two single-sweep passes
         it replaces per time."""
@@ -515,17 +515,19 @@ def main():
                     "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                     "bytes_per_launch": int(bb), "mean_launch_ms": e["mean_ms"],
                     **hbm(("fp64:" if sz == 8 else "") + "sweep.d0", e["mean_ms"])}
-        e = stt.get("sweep2.d0")
-        if not e:
+        # FP64 cycles never continue a correction: their pairs start from zero or end in phi
+        key = next((k for k in ("sweep2.d0", "sweep2_u.d0") if stt.get(k)), None)
+        if not key:
             return None
-        bb = kernel_bytes("sweep2.d0", ncell, npart, halo_cells, sz)
+        e = stt[key]
+        bb = kernel_bytes(key, ncell, npart, halo_cells, sz)
         ach = bb / (e["mean_ms"] * 1e-3) / 1e9
-        return {"kernel": "sweep2.d0 (two red+black sweeps in one pass, finest level)", "achieved": round(ach, 1),
+        return {"kernel": f"{key} (two red+black sweeps in one pass, finest level)", "achieved": round(ach, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s", "frac": round(ach / HBM_PEAK_GBS, 4),
                 "bytes_per_launch": int(bb), "mean_launch_ms": e["mean_ms"],
                 "per_sweep_equivalent": {"achieved": round(2 * ach, 1), "frac": round(2 * ach / HBM_PEAK_GBS, 4),
                                          "bytes_of_two_passes": int(2 * bb)},
-                **hbm("sweep2.d0", e["mean_ms"])}
+                **hbm(("fp64:" if sz == 8 else "") + key, e["mean_ms"])}
 
     copy = stream_copy()
     log(f"device copy {copy['gbs']} GB/s")
@@ -663,11 +665,11 @@ def kernel_level(name, grid, n, tuned, sw2_zc=128, only=None):
             nd = n >> d
             if nd < 8:
                 break
-            cfg = (tuned or {}).get(f"sweep2.d{d}")
+            cfg = (tuned or {}).get(("sweep2.fp64" if mt.group(1) == "double" else "sweep2") + f".d{d}")
             if cfg and tuple(cfg["shape"]) != (tx, ty):
                 continue
             zc = min(cfg["zchunk"] if cfg else sw2_zc, nd)
-            if nd % tx == 0 and nd % ty == 0 and (nd // tx) * (nd // ty) * _ceil(nd, zc) * nt == grid:
+            if nd >= tx and nd >= ty and _ceil(nd, tx) * _ceil(nd, ty) * _ceil(nd, zc) * nt == grid:
                 return d
         return None
     mt = re.search(r"k_rb_sweep<(\w+), *(\d+), *(\d+), *(\d+)>", name)

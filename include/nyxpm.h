@@ -133,14 +133,15 @@ typedef struct nyxpm_opts {
                           cycle earlier); 1 = a test after every cycle.
                           Needs nu1 + nu2 even (else 1); FP64 solves and fixed
                           iteration counts always test after every cycle. */
-    int sweep2;        /* FP32 levels with V(2,2) cycles: each pair of smoothing
-                          sweeps as one pass over the level (e and r read once, e
-                          written once; same results bit for bit).  0 = default
-                          (on, 128 z-planes per block), > 1 = on with that many
-                          z-planes per block, < 0 = off. */
+    int sweep2;        /* V(2,2) cycles: each pair of smoothing sweeps as one pass
+                          over the level (e and r read once, e written once; same
+                          results bit for bit).  0 = default (on, column and
+                          z-chunk chosen per level; off where sweep_tx or
+                          sweep_zchunk asks for single sweeps), > 1 = on with that
+                          many z-planes per block, < 0 = off. */
     int sweep2_tx, sweep2_ty; /* column of the one-pass smoothing pair: 32 x 16,
-                          64 x 16 or 32 x 32 cells (0 = default 32 x 16; the
-                          autotuner may pick another per level) */
+                          64 x 16 or 32 x 32 cells (0 = chosen per level; the
+                          autotuner may pick another) */
 } nyxpm_opts;
 
 /* ---- lifecycle ---------------------------------------------------------- */
@@ -299,9 +300,9 @@ int nyxpm_pm_steps_comoving(nyxpm_ctx *ctx, int nsteps, double dt, double *a_io,
 /* Autotune launch shapes on this context's own arrays and keep the fastest.
  * precision_mask bit 0 (FP64) and bit 1 (FP32): for every multigrid depth, the
  * fused smoother's column shape the level allows (128x8, 64x16, 64x8, 32x8,
- * 16x8) and z-chunk (2..256 planes); with bit 1 also the one-pass smoothing
- * pair's column (32x16, 64x16, 32x32) and z-chunk (32..512), switched on at a
- * level of 2^22 cells or more where it beats two single sweeps.  Bit 2, with
+ * 16x8) and z-chunk (2..256 planes), and the one-pass smoothing pair's column
+ * (32x16, 64x16, 32x32, 16x16) and z-chunk (8..512), switched off at a level of
+ * 2^22 cells or more where two single sweeps are faster.  Bit 2, with
  * particles uploaded: the particle tile of the deposit and the kicks (16x8x8,
  * 12x8x8, 24x8x8, 16x16x8, 16x8x4, 32x8x4, 8x8x8), timed on a deposit, fold,
  * re-sort and paired kick of dt = 0 in the context's precision; the particles
@@ -312,7 +313,8 @@ int nyxpm_pm_steps_comoving(nyxpm_ctx *ctx, int nsteps, double dt, double *a_io,
  * from the tiles that hold them in FP64), as the tile option does.  report
  * (may be NULL) receives a JSON
  * object {"fp64.d0": {"shape": [tx, ty], "zchunk": z, "us": t}, ...,
- * "tile": {"shape": [tx, ty, tz], "us": t}, "sweep2.d0": {...}}.  No
+ * "tile": {"shape": [tx, ty, tz], "us": t}, "sweep2.d0": {...},
+ * "sweep2.fp64.d0": {...}}.  No
  * counterpart in the reference (AMReX's MLMG and particle tiling have fixed
  * launch shapes). */
 int nyxpm_autotune(nyxpm_ctx *ctx, int precision_mask, char *report, int report_len);

@@ -531,10 +531,13 @@ __global__ void __launch_bounds__(TX * TY / 2) k_rb_sweep(const CellSeg* segs, i
 // k_rb_sweep passes (and four k_gsrb_half) bit for bit.
 // MODE bits as k_rb_sweep's: kSweepZero (sweep 1 from e = 0), kSweepProlong
 // (sweep 1's input is ein plus the coarse correction), kSweepUpdate (sweep 2's
-// result is added to phi instead of stored).  Needs nx % TX == 0, ny % TY == 0,
-// even nx, ny, nz, nz >= 8 and nx * ny < 2^31.  HBM bytes per cell:
-// 3*sizeof(T) (e read, r read, e write) for both sweeps (+16 with
-// kSweepUpdate: phi read and written).
+// result is added to phi instead of stored).  Needs nx >= TX, ny >= TY, even nx,
+// ny, nz, nz >= 8 and nx * ny < 2^31.  HBM bytes per cell: 3*sizeof(T) (e read, r
+// read, e write) for both sweeps (+16 with kSweepUpdate: phi read and written).
+// In FP64 the pass holds 84-114 VGPRs (4-5 waves per SIMD) and is bound, as in FP32,
+// by what the L2s deliver (halo lines included); at 512^3 the pair from zero takes
+// 0.42 ms and the pair that ends in phi 0.82 ms, against 0.36 + 0.61 and 0.67 + 0.81
+// ms as single sweeps (FP32: 0.27 and 0.61 ms; the shape is chosen by sw2_choose).
 template <typename T>
 struct alignas(2 * sizeof(T)) CellPair {
     T a, b;
@@ -563,11 +566,13 @@ __global__ void __launch_bounds__((sw2_threads<TX, TY>())) k_rb_sweep2(const Cel
     const CellSeg& sg = segs[s];
     if (!active[sg.box]) return;
     const int nx = sg.n[0], ny = sg.n[1], nz = sg.n[2];
-    const int ntx = nx / TX, nty = ny / TY;
+    const int ntx = (nx + TX - 1) / TX, nty = (ny + TY - 1) / TY;
     const int zc = sg.zchunk;
     const int b = bid - sg.blk0;
     const int tx = b % ntx, ty = (b / ntx) % nty, tz = b / (ntx * nty);
-    const int x0 = tx * TX, y0 = ty * TY, z0 = tz * zc;
+    // the last column of a row is moved back to end at the level's edge; it
+    // computes the cells it shares with its neighbour and leaves them to it
+    const int x0 = min(tx * TX, nx - TX), y0 = min(ty * TY, ny - TY), z0 = tz * zc;
     const int z1 = min(nz, z0 + zc);
     const T dhx = T(sg.dh[0]), dhy = T(sg.dh[1]), dhz = T(sg.dh[2]);
     const T gamma = T(sg.gamma), inv_gamma = T(sg.inv_gamma);
@@ -602,7 +607,8 @@ __global__ void __launch_bounds__((sw2_threads<TX, TY>())) k_rb_sweep2(const Cel
     gy = gy < 0 ? gy + ny : (gy >= ny ? gy - ny : gy);
     const unsigned po = (unsigned)gy * (unsigned)nx + (unsigned)gx;      // pair's in-plane offset
     const unsigned cpo = (unsigned)(gy >> 1) * (unsigned)cnx + (unsigned)(gx >> 1);  // its parent's
-    const bool own = ly >= 4 && ly < 4 + TY && m >= 2 && m < 2 + TX / 2;
+    const bool own = ly >= 4 && ly < 4 + TY && m >= 2 && m < 2 + TX / 2 && x0 - 4 + 2 * m >= tx * TX &&
+                     y0 - 4 + ly >= ty * TY;
     // the own pair nearest to this one (phi is read there by every thread, so
     // that no load is conditional: a conditional load costs the compiler its
     // count of loads in flight, and then every wait is a wait for all of them)

@@ -277,21 +277,19 @@ struct nyxpm_ctx {
         Table t;
     };
     std::vector<SweepCfg> sw[2];
-    // FP32 levels whose pre- and post-smoothing pairs run as one pass each
-    // (k_rb_sweep2): column shape, z-chunk and launch table per depth (count 0:
-    // two k_rb_sweep passes)
+    // levels whose pre- and post-smoothing pairs run as one pass each
+    // (k_rb_sweep2): column shape, z-chunk and launch table per precision and depth
+    // (count 0: single sweeps)
     struct Sw2Cfg {
         int tx = kSw2TX, ty = kSw2TY;
-        int zc = 0;        // z-chunk chosen by the autotuner (0: sw2_zc)
-        double us = 0.0;   // autotuned launch time (0: not tuned)
-        bool on = false;   // the pass is used (t: its pieces wherever the level fits)
+        int zc = 128;      // z-planes per block
+        bool on = true;    // the pass is used (the autotuner may find single sweeps faster)
         Table t;
     };
-    std::vector<Sw2Cfg> sw2;
+    std::vector<Sw2Cfg> sw2[2];
     bool sweep2 = true;  // opts.sweep2 >= 0
-    int sw2_zc = 128;    // z-planes per block of k_rb_sweep2
-    int sw2_tx = kSw2TX, sw2_ty = kSw2TY;  // its column (before autotuning)
-    bool sw2_auto = true;  // default z-chunk (not set in the options)
+    int sw2_zc = 0;      // z-planes per block set in the options (0: chosen per level)
+    int sw2_tx = 0, sw2_ty = 0;  // column set in the options (0: chosen per level)
     std::vector<int> pre_buf;    // buffer holding e after pre-smoothing, per depth
     std::vector<int> fin_buf;    // buffer holding e after post-smoothing, per depth
     Table t_bottom, t_l0, t_res;  // t_res: level 0, at most kReduceBlocks blocks per box
@@ -486,7 +484,7 @@ int setup_boxes(nyxpm_ctx* c, int nbox, const nyxpm_geom* geoms) {
         B.G_off = Gtot;
         Gtot += nb;
         B.cell_off = cell;
-        cell += B.lev[0].nc;
+        cell += (B.lev[0].nc + 63) / 64 * 64;  // every box starts 64-cell aligned (paired loads of phi)
         c->dmax = std::max(c->dmax, B.nlev);
     }
     c->ncell_total = cell;
@@ -536,16 +534,71 @@ void sweep_seg_shape(nyxpm_ctx* c, int pr, int d, const Level& L, CellSeg& w) {
 
 // Whether a level suits k_rb_sweep2 with a tx x ty column.
 bool sw2_fits(const Level& L, int tx, int ty) {
-    return L.n[0] % tx == 0 && L.n[1] % ty == 0 && L.n[2] % 2 == 0 && L.n[2] >= 8 &&
+    return L.n[0] >= tx && L.n[1] >= ty && L.n[0] % 2 == 0 && L.n[1] % 2 == 0 && L.n[2] % 2 == 0 && L.n[2] >= 8 &&
            (long long)L.n[0] * L.n[1] < (1LL << 31);
 }
 
-// Blocks and z-chunk of one box's k_rb_sweep2 piece for depth d's current
-// shape and z-chunk.
-void sw2_seg_shape(nyxpm_ctx* c, int d, const Level& L, CellSeg& w) {
-    const auto& s2 = c->sw2[d];
-    w.zchunk = std::min(s2.zc > 0 ? s2.zc : c->sw2_zc, L.n[2]);
-    w.nblk = (L.n[0] / s2.tx) * (L.n[1] / s2.ty) * ((L.n[2] + w.zchunk - 1) / w.zchunk);
+// Blocks and z-chunk of one box's k_rb_sweep2 piece for the current shape and
+// z-chunk of (precision pr, depth d).
+void sw2_seg_shape(nyxpm_ctx* c, int pr, int d, const Level& L, CellSeg& w) {
+    const auto& s2 = c->sw2[pr][d];
+    w.zchunk = std::min(s2.zc, L.n[2]);
+    w.nblk = ((L.n[0] + s2.tx - 1) / s2.tx) * ((L.n[1] + s2.ty - 1) / s2.ty) *
+             ((L.n[2] + w.zchunk - 1) / w.zchunk);
+}
+
+// Time of a k_rb_sweep2 launch over the levels `lev` (one per box) by a two-term
+// model, in us.  (1) A block is a serial march of zc + 7 planes, each 0.33 + 0.034 w
+// us in FP64 and 0.27 + 0.022 w in FP32 with w wavefronts on its CU (of at most 16
+// and 24 at a time): measured 0.50, 0.62 and 0.80 us a plane FP64 for blocks of 5, 8
+// and 14 wavefronts alone on a CU, 0.40, 0.46 and 0.58 FP32.  (2) Each plane of e and
+// r is read in 128-byte lines with a halo of 4, at the ~10 TB/s that the L2s delivered
+// in every shape at 512^3 (FP64 and FP32: 16x16 1078 and 702 us, 32x16 753 and 468,
+// 32x32 649 and 414, 64x16 566 and 377).  The first term wants one block per CU, the
+// second wide columns: 64x16 with 256 blocks is the best of the shapes from 128^3 (16
+// us FP64, 12 us FP32) to 512^3, narrow columns with short chunks below.
+double sw2_model(int pr, int tx, int ty, int zc, const std::vector<const Level*>& lev) {
+    const int sz = pr == 0 ? 8 : 4;
+    const double wpb = ((tx + 8) / 2 * (ty + 8) + 63) / 64;
+    double blocks = 0, lines = 0, planes = 0;
+    for (const Level* L : lev) {
+        const int z = std::min(zc, L->n[2]);
+        const double cols = (double)((L->n[0] + tx - 1) / tx) * ((L->n[1] + ty - 1) / ty);
+        const double b = cols * ((L->n[2] + z - 1) / z);
+        blocks += b;
+        planes = std::max(planes, z + 7.0);
+        lines += b * (2.0 * (tx * sz + 256.0) * (ty + 8) * (z + 7) + (double)tx * ty * z * sz);
+    }
+    const double cap = pr == 0 ? 16 : 24;
+    const double per_cu = std::ceil(blocks / 256.0), fit = std::max(1.0, std::floor(cap / wpb));
+    const double w = std::min(per_cu, fit) * wpb, rounds = std::max(1.0, per_cu / fit);
+    const double march = 3.0 + rounds * planes * (pr == 0 ? 0.33 + 0.034 * w : 0.27 + 0.022 * w);
+    return std::max(march, lines / 1e7);
+}
+
+// Column and z-chunk of k_rb_sweep2 at (pr, d) for the levels `lev`: those of the
+// options, else the best by the model.  Returns false where no shape fits every level.
+constexpr int kSw2Shapes[][2] = {{64, 16}, {32, 32}, {32, 16}, {16, 16}, {16, 8}};
+constexpr int kSw2Z[] = {512, 384, 256, 192, 128, 96, 64, 48, 32, 24, 16, 12, 8};
+bool sw2_choose(nyxpm_ctx* c, int pr, int d, const std::vector<const Level*>& lev) {
+    auto& s2 = c->sw2[pr][d];
+    double best = -1.0;
+    for (auto& sh : kSw2Shapes) {
+        const int tx = c->sw2_tx ? c->sw2_tx : sh[0], ty = c->sw2_tx ? c->sw2_ty : sh[1];
+        bool fits = true;
+        for (const Level* L : lev) fits = fits && sw2_fits(*L, tx, ty);
+        if (!fits) continue;
+        for (int z : kSw2Z) {
+            const int zc = c->sw2_zc > 0 ? c->sw2_zc : z;
+            const double us = sw2_model(pr, tx, ty, zc, lev);
+            if (best >= 0.0 && us >= best) continue;
+            best = us;
+            s2.tx = tx;
+            s2.ty = ty;
+            s2.zc = zc;
+        }
+    }
+    return best >= 0.0;
 }
 
 // Coarse tile of k_resid_restrict_z: kRrCX x CY coarse columns, CY by precision
@@ -595,12 +648,8 @@ int build_tables(nyxpm_ctx* c) {
     // not depend on the column shape, so both precisions share it).
     c->t_full.assign(c->dmax, {});
     c->t_half.assign(c->dmax, {});
-    c->sw2.assign(c->dmax, {});
-    for (auto& s2 : c->sw2) {
-        s2.tx = c->sw2_tx;
-        s2.ty = c->sw2_ty;
-    }
     for (int pr = 0; pr < 2; ++pr) {
+        c->sw2[pr].assign(c->dmax, {});
         c->t_rrz[pr].assign(c->dmax, {});
         c->t_rrc[pr].assign(c->dmax, {});
     }
@@ -620,7 +669,7 @@ int build_tables(nyxpm_ctx* c) {
                     break;
                 }
     }
-    std::vector<bool> fusable(c->dmax, false);
+    std::vector<bool> fusable(c->dmax, false), pairs(c->dmax, false);
     for (int d = 0; d + 1 < c->dmax; ++d) {
         bool any = false, even = true;
         for (int b = 0; b < nbox; ++b) {
@@ -658,8 +707,18 @@ int build_tables(nyxpm_ctx* c) {
             c->sw[0][d].tx = c->sw[1][d].tx = 0;
             fusable[d] = false;
         }
+        // smoothing pairs as one pass: V(2,2) cycles on levels a column shape fits,
+        // unless the options ask for single sweeps (a set single-sweep shape or
+        // z-chunk, half sweeps, the residual formed in the first sweep)
+        if (any && even && !c->no_fused && c->sweep2 && c->nu1 == 2 && c->nu2 == 2 && !c->fuse_res &&
+            !(c->sw2_zc == 0 && (c->force_tx[0] || c->sweep_zchunk > 0))) {
+            std::vector<const Level*> lev;
+            for (int b = 0; b < nbox; ++b)
+                if (d < c->boxes[b].dc) lev.push_back(&c->boxes[b].lev[d]);
+            pairs[d] = sw2_choose(c, 0, d, lev) && sw2_choose(c, 1, d, lev);
+        }
         int cur = 0;
-        if (fusable[d]) {
+        if (fusable[d] || pairs[d]) {
             for (int q = 1; q < c->nu1; ++q) cur ^= 1;
             c->pre_buf[d] = cur;
             for (int q = 0; q < c->nu2; ++q) cur ^= 1;
@@ -721,31 +780,18 @@ int build_tables(nyxpm_ctx* c) {
             c->t_rrz[pr][d] = add_table(vrz[pr]);
             c->t_rrc[pr][d] = add_table(vrc[pr]);
         }
-        // the two-sweep pass (FP32) where every box's level fits its column shape
-        // and offers at least 1024 blocks, with V(2,2) cycles
-        std::vector<CellSeg> v2;
-        bool ok2 = c->sweep2 && c->sw[1][d].tx != 0 && c->nu1 == 2 && c->nu2 == 2 && !c->fuse_res;
-        long long blocks2 = 0;
-        for (int b = 0; b < nbox && ok2; ++b) {
-            const Box& B = c->boxes[b];
-            if (d >= B.dc) continue;
-            const Level& L = B.lev[d];
-            if (!sw2_fits(L, c->sw2_tx, c->sw2_ty)) {
-                ok2 = false;
-                break;
+        for (int pr = 0; pr < 2; ++pr) {
+            std::vector<CellSeg> v2;
+            for (int b = 0; b < nbox && pairs[d]; ++b) {
+                const Box& B = c->boxes[b];
+                if (d >= B.dc) continue;
+                CellSeg w = mk(b, d, 1);
+                w.ebuf = coarse_buf(B, d);
+                sw2_seg_shape(c, pr, d, B.lev[d], w);
+                v2.push_back(w);
             }
-            CellSeg w = mk(b, d, 1);
-            w.ebuf = coarse_buf(B, d);
-            sw2_seg_shape(c, d, L, w);
-            blocks2 += w.nblk;
-            v2.push_back(w);
+            c->sw2[pr][d].t = add_table(v2);
         }
-        // used with the default z-chunk where the level offers enough blocks (the
-        // autotuner may switch it on elsewhere), with a z-chunk set in the
-        // options wherever the shape fits
-        if (!ok2) v2.clear();
-        c->sw2[d].t = add_table(v2);
-        c->sw2[d].on = ok2 && !v2.empty() && !(c->sw2_auto && blocks2 < 1024);
     }
     {
         std::vector<CellSeg> vb;
@@ -1276,28 +1322,33 @@ void launch_sweep(nyxpm_ctx* c, int d, const T* ein, T* eout, const T* r, const 
 #undef NYXPM_SWEEP
 }
 
-// Two red-black sweeps in one pass (k_rb_sweep2, FP32) at depth d.
-template <int MODE>
-void launch_sweep2(nyxpm_ctx* c, int d, const float* ein, float* eout, const float* r, const float* ec0,
-                   const float* ec1) {
-    const auto& s2 = c->sw2[d];
+// Two red-black sweeps in one pass (k_rb_sweep2) at depth d.
+template <typename T, int MODE>
+void launch_sweep2(nyxpm_ctx* c, int d, const T* ein, T* eout, const T* r, const T* ec0, const T* ec1) {
+    const auto& s2 = c->sw2[sizeof(T) == 8 ? 0 : 1][d];
     const auto& t = s2.t;
-#define NYXPM_SW2(TX, TY)                                                                               \
-    hipLaunchKernelGGL((k_rb_sweep2<float, TX, TY, MODE>), dim3(t.blocks), dim3(sw2_threads<TX, TY>()), 0, \
-                       c->stream, c->segs(t), t.count, c->active, ein, eout, r, ec0, ec1, c->phi)
-    if (s2.tx == 64 && s2.ty == 16)
-        NYXPM_SW2(64, 16);
-    else if (s2.tx == 32 && s2.ty == 32)
-        NYXPM_SW2(32, 32);
-    else
-        NYXPM_SW2(32, 16);
+#define NYXPM_SW2(TX, TY)                                                                            \
+    case TX * 100 + TY:                                                                              \
+        hipLaunchKernelGGL((k_rb_sweep2<T, TX, TY, MODE>), dim3(t.blocks), dim3(sw2_threads<TX, TY>()), 0, \
+                           c->stream, c->segs(t), t.count, c->active, ein, eout, r, ec0, ec1, c->phi); \
+        break;
+    switch (s2.tx * 100 + s2.ty) {
+        NYXPM_SW2(32, 16)
+        NYXPM_SW2(16, 16)
+        NYXPM_SW2(16, 8)
+        NYXPM_SW2(64, 16)
+        NYXPM_SW2(32, 32)
+        default:
+            break;
+    }
 #undef NYXPM_SW2
 }
 
 // Whether depth d runs its smoothing pairs as k_rb_sweep2 passes.
 template <typename T>
 bool two_sweep(const nyxpm_ctx* c, int d) {
-    return sizeof(T) == 4 && d < (int)c->sw2.size() && c->sw2[d].on && c->sw2[d].t.count > 0;
+    const auto& s2 = c->sw2[sizeof(T) == 8 ? 0 : 1][d];
+    return s2.on && s2.t.count > 0;
 }
 
 // One V-cycle on every active box.  Returns in *updated whether phi += e has
@@ -1324,16 +1375,12 @@ int vcycle(nyxpm_ctx* c, bool* updated, bool sweep0_done = false, bool first = t
             // both pre-smoothing sweeps in one pass, into the buffer the two
             // post-smoothing sweeps then read (so that they end in fin_buf)
             cur = 1 - c->pre_buf[d];
-            float* e0 = reinterpret_cast<float*>(eb[0]);
-            float* e1 = reinterpret_cast<float*>(eb[1]);
-            float* ebf[2] = {e0, e1};
-            const float* rf = reinterpret_cast<const float*>(r);
             if (keep) {
                 Timed t(c, lvl_name("sweep2", d));
-                launch_sweep2<0>(c, d, ebf[c->fin_buf[d]], ebf[cur], rf, e0, e1);
+                launch_sweep2<T, 0>(c, d, eb[c->fin_buf[d]], eb[cur], r, eb[0], eb[1]);
             } else {
                 Timed t(c, lvl_name("sweep2_0", d));
-                launch_sweep2<kSweepZero>(c, d, ebf[cur], ebf[cur], rf, e0, e1);
+                launch_sweep2<T, kSweepZero>(c, d, eb[cur], eb[cur], r, eb[0], eb[1]);
             }
         } else if (c->sw[pr][d].tx) {
             if (keep) {
@@ -1401,18 +1448,14 @@ int vcycle(nyxpm_ctx* c, bool* updated, bool sweep0_done = false, bool first = t
             // both post-smoothing sweeps in one pass (prolongation on load), from
             // the pre-smoothing pass's buffer into fin_buf (or into phi)
             cur = 1 - c->pre_buf[d];
-            float* e0 = reinterpret_cast<float*>(eb[0]);
-            float* e1 = reinterpret_cast<float*>(eb[1]);
-            float* ebf[2] = {e0, e1};
-            const float* rf = reinterpret_cast<const float*>(r);
             const bool upd = last && d == 0 && c->fuse_update;
             if (upd) {
                 Timed t(c, lvl_name("sweep2_u", d));
-                launch_sweep2<kSweepProlong | kSweepUpdate>(c, d, ebf[cur], ebf[1 - cur], rf, e0, e1);
+                launch_sweep2<T, kSweepProlong | kSweepUpdate>(c, d, eb[cur], eb[1 - cur], r, eb[0], eb[1]);
                 *updated = true;
             } else {
                 Timed t(c, lvl_name("sweep2_p", d));
-                launch_sweep2<kSweepProlong>(c, d, ebf[cur], ebf[1 - cur], rf, e0, e1);
+                launch_sweep2<T, kSweepProlong>(c, d, eb[cur], eb[1 - cur], r, eb[0], eb[1]);
             }
         } else if (c->sw[pr][d].tx && c->nu2 > 0) {
             // prolongation fused into the first sweep; phi += e into the last one
@@ -1902,10 +1945,7 @@ int nyxpm_create_batch(nyxpm_ctx** out, int nbox, const nyxpm_geom* geoms, const
             c->sw2_ty = ty;
         }
         if (opts->sweep2 < 0) c->sweep2 = false;
-        if (opts->sweep2 > 1) {
-            c->sw2_zc = std::max(8, opts->sweep2);
-            c->sw2_auto = false;
-        }
+        if (opts->sweep2 > 1) c->sw2_zc = std::max(8, opts->sweep2);
         if (opts->resort_slack < 0) {
             c->slack_num = 0;
             c->slack_pad = 0;
@@ -3060,14 +3100,14 @@ static int rebuild_rrz_table(nyxpm_ctx* c, int pr, int d, int zc) {
     return NYXPM_OK;
 }
 
-// Re-derive the k_rb_sweep2 pieces of depth d in place for its current shape
+// Re-derive the k_rb_sweep2 pieces of (pr, d) in place for their current shape
 // and z-chunk, and upload them.
-static int rebuild_sw2_table(nyxpm_ctx* c, int d) {
-    auto& t = c->sw2[d].t;
+static int rebuild_sw2_table(nyxpm_ctx* c, int pr, int d) {
+    auto& t = c->sw2[pr][d].t;
     int blk = 0;
     for (int q = 0; q < t.count; ++q) {
         CellSeg& w = c->seg_host[t.first + q];
-        sw2_seg_shape(c, d, c->boxes[w.box].lev[d], w);
+        sw2_seg_shape(c, pr, d, c->boxes[w.box].lev[d], w);
         w.blk0 = blk;
         blk += w.nblk;
     }
@@ -3222,7 +3262,6 @@ int nyxpm_autotune(nyxpm_ctx* c, int precision_mask, char* report, int report_le
         for (int d = 0; d + 1 < c->dmax; ++d) {
             auto& cfg = c->sw[pr][d];
             if (!cfg.tx || cfg.t.count == 0) continue;
-            if (pr == 1 && two_sweep<float>(c, d)) continue;  // k_rb_sweep2 smooths this depth
             const int tx0 = cfg.tx, ty0 = cfg.ty, zc0 = cfg.zc;
             double best = 1e30;
             int btx = tx0, bty = ty0, bzc = zc0;
@@ -3373,71 +3412,74 @@ int nyxpm_autotune(nyxpm_ctx* c, int precision_mask, char* report, int report_le
         rep += buf;
         first_entry = false;
     }
-    // the two-sweep pass: column shape and z-chunk per depth (FP32)
-    static const int sw2_shapes[][2] = {{32, 16}, {64, 16}, {32, 32}};
-    static const int sw2_zcs[] = {32, 64, 128, 256, 512};
-    for (int d = 0; (precision_mask & 2) && d + 1 < c->dmax; ++d) {
-        auto& s2 = c->sw2[d];
-        if (s2.t.count == 0) continue;
-        const int tx0 = s2.tx, ty0 = s2.ty;
-        int maxnz = 0;
-        for (int q = 0; q < s2.t.count; ++q)
-            maxnz = std::max(maxnz, c->boxes[c->seg_host[s2.t.first + q].box].lev[d].n[2]);
-        double best = 1e30;
-        int btx = tx0, bty = ty0, bzc = s2.zc;
-        for (auto& sh : sw2_shapes) {
-            bool ok = true;
-            for (int q = 0; q < s2.t.count && ok; ++q)
-                ok = sw2_fits(c->boxes[c->seg_host[s2.t.first + q].box].lev[d], sh[0], sh[1]);
-            if (!ok) continue;
-            for (int zc : sw2_zcs) {
-                if (zc != sw2_zcs[0] && zc >= 2 * maxnz) continue;
-                s2.tx = sh[0];
-                s2.ty = sh[1];
-                s2.zc = zc;
-                if ((rc = rebuild_sw2_table(c, d))) return rc;
-                float ms = 0.f;
-                for (int rep_i = 0; rep_i < 2; ++rep_i) {  // warm-up, then a timed batch of 4
-                    HIPCK(c, hipEventRecord(e0, c->stream));
-                    for (int k = 0; k < (rep_i ? 4 : 1); ++k)
-                        launch_sweep2<0>(c, d, c->e32, c->e32b, c->r32, c->e32, c->e32b);
-                    HIPCK(c, hipEventRecord(e1, c->stream));
-                    HIPCK(c, hipEventSynchronize(e1));
-                    HIPCK(c, hipEventElapsedTime(&ms, e0, e1));
-                }
-                LAUNCHCK(c);
-                const double us = ms * 1e3 / 4.0;
-                if (c->verbose)
-                    std::fprintf(stderr, "nyxpm autotune: sweep2.d%d %dx%d z-chunk %d: %.2f us\n", d, sh[0], sh[1],
-                                 zc, us);
-                if (us < best) {
-                    best = us;
-                    btx = sh[0];
-                    bty = sh[1];
-                    bzc = zc;
+    // the two-sweep pass: column shape and z-chunk per precision and depth
+    static const int sw2_shapes[][2] = {{32, 16}, {64, 16}, {32, 32}, {16, 16}};
+    static const int sw2_zcs[] = {8, 16, 32, 64, 128, 256, 512};
+    for (int pr = 0; pr < 2; ++pr) {
+        if (!(precision_mask & (1 << pr))) continue;
+        for (int d = 0; d + 1 < c->dmax; ++d) {
+            auto& s2 = c->sw2[pr][d];
+            if (s2.t.count == 0) continue;
+            int maxnz = 0;
+            for (int q = 0; q < s2.t.count; ++q)
+                maxnz = std::max(maxnz, c->boxes[c->seg_host[s2.t.first + q].box].lev[d].n[2]);
+            double best = 1e30;
+            int btx = s2.tx, bty = s2.ty, bzc = s2.zc;
+            for (auto& sh : sw2_shapes) {
+                bool ok = true;
+                for (int q = 0; q < s2.t.count && ok; ++q)
+                    ok = sw2_fits(c->boxes[c->seg_host[s2.t.first + q].box].lev[d], sh[0], sh[1]);
+                if (!ok) continue;
+                for (int zc : sw2_zcs) {
+                    if (zc != sw2_zcs[0] && zc >= 2 * maxnz) continue;
+                    s2.tx = sh[0];
+                    s2.ty = sh[1];
+                    s2.zc = zc;
+                    if ((rc = rebuild_sw2_table(c, pr, d))) return rc;
+                    float ms = 0.f;
+                    for (int rep_i = 0; rep_i < 2; ++rep_i) {  // warm-up, then a timed batch of 4
+                        HIPCK(c, hipEventRecord(e0, c->stream));
+                        for (int k = 0; k < (rep_i ? 4 : 1); ++k) {
+                            if (pr == 0)
+                                launch_sweep2<double, 0>(c, d, c->e64, c->e64b, c->r64, c->e64, c->e64b);
+                            else
+                                launch_sweep2<float, 0>(c, d, c->e32, c->e32b, c->r32, c->e32, c->e32b);
+                        }
+                        HIPCK(c, hipEventRecord(e1, c->stream));
+                        HIPCK(c, hipEventSynchronize(e1));
+                        HIPCK(c, hipEventElapsedTime(&ms, e0, e1));
+                    }
+                    LAUNCHCK(c);
+                    const double us = ms * 1e3 / 4.0;
+                    if (c->verbose)
+                        std::fprintf(stderr, "nyxpm autotune: sweep2 %s.d%d %dx%d z-chunk %d: %.2f us\n",
+                                     pr == 0 ? "fp64" : "fp32", d, sh[0], sh[1], zc, us);
+                    if (us < best) {
+                        best = us;
+                        btx = sh[0];
+                        bty = sh[1];
+                        bzc = zc;
+                    }
                 }
             }
+            s2.tx = btx;
+            s2.ty = bty;
+            s2.zc = bzc;
+            if ((rc = rebuild_sw2_table(c, pr, d))) return rc;
+            // two single sweeps where they are faster on a level of at least 2^22
+            // cells (on smaller ones the launches take a few microseconds, and a
+            // timing is mostly launch overhead, which a tracer inflates)
+            const double us1 = c->sw[pr][d].us;
+            long long cells = 0;
+            for (int q = 0; q < s2.t.count; ++q) cells += c->boxes[c->seg_host[s2.t.first + q].box].lev[d].nc;
+            s2.on = !(us1 > 0.0 && best > 2.0 * us1 && cells >= (1LL << 22));
+            char buf[200];
+            snprintf(buf, sizeof(buf),
+                     "%s\"sweep2%s.d%d\": {\"shape\": [%d, %d], \"zchunk\": %d, \"us\": %.2f, \"on\": %s}",
+                     first_entry ? "" : ", ", pr == 0 ? ".fp64" : "", d, btx, bty, bzc, best, s2.on ? "true" : "false");
+            rep += buf;
+            first_entry = false;
         }
-        s2.tx = btx;
-        s2.ty = bty;
-        s2.zc = bzc;
-        s2.us = best;
-        // where the default left the pass off (too few blocks), it replaces the
-        // two k_rb_sweep passes on a level of at least 2^22 cells if it is faster
-        // than two of them (on smaller levels the launches take a few
-        // microseconds, and a timing is mostly launch overhead, which a tracer
-        // inflates)
-        const double us1 = c->sw[1][d].us;
-        long long cells = 0;
-        for (int q = 0; q < s2.t.count; ++q) cells += c->boxes[c->seg_host[s2.t.first + q].box].lev[d].nc;
-        if (!s2.on && us1 > 0.0 && best < 2.0 * us1 && cells >= (1LL << 22)) s2.on = true;
-        if ((rc = rebuild_sw2_table(c, d))) return rc;
-        char buf[200];
-        snprintf(buf, sizeof(buf),
-                 "%s\"sweep2.d%d\": {\"shape\": [%d, %d], \"zchunk\": %d, \"us\": %.2f, \"on\": %s}",
-                 first_entry ? "" : ", ", d, btx, bty, bzc, best, s2.on ? "true" : "false");
-        rep += buf;
-        first_entry = false;
     }
     rep += "}";
     hipEventDestroy(e0);

@@ -67,7 +67,7 @@ class PMContext:
         each pm_steps solve, "default" = "previous" (Nyx's) or "extrapolate"
         (2 phi_n - phi_{n-1}).  ir_first: mixed precision, FP32 V-cycles before a
         solve's first FP64 residual test (0: library default; 1: after every
-        cycle).  sweep2: FP32 smoothing pairs as one pass (0: on, > 1: on with
+        cycle).  sweep2: smoothing pairs as one pass (0: on, > 1: on with
         that many z-planes per block, < 0: off); sweep2_shape: its column,
         (32, 16), (64, 16) or (32, 32).  verbose: the library reports to stderr
         (the autotuner's trials)."""
