@@ -326,7 +326,8 @@ int nyxpm_autotune(nyxpm_ctx *ctx, int precision_mask, char *report, int report_
  * particle stages "keys", "scan", "scatter" (full sort), "migrate" (incremental
  * re-sort), "items", "deposit", "fold", "rhs", "kick_drift", "kick",
  * "kick_pair"; multigrid stages "residual", "update", "coarse", "bottom" and,
- * per depth d, "sweep0.dD", "sweep.dD", "sweep_p.dD", "sweep_u.dD",
+ * per depth d, "leg_down.dD", "leg_up.dD", "sweep2_0.dD", "sweep2.dD",
+ * "sweep2_p.dD", "sweep2_u.dD", "sweep0.dD", "sweep.dD", "sweep_p.dD", "sweep_u.dD",
  * "smooth.dD", "resid_restrict.dD", "prolong.dD", "fill.dD". */
 int nyxpm_timing_enable(nyxpm_ctx *ctx, int on);
 /* Restricts the timing to the stages named in `names` (comma-separated, e.g.

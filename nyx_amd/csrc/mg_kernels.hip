@@ -829,6 +829,176 @@ __global__ void __launch_bounds__((sw2_threads<TX, TY>())) k_rb_sweep2(const Cel
     }
 }
 
+// One leg of a V(2,2) cycle on a small level in one launch.  Down: two red-black
+// sweeps (from zero, or from ein with kSweepKeep), e out, and the residual
+// restricted to the next level's r.  Up: the prolongation on load and two sweeps,
+// e out (kSweepUpdate: phi += e).  A block owns 8 x 8 x 8 cells and works on them
+// widened by the halo the steps need: the sweeps are right one cell further in
+// after each of the four half sweeps (down: halo 4 around what the residual reads,
+// from zero; 5 from ein; up: 4), and a value computed outside that region never
+// reaches a cell inside it, so the results equal the separate launches bit for bit.
+// Pairs of x-adjacent cells live in registers and pass values through one LDS array
+// per colour, as in the coarse workgroup.  Per own cell the halo costs 8 (13) times
+// the updates, which a level too small to fill the chip has idle units for: the
+// separate launches are each bound by the latency of a march of 15 planes or of the
+// launch itself.  Any even level; cells past its edge wrap around.
+// Measured, down and up: 8 + 8 us FP64 and 8 + 8 us FP32 (11 from ein) at 64^3, 6 + 6
+// and 5 + 5 us at 32^3, against 9 + 7 + 11 and 8 + 5 + 10 us as paired passes and a
+// restriction, with a launch less.
+constexpr int kLegThreads = 512, kLegB = 8;
+constexpr int kSweepKeep = 16;  // down: ein is not zero
+template <typename T, int MODE, bool DOWN>
+__global__ void __launch_bounds__(kLegThreads) k_leg(const CellSeg* segs, int nseg, const int* active,
+                                                     const T* __restrict__ ein, T* __restrict__ eout,
+                                                     T* __restrict__ r, const T* ec0, const T* ec1, double* phi) {
+    constexpr bool KEEP = (MODE & kSweepKeep) != 0, UPD = (MODE & kSweepUpdate) != 0;
+    constexpr int B = kLegB;
+    constexpr int H = DOWN && KEEP ? 5 : 4, XH = (H + 1) / 2 * 2;  // halo (even in x: whole pairs)
+    constexpr int HS = DOWN ? 4 : 3;                               // halo the first half sweep must get right
+    constexpr int PX = B / 2 + XH, RY = B + 2 * H, RZ = B + 2 * H, PL = PX * RY, NPAIR = PL * RZ;
+    constexpr int NP = (NPAIR + kLegThreads - 1) / kLegThreads;
+    // a plane of padding below and above takes the reads of the region's rim
+    __shared__ T sr_[NPAIR + 2 * PL], sb_[NPAIR + 2 * PL];
+    T *sr = sr_ + PL, *sb = sb_ + PL;
+    const int bid = blockIdx.x;
+    const CellSeg& sg = segs[find_seg(segs, nseg, bid)];
+    if (!active[sg.box]) return;
+    const int nx = sg.n[0], ny = sg.n[1], nz = sg.n[2];
+    const int ntx = (nx + B - 1) / B, nty = (ny + B - 1) / B;
+    const int b = bid - sg.blk0;
+    const int tx = b % ntx, ty = (b / ntx) % nty, tz = b / (ntx * nty);
+    const int x0 = tx * B, y0 = ty * B, z0 = tz * B;
+    const T dhx = T(sg.dh[0]), dhy = T(sg.dh[1]), dhz = T(sg.dh[2]);
+    const T gamma = T(sg.gamma), inv_gamma = T(sg.inv_gamma);
+    const T* Ein = ein + sg.off;
+    T* Eout = eout + sg.off;
+    const T* R = r + sg.off;
+    const T* Ec = (sg.ebuf ? ec1 : ec0) + sg.coff;
+    const int cnx = nx >> 1, cny = ny >> 1;
+    const int tid = threadIdx.x;
+    auto wrap = [](int g, int n) {
+        g = g < 0 ? g + n : (g >= n ? g - n : g);
+        if (n < 2 * B) {  // the region may span the level more than once
+            g %= n;
+            g = g < 0 ? g + n : g;
+        }
+        return g;
+    };
+    T er[NP], eb[NP], fr[NP], fb[NP];
+    bool c[NP];   // the red cell is the pair's second
+    int kk[NP];   // plane of the pair in the region (past it: no pair)
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+        const int q = min(tid + u * kLegThreads, NPAIR - 1);
+        const int m = q % PX, j = (q / PX) % RY, k = q / PL;
+        const int gx = wrap(x0 - XH + 2 * m, nx), gy = wrap(y0 - H + j, ny), gz = wrap(z0 - H + k, nz);
+        const size_t o = cidx(gx, gy, gz, nx, ny);
+        c[u] = (y0 - H + j + z0 - H + k) & 1;
+        kk[u] = tid + u * kLegThreads < NPAIR ? k : 2 * RZ;
+        const CellPair<T> f = *reinterpret_cast<const CellPair<T>*>(R + o);
+        fr[u] = c[u] ? f.b : f.a;
+        fb[u] = c[u] ? f.a : f.b;
+        er[u] = eb[u] = T(0);
+        if (!DOWN || KEEP) {
+            CellPair<T> v = *reinterpret_cast<const CellPair<T>*>(Ein + o);
+            if (!DOWN) {
+                const T cv = Ec[cidx(gx >> 1, gy >> 1, gz >> 1, cnx, cny)];
+                v.a = v.a + cv;
+                v.b = v.b + cv;
+            }
+            er[u] = c[u] ? v.b : v.a;
+            eb[u] = c[u] ? v.a : v.b;
+            if (kk[u] < RZ) sb[tid + u * kLegThreads] = eb[u];
+        }
+    }
+    constexpr bool ZERO = DOWN && !KEEP;
+    if (!ZERO) __syncthreads();
+    // whether half sweep s (0..3) must be right on plane k of the region
+    auto need = [&](int s, int k) { return k >= H - (HS - s) && k < H + B + (HS - s); };
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (need(2 * it, kk[u])) {
+                const int q = tid + u * kLegThreads;
+                T sx = T(0) + T(0), sy = sx, sz = sx;
+                if (!(ZERO && it == 0)) {
+                    sx = eb[u] + sb[c[u] ? q + 1 : q - 1];
+                    sy = sb[q - PX] + sb[q + PX];
+                    sz = sb[q - PL] + sb[q + PL];
+                }
+                er[u] = gs_update(er[u], fr[u], sx, sy, sz, gamma, inv_gamma, dhx, dhy, dhz);
+                sr[q] = er[u];
+            }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < NP; ++u)
+            if (need(2 * it + 1, kk[u])) {
+                const int q = tid + u * kLegThreads;
+                eb[u] = gs_update(eb[u], fb[u], er[u] + sr[c[u] ? q - 1 : q + 1], sr[q - PX] + sr[q + PX],
+                                  sr[q - PL] + sr[q + PL], gamma, inv_gamma, dhx, dhy, dhz);
+                sb[q] = eb[u];
+            }
+        if (DOWN || it == 0) __syncthreads();
+    }
+    // the own cells out (and, going down, their residual in lap7's arithmetic)
+    T ra[NP], rb[NP];
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+        if (kk[u] < H || kk[u] >= H + B) continue;
+        const int q = tid + u * kLegThreads;
+        const int m = q % PX, j = (q / PX) % RY;
+        const int gx = x0 - XH + 2 * m, gy = y0 - H + j, gz = z0 - H + kk[u];
+        if (gx < x0 || gx >= x0 + B || gy < y0 || gy >= y0 + B) continue;
+        const T a = c[u] ? eb[u] : er[u], bb = c[u] ? er[u] : eb[u];
+        if (gx < nx && gy < ny && gz < nz) {
+            const size_t o = cidx(gx, gy, gz, nx, ny);
+            if (UPD) {
+                double* P = phi + sg.foff + o;
+                P[0] = P[0] + (double)a;
+                P[1] = P[1] + (double)bb;
+            } else {
+                *reinterpret_cast<CellPair<T>*>(Eout + o) = CellPair<T>{a, bb};
+            }
+        }
+        if (DOWN) {
+            const T* oa = c[u] ? sr : sb;  // the colour of a's neighbours
+            const T* ob = c[u] ? sb : sr;
+            const T ax = dhx * (oa[q - 1] - T(2) * a + bb), bx = dhx * (a - T(2) * bb + ob[q + 1]);
+            const T ay = dhy * (oa[q - PX] - T(2) * a + oa[q + PX]), by = dhy * (ob[q - PX] - T(2) * bb + ob[q + PX]);
+            const T az = dhz * (oa[q - PL] - T(2) * a + oa[q + PL]), bz = dhz * (ob[q - PL] - T(2) * bb + ob[q + PL]);
+            ra[u] = (c[u] ? fb[u] : fr[u]) - (ax + ay + az);
+            rb[u] = (c[u] ? fr[u] : fb[u]) - (bx + by + bz);
+        }
+    }
+    if (!DOWN) return;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < NP; ++u) {
+        if (kk[u] < H || kk[u] >= H + B) continue;
+        const int q = tid + u * kLegThreads;
+        const int m = q % PX, j = (q / PX) % RY;
+        if (m < XH / 2 || m >= XH / 2 + B / 2 || j < H || j >= H + B) continue;
+        sr[q] = ra[u];
+        sb[q] = rb[u];
+    }
+    __syncthreads();
+    if (tid < B * B * B / 8) {
+        const int I = tid % (B / 2), J = (tid / (B / 2)) % (B / 2), K = tid / (B * B / 4);
+        const int cx = x0 / 2 + I, cy = y0 / 2 + J, cz = z0 / 2 + K;
+        T acc = T(0);
+#pragma unroll
+        for (int k2 = 0; k2 < 2; ++k2)
+#pragma unroll
+            for (int j2 = 0; j2 < 2; ++j2) {
+                const int q = (H + 2 * K + k2) * PL + (H + 2 * J + j2) * PX + XH / 2 + I;
+                acc += sr[q];
+                acc += sb[q];
+            }
+        if (cx < cnx && cy < cny && cz < (nz >> 1)) r[sg.coff + cidx(cx, cy, cz, cnx, cny)] = T(0.125) * acc;
+    }
+}
+
 // Residual of the correction, restricted: r_c(I) = 0.125 * sum_children (r - L e),
 // children summed k, then j, then i innermost.  One thread per coarse cell.
 template <typename T>

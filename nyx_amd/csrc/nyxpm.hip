@@ -287,6 +287,7 @@ struct nyxpm_ctx {
         Table t;
     };
     std::vector<Sw2Cfg> sw2[2];
+    std::vector<Table> t_leg;    // depths whose legs run as one launch each (k_leg), both precisions
     bool sweep2 = true;  // opts.sweep2 >= 0
     int sw2_zc = 0;      // z-planes per block set in the options (0: chosen per level)
     int sw2_tx = 0, sw2_ty = 0;  // column set in the options (0: chosen per level)
@@ -576,6 +577,12 @@ double sw2_model(int pr, int tx, int ty, int zc, const std::vector<const Level*>
     return std::max(march, lines / 1e7);
 }
 
+// Cells of a depth's levels (all boxes) up to which its V-cycle legs run as one launch
+// each (k_leg); above, a paired pass and a restriction, whose halos cost less.
+// Measured, us per V-cycle FP64 / mixed with legs on the finest level and without:
+// 64^3 82 / 64 and 100 / 78, 80^3 108 / 85 and 107 / 84, 96^3 122 / 97 and 109 / 86.
+constexpr long long kLegCells = 1ll << 19;
+
 // Column and z-chunk of k_rb_sweep2 at (pr, d) for the levels `lev`: those of the
 // options, else the best by the model.  Returns false where no shape fits every level.
 constexpr int kSw2Shapes[][2] = {{64, 16}, {32, 32}, {32, 16}, {16, 16}, {16, 8}};
@@ -669,7 +676,8 @@ int build_tables(nyxpm_ctx* c) {
                     break;
                 }
     }
-    std::vector<bool> fusable(c->dmax, false), pairs(c->dmax, false);
+    std::vector<bool> fusable(c->dmax, false), pairs(c->dmax, false), legs(c->dmax, false);
+    c->t_leg.assign(c->dmax, {});
     for (int d = 0; d + 1 < c->dmax; ++d) {
         bool any = false, even = true;
         for (int b = 0; b < nbox; ++b) {
@@ -713,12 +721,19 @@ int build_tables(nyxpm_ctx* c) {
         if (any && even && !c->no_fused && c->sweep2 && c->nu1 == 2 && c->nu2 == 2 && !c->fuse_res &&
             !(c->sw2_zc == 0 && (c->force_tx[0] || c->sweep_zchunk > 0))) {
             std::vector<const Level*> lev;
+            long long cells = 0;
             for (int b = 0; b < nbox; ++b)
-                if (d < c->boxes[b].dc) lev.push_back(&c->boxes[b].lev[d]);
+                if (d < c->boxes[b].dc) {
+                    lev.push_back(&c->boxes[b].lev[d]);
+                    cells += lev.back()->nc;
+                }
             pairs[d] = sw2_choose(c, 0, d, lev) && sw2_choose(c, 1, d, lev);
+            // one launch per leg on small levels and on those no column fits, unless
+            // the options set the pair's column or chunk
+            legs[d] = c->sw2_zc == 0 && c->sw2_tx == 0 && (cells <= kLegCells || !pairs[d]);
         }
         int cur = 0;
-        if (fusable[d] || pairs[d]) {
+        if (fusable[d] || pairs[d] || legs[d]) {
             for (int q = 1; q < c->nu1; ++q) cur ^= 1;
             c->pre_buf[d] = cur;
             for (int q = 0; q < c->nu2; ++q) cur ^= 1;
@@ -780,9 +795,23 @@ int build_tables(nyxpm_ctx* c) {
             c->t_rrz[pr][d] = add_table(vrz[pr]);
             c->t_rrc[pr][d] = add_table(vrc[pr]);
         }
+        if (legs[d]) {
+            std::vector<CellSeg> vl;
+            for (int b = 0; b < nbox; ++b) {
+                const Box& B = c->boxes[b];
+                if (d >= B.dc) continue;
+                const Level& L = B.lev[d];
+                CellSeg w = mk(b, d, 1);
+                w.ebuf = coarse_buf(B, d);
+                w.nblk = ((L.n[0] + kLegB - 1) / kLegB) * ((L.n[1] + kLegB - 1) / kLegB) *
+                         ((L.n[2] + kLegB - 1) / kLegB);
+                vl.push_back(w);
+            }
+            c->t_leg[d] = add_table(vl);
+        }
         for (int pr = 0; pr < 2; ++pr) {
             std::vector<CellSeg> v2;
-            for (int b = 0; b < nbox && pairs[d]; ++b) {
+            for (int b = 0; b < nbox && pairs[d] && !legs[d]; ++b) {
                 const Box& B = c->boxes[b];
                 if (d >= B.dc) continue;
                 CellSeg w = mk(b, d, 1);
@@ -1344,6 +1373,14 @@ void launch_sweep2(nyxpm_ctx* c, int d, const T* ein, T* eout, const T* r, const
 #undef NYXPM_SW2
 }
 
+// One leg of the V-cycle at depth d (k_leg).
+template <typename T, int MODE, bool DOWN>
+void launch_leg(nyxpm_ctx* c, int d, const T* ein, T* eout, T* r, const T* ec0, const T* ec1) {
+    const auto& t = c->t_leg[d];
+    hipLaunchKernelGGL((k_leg<T, MODE, DOWN>), dim3(t.blocks), dim3(kLegThreads), 0, c->stream, c->segs(t), t.count,
+                       c->active, ein, eout, r, ec0, ec1, c->phi);
+}
+
 // Whether depth d runs its smoothing pairs as k_rb_sweep2 passes.
 template <typename T>
 bool two_sweep(const nyxpm_ctx* c, int d) {
@@ -1371,6 +1408,15 @@ int vcycle(nyxpm_ctx* c, bool* updated, bool sweep0_done = false, bool first = t
         if (tf.count == 0) continue;
         int cur = 0;
         const bool keep = !first && d == 0;
+        if (c->t_leg[d].count) {
+            cur = 1 - c->pre_buf[d];
+            Timed t(c, lvl_name("leg_down", d));
+            if (keep)
+                launch_leg<T, kSweepKeep, true>(c, d, eb[c->fin_buf[d]], eb[cur], r, eb[0], eb[1]);
+            else
+                launch_leg<T, 0, true>(c, d, eb[cur], eb[cur], r, eb[0], eb[1]);
+            continue;
+        }
         if (two_sweep<T>(c, d) && !(sweep0_done && d == 0)) {
             // both pre-smoothing sweeps in one pass, into the buffer the two
             // post-smoothing sweeps then read (so that they end in fin_buf)
@@ -1444,6 +1490,17 @@ int vcycle(nyxpm_ctx* c, bool* updated, bool sweep0_done = false, bool first = t
         auto& th = c->t_half[d];
         if (tf.count == 0) continue;
         int cur = c->pre_buf[d];
+        if (c->t_leg[d].count) {
+            cur = 1 - c->pre_buf[d];
+            const bool upd = last && d == 0 && c->fuse_update;
+            Timed t(c, lvl_name("leg_up", d));
+            if (upd)
+                launch_leg<T, kSweepUpdate, false>(c, d, eb[cur], eb[1 - cur], r, eb[0], eb[1]);
+            else
+                launch_leg<T, 0, false>(c, d, eb[cur], eb[1 - cur], r, eb[0], eb[1]);
+            if (upd) *updated = true;
+            continue;
+        }
         if (two_sweep<T>(c, d) && !(sweep0_done && d == 0)) {
             // both post-smoothing sweeps in one pass (prolongation on load), from
             // the pre-smoothing pass's buffer into fin_buf (or into phi)

@@ -115,19 +115,22 @@ def test_device_download_equals_host_download(nyx, npart, slack):
         check((0, 5))
 
 
+@pytest.mark.parametrize("sweep2", [0, 9])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("boxes", [
     [(64, 64, 64)],
+    [(8, 12, 64)],                # narrower than a leg's region
     [(72, 40, 24)],               # columns that overlap their neighbours in x and y
     [(36, 20, 16)],               # a narrow column shape, one level above the workgroup
     [(16, 8, 40)],                # the smallest shape
     [(5, 5, 5), (100, 36, 28)],   # a batch whose first box has no smoothing level
     [(144, 80, 48), (48, 64, 40)],
 ])
-def test_paired_smoothing_equals_half_sweeps(nyx, boxes, precision):
-    # smoothing pairs as one pass in both precisions and for every column choice,
-    # against separate half sweeps, bit for bit: the solves of two steps (the
-    # correction kept between grouped FP32 cycles, phi updated by the last pass)
+def test_paired_smoothing_equals_half_sweeps(nyx, boxes, precision, sweep2):
+    # whole cycle legs in one launch (sweep2 = 0, these sizes) and smoothing pairs as
+    # one pass (sweep2 = 9: uneven z-chunks of 9) in both precisions, against separate
+    # half sweeps, bit for bit: the solves of two steps (the correction kept between
+    # grouped FP32 cycles, phi updated by the last pass)
     r = np.random.default_rng(51)
     parts = []
     for n in boxes:
@@ -136,7 +139,7 @@ def test_paired_smoothing_equals_half_sweeps(nyx, boxes, precision):
     out = []
     for sm in ("fused", "half"):
         geoms = [nyx.BoxGeom(n, (0, 0, 0), tuple(v / 32 for v in n)) for n in boxes]
-        with nyx.PMContext(geoms, precision=precision, smoother=sm) as c:
+        with nyx.PMContext(geoms, precision=precision, smoother=sm, sweep2=sweep2) as c:
             for b, (pos, vel) in enumerate(parts):
                 c.upload(b, pos, vel, m_const=1e-3)
             c.pm_init()
