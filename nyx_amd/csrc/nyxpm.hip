@@ -230,9 +230,13 @@ struct nyxpm_ctx {
     int scan_blocks = 0;
     TileItem* items = nullptr;  // tile chunks of the last sort (tile-staged kernels)
     int* nitems = nullptr;
-    int* heavy = nullptr;       // tiles of more than kHeavyTile slots (deposit order)
-    int* nheavy = nullptr;
+    HeavyItem* heavy = nullptr; // tiles of more than kHeavyTile slots, or their parts (deposit order)
+    int* nheavy = nullptr;      // nitems + 1
+    int* nsplit = nullptr;      // nitems + 2: tiles deposited in parts
     int heavy_cap = 0;
+    unsigned long long* split_acc = nullptr;  // their accumulators (zero between deposits)
+    int* split_done = nullptr;                // parts arrived
+    int split_cap = 0;
     int* ndefer = nullptr;  // entries of the list handed from the tile-staged kick to k_kick_deferred
     // particle time step (estTimestep): per-box minimum as bits, kept by the closing
     // kicks when cfl > 0; valid for the state after the last such kick (a = dt_a)
@@ -1026,9 +1030,10 @@ int alloc_fields(nyxpm_ctx* c) {
     if ((rc = dalloc(c, &c->iters, nbox))) return rc;
     if ((rc = dalloc(c, &c->failed, nbox))) return rc;
     if ((rc = dalloc(c, &c->err_flag, 1))) return rc;
-    if ((rc = dalloc(c, &c->nitems, 1))) return rc;
-    if ((rc = dalloc(c, &c->nheavy, 1))) return rc;
-    HIPCK(c, hipMemset(c->nheavy, 0, sizeof(int)));
+    if ((rc = dalloc(c, &c->nitems, 3))) return rc;
+    c->nheavy = c->nitems + 1;
+    c->nsplit = c->nitems + 2;
+    HIPCK(c, hipMemset(c->nitems, 0, 3 * sizeof(int)));
     if ((rc = dalloc(c, &c->ndefer, 1))) return rc;
     if ((rc = dalloc(c, &c->dtmin, nbox))) return rc;
     if ((rc = dalloc(c, &c->nr, (size_t)nbox * kNormSlots))) return rc;
@@ -1071,6 +1076,8 @@ void free_particles(nyxpm_ctx* c) {
     dfree(c->key);
     dfree(c->items);
     dfree(c->heavy);
+    dfree(c->split_acc);
+    dfree(c->split_done);
 }
 
 // A particle buffer of n slots: one allocation, each array 256-byte aligned in it.
@@ -1126,12 +1133,66 @@ int phase_keys(nyxpm_ctx* c) {
     return NYXPM_OK;
 }
 
+// Words of a split tile's accumulator (two per LDS cell in FP64).
+int split_words(const nyxpm_ctx* c) { return 2 * (c->tile[0] + 1) * (c->tile[1] + 1) * (c->tile[2] + 1); }
+
+// The work item tables of a particle layout: kick items, heavy deposit blocks and the
+// accumulators of split tiles.
+struct ItemTables {
+    TileItem* items = nullptr;
+    HeavyItem* heavy = nullptr;
+    unsigned long long* split_acc = nullptr;
+    int* split_done = nullptr;
+    long long items_cap = 0, heavy_cap = 0, split_cap = 0;
+};
+
+// New tables for `slots` particle slots (the context's stay until set_items).
+int alloc_items(nyxpm_ctx* c, long long slots, ItemTables* t) {
+    t->items_cap = c->ntiles_total + slots / c->kick_chunk + 1;
+    if (t->items_cap > 0x7fffffffLL) FAIL(c, NYXPM_ERR_ARG, "too many tile chunks");
+    // a heavy tile's whole block stands for more than kHeavyTile slots, a part of a
+    // split one for at least 2/3 kSplitPart on average (three parts from 4097 slots,
+    // at least 4/5 of a longer part from four times its length)
+    t->heavy_cap = slots / (kSplitPart * 2 / 3) + 1;
+    t->split_cap = std::min<long long>(kSplitShare, slots / kSplitTile);
+    const size_t words = (size_t)t->split_cap * split_words(c);
+    int rc = dalloc(c, &t->items, t->items_cap);
+    if (!rc) rc = dalloc(c, &t->heavy, t->heavy_cap);
+    if (!rc) rc = dalloc(c, &t->split_acc, words);
+    if (!rc) rc = dalloc(c, &t->split_done, t->split_cap);
+    if (rc) {
+        dfree(t->items);
+        dfree(t->heavy);
+        dfree(t->split_acc);
+        dfree(t->split_done);
+        return rc;
+    }
+    if (t->split_cap) {
+        HIPCK(c, hipMemsetAsync(t->split_acc, 0, words * 8, c->stream));
+        HIPCK(c, hipMemsetAsync(t->split_done, 0, t->split_cap * sizeof(int), c->stream));
+    }
+    return NYXPM_OK;
+}
+
+// Into the context, which holds none (free_particles).
+void set_items(nyxpm_ctx* c, const ItemTables& t) {
+    c->items = t.items;
+    c->items_cap = t.items_cap;
+    c->heavy = t.heavy;
+    c->heavy_cap = (int)t.heavy_cap;
+    c->split_acc = t.split_acc;
+    c->split_done = t.split_done;
+    c->split_cap = (int)t.split_cap;
+}
+
 int make_items(nyxpm_ctx* c) {
     Timed t(c, "items");
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nitems, 1LL, 0);
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nheavy, 1LL, 0);
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nitems, 3LL, 0);
+    const long long split_min = std::max((long long)kSplitTile, c->npart_total / kSplitShare);
+    const int split_part = (int)std::max((long long)kSplitPart, c->npart_total / kSplitParts);
     hipLaunchKernelGGL(k_make_items, dim3(nblocks(c->ntiles_total)), dim3(kBlock), 0, c->stream, c->tbase,
-                       c->cursor, c->ntiles_total, c->items, c->nitems, c->kick_chunk, c->heavy, c->nheavy);
+                       c->cursor, c->ntiles_total, c->items, c->nitems, c->kick_chunk, c->heavy, c->nheavy,
+                       c->nsplit, split_min, split_part, c->split_cap);
     LAUNCHCK(c);
     c->items_valid = true;
     return NYXPM_OK;
@@ -1230,7 +1291,8 @@ int phase_deposit(nyxpm_ctx* c, bool want_rho, bool f32 = false) {
         Timed t(c, "deposit");
         hipLaunchKernelGGL(f32 ? k_deposit<true> : k_deposit<false>, dim3(c->heavy_cap + c->tseg_blocks),
                            dim3(kBlock), lds, c->stream, c->tseg, c->tseg_n, c->dboxes, c->tbase, c->cursor,
-                           c->heavy, c->nheavy, c->heavy_cap, A.x, A.y, A.z, A.m, c->own, c->halo, c->err_flag);
+                           c->heavy, c->nheavy, c->heavy_cap, c->split_acc, split_words(c), c->split_done, A.x,
+                           A.y, A.z, A.m, c->own, c->halo, c->err_flag);
     }
     {
         Timed t(c, "fold");
@@ -2049,7 +2111,7 @@ int nyxpm_destroy(nyxpm_ctx* c) {
     dfree(c->r64); dfree(c->e64); dfree(c->e64b); dfree(c->G64);
     dfree(c->r32); dfree(c->e32); dfree(c->e32b);
     dfree(c->active); dfree(c->iters); dfree(c->failed); dfree(c->err_flag); dfree(c->nitems); dfree(c->nr); dfree(c->nf);
-    dfree(c->ndefer); dfree(c->dtmin); dfree(c->nheavy);
+    dfree(c->ndefer); dfree(c->dtmin);
     dfree(c->state); dfree(c->solv); dfree(c->dv_size); dfree(c->dboxes);
     dfree(c->seg_pool); dfree(c->pseg); dfree(c->tseg); dfree(c->cc_first);
     dfree(c->gstat);
@@ -2202,23 +2264,13 @@ static int upload_impl(nyxpm_ctx* c, int box, int64_t np, const double* x, const
         }
     }
     HIPCK(c, hipStreamSynchronize(c->stream));
-    const long long icap = c->ntiles_total + slots / c->kick_chunk + 1;
-    if (icap > 0x7fffffffLL) FAIL(c, NYXPM_ERR_ARG, "too many tile chunks");
-    TileItem* nitm = nullptr;
-    if ((rc = dalloc(c, &nitm, icap))) return rc;
-    // a tile above kHeavyTile slots holds more than kHeavyTile particles or holes
-    const long long hcap = std::min<long long>(c->ntiles_total, slots / kHeavyTile + 1);
-    int* nheavy_list = nullptr;
-    if ((rc = dalloc(c, &nheavy_list, hcap))) return rc;
+    ItemTables tables;
+    if ((rc = alloc_items(c, slots, &tables))) return rc;
     free_particles(c);
     c->P[0] = N[0];
     c->P[1] = N[1];
     c->key = nkey;
-    c->items = nitm;
-    c->items_cap = icap;
-    dfree(c->heavy);
-    c->heavy = nheavy_list;
-    c->heavy_cap = (int)hcap;
+    set_items(c, tables);
     c->items_valid = false;
     c->dt_valid = false;
     c->cur = 0;
@@ -2663,8 +2715,8 @@ static int density_and_vels_impl(nyxpm_ctx* c, int box, double* dst, double* sum
     const int nbox = (int)c->boxes.size();
     const size_t lds = 2 * sizeof(unsigned long long) * (c->tile[0] + 1) * (c->tile[1] + 1) * (c->tile[2] + 1);
     hipLaunchKernelGGL(k_deposit<false>, dim3(c->heavy_cap + c->tseg_blocks), dim3(kBlock), lds, c->stream,
-                       c->tseg, c->tseg_n, c->dboxes, c->tbase, c->cursor, c->heavy, c->nheavy, c->heavy_cap, A.x,
-                       A.y, A.z, A.m, c->own, c->halo, c->err_flag);
+                       c->tseg, c->tseg_n, c->dboxes, c->tbase, c->cursor, c->heavy, c->nheavy, c->heavy_cap,
+                       c->split_acc, split_words(c), c->split_done, A.x, A.y, A.z, A.m, c->own, c->halo, c->err_flag);
     hipLaunchKernelGGL(k_fold_raw, dim3(c->t_res.blocks), dim3(kBlock), 0, c->stream, c->segs(c->t_res),
                        c->t_res.count, c->dboxes, c->own, c->halo, sums);
     // the per-box maxima start at zero on every call (the scratch keeps the last
@@ -3267,21 +3319,13 @@ static int retile_from(nyxpm_ctx* c, const int t[3], const ParticleSnapshot& s) 
         }
     }
     HIPCK(c, hipStreamSynchronize(c->stream));
-    const long long icap = c->ntiles_total + slots / c->kick_chunk + 1;
-    if (icap > 0x7fffffffLL) FAIL(c, NYXPM_ERR_ARG, "too many tile chunks");
-    TileItem* nitm = nullptr;
-    if ((rc = dalloc(c, &nitm, icap))) return rc;
-    const long long hcap = std::min<long long>(c->ntiles_total, slots / kHeavyTile + 1);
-    int* nheavy_list = nullptr;
-    if ((rc = dalloc(c, &nheavy_list, hcap))) return rc;
+    ItemTables tables;
+    if ((rc = alloc_items(c, slots, &tables))) return rc;
     free_particles(c);
     c->P[0] = N;
     c->P[1] = PartPtrs{};
     c->key = nkey;
-    c->items = nitm;
-    c->items_cap = icap;
-    c->heavy = nheavy_list;
-    c->heavy_cap = (int)hcap;
+    set_items(c, tables);
     c->items_valid = false;
     c->dt_valid = false;
     c->cur = 0;

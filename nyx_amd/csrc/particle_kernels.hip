@@ -81,6 +81,22 @@ __device__ __forceinline__ double empty_slot() { return __longlong_as_double(0x7
 
 // Slots above which a tile's deposit block is launched ahead of the others.
 constexpr int kHeavyTile = 2048;
+// A tile with more than kSplitTile slots and more than 1/kSplitShare of all particles
+// (so about kSplitShare tiles at most) is deposited by several blocks, which add their
+// fixed-point sums in global memory: one block takes ~3.7 ns a slot, the whole chip
+// ~17 ps, so such a tile alone holds the launch for about as long as everything else
+// (131 us for a clump of 35000 in 10^6 particles).  Below that share the blocks of the
+// other tiles hide it, and the parts' additions (2754 64-bit atomics each, ~30 per ns)
+// cost more than they save; parts of at least kSplitPart slots and 1/kSplitParts of
+// all particles keep them to ~100 us at the most.  At 2 10^7 particles, splitting the
+// tiles above 1/1024 into parts of 2048 took 900 us, none 340 us.
+constexpr int kSplitTile = 4096, kSplitPart = 2048, kSplitShare = 256, kSplitParts = 1024;
+
+// One block of the deposit ahead of the ordinary tiles: `len` slots from `off` of a
+// heavy tile, one of nparts pieces (1: the whole tile); split: the tile's accumulator.
+struct HeavyItem {
+    int tile, off, len, nparts, split;
+};
 
 // i / T for 0 <= i < 2^17 and T <= 32 with magic = ceil(2^31 / T) (exact over that
 // range; the bound is checked when a context is created).
@@ -292,6 +308,28 @@ __device__ __forceinline__ unsigned fx32_units(float w, float scale) {
     return __float2uint_rz(w * scale + 0.5f);
 }
 
+// The parts of a split tile: adds the block's LDS words to the tile's accumulator
+// (integers: exact in any order); the last part to arrive takes the sums back into
+// LDS, leaving the accumulator and its counter at zero for the next deposit, and
+// returns true.
+__device__ __forceinline__ bool split_combine(unsigned long long* acc, int words, const HeavyItem& hv,
+                                              unsigned long long* split_acc, int split_words, int* split_done) {
+    __shared__ int s_last;
+    unsigned long long* g = split_acc + (size_t)hv.split * split_words;
+    for (int c = threadIdx.x; c < words; c += blockDim.x)
+        if (acc[c]) atomicAdd(&g[c], acc[c]);
+    __threadfence();  // every addition before the arrival
+    __syncthreads();
+    if (threadIdx.x == 0) s_last = atomicAdd(&split_done[hv.split], 1) == hv.nparts - 1;
+    __syncthreads();
+    if (!s_last) return false;
+    __threadfence();
+    for (int c = threadIdx.x; c < words; c += blockDim.x) acc[c] = atomicExch(&g[c], 0ull);
+    if (threadIdx.x == 0) atomicExch(&split_done[hv.split], 0);
+    __syncthreads();
+    return true;
+}
+
 // One block per tile.  Contributions m*sx[ii]*sy[jj]*sz[kk] (amrex_deposit_cic
 // weights, product left to right) of the tile's particles go to LDS as fixed
 // point; interior cells are written to `own`, the low halo layer to `halo`.
@@ -307,18 +345,22 @@ template <bool F32>
 __global__ void __launch_bounds__(kBlock) k_deposit(const BoxSeg* segs, int nseg, const BoxDev* boxes,
                                                     const long long* __restrict__ tbase,
                                                     const int* __restrict__ thw,
-                                                    const int* __restrict__ heavy, const int* nheavy,
-                                                    int heavy_cap,
+                                                    const HeavyItem* __restrict__ heavy, const int* nheavy,
+                                                    int heavy_cap, unsigned long long* split_acc, int split_words,
+                                                    int* split_done,
                                                     const double* __restrict__ x, const double* __restrict__ y,
                                                     const double* __restrict__ z, const double* __restrict__ m,
                                                     double* __restrict__ own, double* __restrict__ halo, int* err) {
     extern __shared__ unsigned long long acc[];
-    // the first heavy_cap blocks take the heavy tiles (listed by k_make_items), so
-    // the longest blocks start first; the rest take every other tile in order
+    // the first heavy_cap blocks take the heavy tiles or their parts (listed by
+    // k_make_items), so the longest blocks start first; the rest take every other
+    // tile in order
     int tile;
+    HeavyItem hv{0, 0, 0, 1, -1};
     if ((int)blockIdx.x < heavy_cap) {
         if ((int)blockIdx.x >= *nheavy) return;
-        tile = heavy[blockIdx.x];
+        hv = heavy[blockIdx.x];
+        tile = hv.tile;
     } else {
         tile = blockIdx.x - heavy_cap;
         if (thw[tile] > kHeavyTile) return;
@@ -335,7 +377,11 @@ __global__ void __launch_bounds__(kBlock) k_deposit(const BoxSeg* segs, int nseg
     const int Lx = bx + 1, Ly = by + 1, Lz = bz + 1;
     const int LC = Lx * Ly * Lz;
     const long long gt = B.tile_off + lt;
-    const long long p0 = tbase[gt], p1 = p0 + thw[gt];
+    long long p0 = tbase[gt], p1 = p0 + thw[gt];
+    if (hv.nparts > 1) {
+        p0 += hv.off;
+        p1 = p0 + hv.len;
+    }
     // the thread's first two particles are loaded before the accumulator is
     // cleared, so their latency overlaps the clearing
     double xa = 0.0, ya = 0.0, za = 0.0, ma = 0.0, xb = 0.0, yb = 0.0, zb = 0.0, mb = 0.0;
@@ -423,6 +469,7 @@ __global__ void __launch_bounds__(kBlock) k_deposit(const BoxSeg* segs, int nseg
         if (pa + kBlock < p1) dep(xb, yb, zb, mb);
     }
     __syncthreads();
+    if (hv.nparts > 1 && !split_combine(acc, F32 ? LC : 2 * LC, hv, split_acc, split_words, split_done)) return;
     // write-out by rows of Lx cells (Lx <= 33 < 64): a wave takes rpw rows per
     // pass, so no cell needs a division for its coordinates
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
@@ -951,7 +998,8 @@ struct TileItem {
 __global__ void __launch_bounds__(kBlock) k_make_items(const long long* __restrict__ tbase,
                                                        const int* __restrict__ thw, long long ntiles,
                                                        TileItem* __restrict__ items, int* nitems, int chunk,
-                                                       int* __restrict__ heavy, int* nheavy) {
+                                                       HeavyItem* __restrict__ heavy, int* nheavy, int* nsplit,
+                                                       long long split_min, int split_part, int split_cap) {
     const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
     int nc = 0;
     long long p0 = 0, cnt = 0;
@@ -959,8 +1007,20 @@ __global__ void __launch_bounds__(kBlock) k_make_items(const long long* __restri
         p0 = tbase[t];
         cnt = thw[t];
         nc = (int)((cnt + chunk - 1) / chunk);
-        // tiles the deposit starts first (one block per tile: the longest blocks)
-        if (cnt > kHeavyTile) heavy[atomicAdd(nheavy, 1)] = (int)t;
+        // tiles the deposit starts first (the longest blocks), the heaviest in parts
+        if (cnt > kHeavyTile) {
+            int split = -1, parts = 1, len = (int)cnt;
+            if (cnt > split_min) split = atomicAdd(nsplit, 1);
+            if (split >= split_cap) split = -1;
+            if (split >= 0) {
+                len = split_part;
+                parts = (int)((cnt + len - 1) / len);
+            }
+            const int h = atomicAdd(nheavy, parts);
+            for (int q = 0; q < parts; ++q)
+                heavy[h + q] = HeavyItem{(int)t, q * len, (int)min((long long)len, cnt - (long long)q * len), parts,
+                                         split};
+        }
     }
     // wave-inclusive prefix of nc, one atomic per wave
     const int lane = threadIdx.x & (kWave - 1);

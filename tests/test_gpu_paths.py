@@ -148,3 +148,31 @@ def test_paired_smoothing_equals_half_sweeps(nyx, boxes, precision, sweep2):
                                                                              for x in sum(map(list, c.download(b)), [])])
     for a, b in zip(*out):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("npart", [4096, 4097, 30011])
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_split_tile_deposit(nyx, orc, npart, precision):
+    # a clump inside one tile: one block up to 4096 slots, above that parts whose
+    # fixed-point sums meet in global memory.  AssignDensity (FP64 weights) against
+    # the oracle, repeated (the accumulators are zero again) and through other tile
+    # shapes; the step's deposit (FP32 weights in mixed precision, the interpolation
+    # error of a weight is below 4 roundings of 2^-24) through the right-hand side
+    r = np.random.default_rng(61)
+    n = (32, 32, 32)
+    pos = [(9.0 + 5.0 * r.random(npart)) / 32 for _ in range(3)]
+    pos = [np.concatenate([p, r.random(2000)]) for p in pos]
+    m = 0.5 + r.random(npart + 2000)
+    ref = orc.deposit(n, (0, 0, 0), (1, 1, 1), *pos, m=m)
+    with ctx1(nyx, n, precision=precision) as c, ctx1(nyx, n, tile=(32, 8, 4), precision=precision) as c2:
+        for q in (c, c2):
+            q.upload(0, pos, [np.zeros_like(m)] * 3, m=m)
+        rho = c.assign_density()
+        assert np.abs(rho - ref).max() <= 1e-13 * ref.max()
+        assert np.array_equal(c.assign_density(), rho)
+        assert np.abs(c2.assign_density() - ref).max() <= 1e-13 * ref.max()
+        c.pm_init()
+        rhs = -(ref - ref.mean())
+        tol = 1e-13 if precision == "fp64" else 4 * 2.0 ** -24
+        assert np.abs(c.get_rhs() - rhs).max() <= tol * ref.max()
+        assert np.array_equal(c.assign_density(), rho)
