@@ -227,6 +227,10 @@ struct nyxpm_ctx {
     int* mig = nullptr;           // k_migrate flags: overflow, moved
     int* h_mig = nullptr;         // pinned mirror
     long long* bsum = nullptr;
+    // AssignDensityAndVels: halo slots of the three momentum deposits (allocated by the
+    // first call, with the tile's size) and the per-box maxima
+    double* mom_halo = nullptr;
+    unsigned long long* mom_max = nullptr;
     int scan_blocks = 0;
     TileItem* items = nullptr;  // tile chunks of the last sort (tile-staged kernels)
     int* nitems = nullptr;
@@ -1006,6 +1010,7 @@ int alloc_tile_buffers(nyxpm_ctx* c) {
 void free_tile_buffers(nyxpm_ctx* c) {
     dfree(c->halo); dfree(c->counts); dfree(c->cursor); dfree(c->tstart);
     dfree(c->tbase); dfree(c->tcap); dfree(c->bsum);
+    dfree(c->mom_halo);
 }
 
 int alloc_fields(nyxpm_ctx* c) {
@@ -1036,6 +1041,7 @@ int alloc_fields(nyxpm_ctx* c) {
     HIPCK(c, hipMemset(c->nitems, 0, 3 * sizeof(int)));
     if ((rc = dalloc(c, &c->ndefer, 1))) return rc;
     if ((rc = dalloc(c, &c->dtmin, nbox))) return rc;
+    if ((rc = dalloc(c, &c->mom_max, 3 * nbox))) return rc;
     if ((rc = dalloc(c, &c->nr, (size_t)nbox * kNormSlots))) return rc;
     if ((rc = dalloc(c, &c->nf, (size_t)nbox * kNormSlots))) return rc;
     if ((rc = dalloc(c, &c->state, 4 * nbox))) return rc;
@@ -1155,11 +1161,12 @@ int alloc_items(nyxpm_ctx* c, long long slots, ItemTables* t) {
     // at least 4/5 of a longer part from four times its length)
     t->heavy_cap = slots / (kSplitPart * 2 / 3) + 1;
     t->split_cap = std::min<long long>(kSplitShare, slots / kSplitTile);
-    const size_t words = (size_t)t->split_cap * split_words(c);
+    // (three accumulators per split tile: the momentum deposit's components)
+    const size_t words = (size_t)t->split_cap * 3 * split_words(c);
     int rc = dalloc(c, &t->items, t->items_cap);
     if (!rc) rc = dalloc(c, &t->heavy, t->heavy_cap);
     if (!rc) rc = dalloc(c, &t->split_acc, words);
-    if (!rc) rc = dalloc(c, &t->split_done, t->split_cap);
+    if (!rc) rc = dalloc(c, &t->split_done, 3 * t->split_cap);
     if (rc) {
         dfree(t->items);
         dfree(t->heavy);
@@ -1169,7 +1176,7 @@ int alloc_items(nyxpm_ctx* c, long long slots, ItemTables* t) {
     }
     if (t->split_cap) {
         HIPCK(c, hipMemsetAsync(t->split_acc, 0, words * 8, c->stream));
-        HIPCK(c, hipMemsetAsync(t->split_done, 0, t->split_cap * sizeof(int), c->stream));
+        HIPCK(c, hipMemsetAsync(t->split_done, 0, 3 * t->split_cap * sizeof(int), c->stream));
     }
     return NYXPM_OK;
 }
@@ -1291,8 +1298,8 @@ int phase_deposit(nyxpm_ctx* c, bool want_rho, bool f32 = false) {
         Timed t(c, "deposit");
         hipLaunchKernelGGL(f32 ? k_deposit<true> : k_deposit<false>, dim3(c->heavy_cap + c->tseg_blocks),
                            dim3(kBlock), lds, c->stream, c->tseg, c->tseg_n, c->dboxes, c->tbase, c->cursor,
-                           c->heavy, c->nheavy, c->heavy_cap, c->split_acc, split_words(c), c->split_done, A.x,
-                           A.y, A.z, A.m, c->own, c->halo, c->err_flag);
+                           c->heavy, c->nheavy, c->heavy_cap, c->split_acc, split_words(c), c->split_done,
+                           c->split_cap, A.x, A.y, A.z, A.m, c->own, c->halo, c->err_flag, DepositMom{});
     }
     {
         Timed t(c, "fold");
@@ -2103,7 +2110,7 @@ int nyxpm_destroy(nyxpm_ctx* c) {
     if (c->graph) hipGraphDestroy(c->graph);
     free_particles(c);
     dfree(c->counts); dfree(c->cursor); dfree(c->tstart); dfree(c->bsum);
-    dfree(c->tbase); dfree(c->tcap); dfree(c->nmove); dfree(c->mig); dfree(c->phi_prev); dfree(c->guess_ok);
+    dfree(c->tbase); dfree(c->tcap); dfree(c->mom_halo); dfree(c->mom_max); dfree(c->nmove); dfree(c->mig); dfree(c->phi_prev); dfree(c->guess_ok);
     if (c->h_mig) hipHostFree(c->h_mig);
     c->rho = nullptr;
     dfree(c->own); dfree(c->halo); dfree(c->f); dfree(c->phi); dfree(c->partial);
@@ -2703,40 +2710,36 @@ int nyxpm_assign_density(nyxpm_ctx* c, int box, double* rho_out) {
     return err_check(c);
 }
 
-// AssignDensityAndVels into `out` (4 fields of box `box`'s cells, device memory
-// when dst_dev, else written through the device buffer dst) with the given
-// scratch: sums (4 N: folded mass and momenta of every box), mown (N) and mhalo
-// (H) for the momentum deposit, maxbits (3 per box).  Stream-ordered; the
-// caller synchronises.
-static int density_and_vels_impl(nyxpm_ctx* c, int box, double* dst, double* sums, double* mown, double* mhalo,
-                                 unsigned long long* maxbits) {
+// AssignDensityAndVels of box `box` into dst (4 fields of its cells, device memory).
+// The momentum deposits' own cells go to the FP64 multigrid pools, which hold nothing
+// between solves.  Stream-ordered; the caller synchronises.
+static int density_and_vels_impl(nyxpm_ctx* c, int box, double* dst) {
     PartPtrs& A = c->P[c->cur];
-    const long long N = c->ncell_total;
     const int nbox = (int)c->boxes.size();
+    const long long H = (long long)c->ntiles_total * c->halo_stride;
+    int rc;
+    if (!c->mom_halo && (rc = dalloc(c, &c->mom_halo, 3 * H))) return rc;
     const size_t lds = 2 * sizeof(unsigned long long) * (c->tile[0] + 1) * (c->tile[1] + 1) * (c->tile[2] + 1);
-    hipLaunchKernelGGL(k_deposit<false>, dim3(c->heavy_cap + c->tseg_blocks), dim3(kBlock), lds, c->stream,
-                       c->tseg, c->tseg_n, c->dboxes, c->tbase, c->cursor, c->heavy, c->nheavy, c->heavy_cap,
-                       c->split_acc, split_words(c), c->split_done, A.x, A.y, A.z, A.m, c->own, c->halo, c->err_flag);
-    hipLaunchKernelGGL(k_fold_raw, dim3(c->t_res.blocks), dim3(kBlock), 0, c->stream, c->segs(c->t_res),
-                       c->t_res.count, c->dboxes, c->own, c->halo, sums);
-    // the per-box maxima start at zero on every call (the scratch keeps the last
-    // call's contents)
-    hipLaunchKernelGGL(k_fill_dbl, dim3(1), dim3(kBlock), 0, c->stream, reinterpret_cast<double*>(maxbits),
+    const dim3 grid(c->heavy_cap + c->tseg_blocks);
+    hipLaunchKernelGGL(k_deposit<false>, grid, dim3(kBlock), lds, c->stream, c->tseg, c->tseg_n, c->dboxes,
+                       c->tbase, c->cursor, c->heavy, c->nheavy, c->heavy_cap, c->split_acc, split_words(c),
+                       c->split_done, c->split_cap, A.x, A.y, A.z, A.m, c->own, c->halo, c->err_flag, DepositMom{});
+    // the per-box maxima start at zero on every call
+    hipLaunchKernelGGL(k_fill_dbl, dim3(1), dim3(kBlock), 0, c->stream, reinterpret_cast<double*>(c->mom_max),
                        (long long)(3 * nbox), 0.0);
     if (c->pseg_blocks > 0)
         hipLaunchKernelGGL(k_max_mom, dim3(c->pseg_blocks), dim3(kBlock), 0, c->stream, c->pseg, c->pseg_n,
-                           c->dboxes, A.x, A.m, A.vx, A.vy, A.vz, maxbits);
-    const double* vel[3] = {A.vx, A.vy, A.vz};
-    for (int d = 0; d < 3; ++d) {
-        hipLaunchKernelGGL(k_deposit_mom, dim3(c->tseg_blocks), dim3(kBlock), lds, c->stream, c->tseg, c->tseg_n,
-                           c->dboxes, c->tbase, c->cursor, A.x, A.y, A.z, A.m, vel[d], maxbits, d, mown, mhalo,
-                           c->err_flag);
-        hipLaunchKernelGGL(k_fold_raw, dim3(c->t_res.blocks), dim3(kBlock), 0, c->stream, c->segs(c->t_res),
-                           c->t_res.count, c->dboxes, mown, mhalo, sums + (d + 1) * N);
-    }
-    const long long nc = c->boxes[box].lev[0].nc;
-    hipLaunchKernelGGL(k_vels_finish, dim3(nblocks(nc)), dim3(kBlock), 0, c->stream, c->dboxes, box, sums,
-                       sums + N, N, dst);
+                           c->dboxes, A.x, A.m, A.vx, A.vy, A.vz, c->mom_max);
+    const DepositMom mom{{A.vx, A.vy, A.vz}, c->mom_max, {c->r64, c->e64, c->e64b},
+                         {c->mom_halo, c->mom_halo + H, c->mom_halo + 2 * H}};
+    hipLaunchKernelGGL((k_deposit<false, true>), dim3(grid.x, 3), dim3(kBlock), lds, c->stream, c->tseg, c->tseg_n,
+                       c->dboxes, c->tbase, c->cursor, c->heavy, c->nheavy, c->heavy_cap, c->split_acc,
+                       split_words(c), c->split_done, c->split_cap, A.x, A.y, A.z, A.m, c->own, c->halo,
+                       c->err_flag, mom);
+    const FoldFields<4> fields{{c->own, mom.own[0], mom.own[1], mom.own[2]},
+                               {c->halo, mom.halo[0], mom.halo[1], mom.halo[2]}};
+    hipLaunchKernelGGL(k_fold_vels, dim3(c->seg_host[c->t_res.first + box].nblk), dim3(kBlock), 0, c->stream,
+                       c->segs(c->t_res) + box, c->dboxes, fields, dst);
     LAUNCHCK(c);
     return NYXPM_OK;
 }
@@ -2747,35 +2750,11 @@ int nyxpm_assign_density_and_vels(nyxpm_ctx* c, int box, double* out) {
     if ((rc = require_particles(c))) return rc;
     if ((rc = check_box(c, box))) return rc;
     if (!c->sorted_valid && (rc = phase_sort(c))) return rc;
-    const long long N = c->ncell_total;
-    const long long H = (long long)c->ntiles_total * c->halo_stride;
-    const int nbox = (int)c->boxes.size();
-    // scratch: mass and three momentum sums (all boxes), the momentum deposit's
-    // own/halo cells, the per-box maxima
-    double *sums = nullptr, *mown = nullptr, *mhalo = nullptr;
-    unsigned long long* maxbits = nullptr;
-    auto release = [&]() {
-        const long long bytes = (sums ? 4 * N * 8 : 0) + (mown ? N * 8 : 0) + (mhalo ? std::max(H, 1LL) * 8 : 0) +
-                                (maxbits ? 3LL * nbox * 8 : 0);
-        dfree(sums);
-        dfree(mown);
-        dfree(mhalo);
-        dfree(maxbits);
-        c->device_bytes -= bytes;
-    };
-    if ((rc = dalloc(c, &sums, 4 * N)) || (rc = dalloc(c, &mown, N)) || (rc = dalloc(c, &mhalo, std::max(H, 1LL))) ||
-        (rc = dalloc(c, &maxbits, 3 * nbox))) {
-        release();
-        return rc;
-    }
     const long long nc = c->boxes[box].lev[0].nc;
     const bool dev = is_device_ptr(out);
     double* dst = out;
-    if (!dev && (rc = dalloc(c, &dst, 4 * nc))) {
-        release();
-        return rc;
-    }
-    rc = density_and_vels_impl(c, box, dst, sums, mown, mhalo, maxbits);
+    if (!dev && (rc = dalloc(c, &dst, 4 * nc))) return rc;
+    rc = density_and_vels_impl(c, box, dst);
     hipError_t e = rc ? hipSuccess : hipGetLastError();
     if (!rc && !dev && e == hipSuccess)
         e = hipMemcpyAsync(out, dst, 4 * nc * sizeof(double), hipMemcpyDeviceToHost, c->stream);
@@ -2784,7 +2763,6 @@ int nyxpm_assign_density_and_vels(nyxpm_ctx* c, int box, double* out) {
         dfree(dst);
         c->device_bytes -= 4 * nc * (long long)sizeof(double);
     }
-    release();
     // the deposit buffers now hold raw mass, not rho
     c->density_valid = false;
     c->f1_valid = false;

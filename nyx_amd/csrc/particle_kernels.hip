@@ -341,17 +341,38 @@ __device__ __forceinline__ bool split_combine(unsigned long long* acc, int words
 // and order independent, with half the atomics: a cell's sum of at most 2^32
 // contributions below 2^32 units each stays below 2^64.  Per contribution the
 // FP32 rounding (~6e-8 relative) dominates the unit (2^-31 of the largest mass).
-template <bool F32>
+//
+// MOM (AssignDensityAndVels, FP64): velocity component blockIdx.y, contributions
+// (sx*sy*sz*m) * v_d as signed fixed point (two's complement in the u64 words, hi in
+// units 2^(E-30) converted through int32, lo in 2^(E-62), 2^E <= max |m v_d| of the
+// box, from maxbits), exact and order independent like the mass deposit's.  The
+// three components are one launch (a launch each, one block per tile: 3 x 287 us for
+// 2 10^6 clustered particles, held by the heaviest tile).
+struct DepositMom {
+    const double* v[3];                 // vx, vy, vz
+    const unsigned long long* maxbits;  // max |m v_d| per box and component
+    double* own[3];                     // per component
+    double* halo[3];
+};
+template <bool F32, bool MOM = false>
 __global__ void __launch_bounds__(kBlock) k_deposit(const BoxSeg* segs, int nseg, const BoxDev* boxes,
                                                     const long long* __restrict__ tbase,
                                                     const int* __restrict__ thw,
                                                     const HeavyItem* __restrict__ heavy, const int* nheavy,
                                                     int heavy_cap, unsigned long long* split_acc, int split_words,
-                                                    int* split_done,
+                                                    int* split_done, int split_cap,
                                                     const double* __restrict__ x, const double* __restrict__ y,
                                                     const double* __restrict__ z, const double* __restrict__ m,
-                                                    double* __restrict__ own, double* __restrict__ halo, int* err) {
+                                                    double* __restrict__ own, double* __restrict__ halo, int* err,
+                                                    DepositMom mom = {}) {
+    static_assert(!(F32 && MOM), "momenta are deposited in FP64");
     extern __shared__ unsigned long long acc[];
+    const int comp = MOM ? (int)blockIdx.y : 0;
+    const double* __restrict__ vel = MOM ? mom.v[comp] : nullptr;
+    if (MOM) {
+        own = mom.own[comp];
+        halo = mom.halo[comp];
+    }
     // the first heavy_cap blocks take the heavy tiles or their parts (listed by
     // k_make_items), so the longest blocks start first; the rest take every other
     // tile in order
@@ -385,25 +406,32 @@ __global__ void __launch_bounds__(kBlock) k_deposit(const BoxSeg* segs, int nseg
     // the thread's first two particles are loaded before the accumulator is
     // cleared, so their latency overlaps the clearing
     double xa = 0.0, ya = 0.0, za = 0.0, ma = 0.0, xb = 0.0, yb = 0.0, zb = 0.0, mb = 0.0;
+    double va = 0.0, vb = 0.0;
     auto load2 = [&](long long pa) {
         const long long pb = pa + kBlock;
         if (pa < p1) {
             xa = x[pa]; ya = y[pa]; za = z[pa];
             ma = B.has_mass ? m[pa] : B.m_const;
+            if (MOM) va = vel[pa];
         }
         if (pb < p1) {
             xb = x[pb]; yb = y[pb]; zb = z[pb];
             mb = B.has_mass ? m[pb] : B.m_const;
+            if (MOM) vb = vel[pb];
         }
     };
     load2(p0 + threadIdx.x);
     for (int c = threadIdx.x; c < (F32 ? LC : 2 * LC); c += kBlock) acc[c] = 0ull;
     __syncthreads();
-    const int E = B.fx_exp;
+    int E = B.fx_exp;
+    if (MOM) {
+        const double vmax = __longlong_as_double((long long)mom.maxbits[3 * sg.box + comp]);
+        E = vmax > 0.0 ? ilogb(vmax) : 0;
+    }
     // one particle's CIC contributions as two fixed-point words: w * 2^(31-E) =
     // hi + lo * 2^-32 (hi < 2^32 since w < 2^(E+1); lo rounded, a rounding up to
     // 2^32 carried into hi), both converted with the native f64 -> u32 instruction
-    auto dep = [&](double px, double py, double pz, double mp) {
+    auto dep = [&](double px, double py, double pz, double mp, double vp) {
         if (isnan(px)) return;  // empty slot
         double xint, yint, zint;
         const int i = cic_index(px, B.plo[0], B.dxi[0], &xint);
@@ -451,11 +479,13 @@ __global__ void __launch_bounds__(kBlock) k_deposit(const BoxSeg* segs, int nseg
 #pragma unroll
                 for (int ii = 0; ii < 2; ++ii) {
                     const double w = sx[ii] * sy[jj] * sz[kk] * mp;
-                    const double s = ldexp(w, 31 - E);
+                    const double s = MOM ? ldexp(w * vp, 30 - E) : ldexp(w, 31 - E);  // MOM: |s| < 2^31
                     const double hf = floor(s);
                     const double lr = rint(ldexp(s - hf, 32));
                     const bool carry = lr >= 4294967296.0;
-                    const unsigned long long hi = (unsigned long long)(unsigned)hf + (carry ? 1ull : 0ull);
+                    const unsigned long long hi =
+                        MOM ? (unsigned long long)((long long)(int)hf + (carry ? 1 : 0))
+                            : (unsigned long long)(unsigned)hf + (carry ? 1ull : 0ull);
                     const unsigned long long lo = carry ? 0ull : (unsigned long long)(unsigned)lr;
                     const int idx = ((kw + kk) * Ly + (jw + jj)) * Lx + (iw + ii);
                     atomicAdd(&acc[idx], hi);
@@ -465,10 +495,11 @@ __global__ void __launch_bounds__(kBlock) k_deposit(const BoxSeg* segs, int nseg
     // two particles per thread, both loaded before either is deposited
     for (long long pa = p0 + threadIdx.x; pa < p1; pa += 2 * kBlock) {
         if (pa != p0 + threadIdx.x) load2(pa);
-        dep(xa, ya, za, ma);
-        if (pa + kBlock < p1) dep(xb, yb, zb, mb);
+        dep(xa, ya, za, ma, va);
+        if (pa + kBlock < p1) dep(xb, yb, zb, mb, vb);
     }
     __syncthreads();
+    if (MOM && hv.split >= 0) hv.split += comp * split_cap;
     if (hv.nparts > 1 && !split_combine(acc, F32 ? LC : 2 * LC, hv, split_acc, split_words, split_done)) return;
     // write-out by rows of Lx cells (Lx <= 33 < 64): a wave takes rpw rows per
     // pass, so no cell needs a division for its coordinates
@@ -482,8 +513,9 @@ __global__ void __launch_bounds__(kBlock) k_deposit(const BoxSeg* segs, int nseg
         const int dly = step % Ly, dlz = step / Ly;
         while (lz < Lz) {
             const int c = (lz * Ly + ly) * Lx + lx;
-            const double v = F32 ? ldexp((double)acc[c], E - 31)
-                                 : ldexp((double)acc[c], E - 31) + ldexp((double)acc[LC + c], E - 63);
+            const double v = F32   ? ldexp((double)acc[c], E - 31)
+                             : MOM ? ldexp((double)(long long)acc[c], E - 30) + ldexp((double)acc[LC + c], E - 62)
+                                   : ldexp((double)acc[c], E - 31) + ldexp((double)acc[LC + c], E - 63);
             if (lx > 0 && ly > 0 && lz > 0)
                 own[B.cell_off + cidx(o0 + lx - 1, o1 + ly - 1, o2 + lz - 1, B.n[0], B.n[1])] = v;
             else
@@ -498,99 +530,40 @@ __global__ void __launch_bounds__(kBlock) k_deposit(const BoxSeg* segs, int nseg
     }
 }
 
-// Momentum deposit for AssignDensityAndVels: one velocity component per launch,
-// contributions (sx*sy*sz*m) * v_d as signed fixed point (two's complement in
-// the u64 words, hi in units 2^(E-30) converted through int32, lo in 2^(E-62),
-// 2^E <= max |m v_d| of the box, from maxbits), so the sums are exact and order
-// independent like the mass deposit's; own cells to `own`, the low halo layer to
-// `halo` (k_deposit's layout).
-__global__ void __launch_bounds__(kBlock) k_deposit_mom(const BoxSeg* segs, int nseg, const BoxDev* boxes,
-                                                        const long long* __restrict__ tbase,
-                                                        const int* __restrict__ thw,
-                                                        const double* __restrict__ x, const double* __restrict__ y,
-                                                        const double* __restrict__ z, const double* __restrict__ m,
-                                                        const double* __restrict__ v,
-                                                        const unsigned long long* maxbits, int comp,
-                                                        double* __restrict__ own, double* __restrict__ halo,
-                                                        int* err) {
-    extern __shared__ unsigned long long acc[];
-    const BoxSeg sg = segs[find_seg(segs, nseg, blockIdx.x)];
-    const BoxDev B = boxes[__builtin_amdgcn_readfirstlane(sg.box)];
-    const int lt = blockIdx.x - sg.blk0;
-    const int tx = lt % B.ntile[0], ty = (lt / B.ntile[0]) % B.ntile[1], tz = lt / (B.ntile[0] * B.ntile[1]);
-    const int o0 = tx * B.tile[0], o1 = ty * B.tile[1], o2 = tz * B.tile[2];
-    const int bx = min(B.tile[0], B.n[0] - o0), by = min(B.tile[1], B.n[1] - o1), bz = min(B.tile[2], B.n[2] - o2);
-    const int Lx = bx + 1, Ly = by + 1, Lz = bz + 1;
-    const int LC = Lx * Ly * Lz;
-    for (int c = threadIdx.x; c < 2 * LC; c += kBlock) acc[c] = 0ull;
+// atomicMax of a block's largest value (bit patterns), skipped where the slot already
+// holds as much: the slot only grows, so a stale read costs an atomic at most (one
+// atomic per block on one word took ~12 ns each, one per particle 1.2 ms in all).
+__device__ __forceinline__ void block_max_to(unsigned long long v, unsigned long long* slot) {
+    for (int o = kWave / 2; o > 0; o >>= 1) v = max(v, (unsigned long long)__shfl_xor((long long)v, o));
+    __shared__ unsigned long long wmax[kBlock / kWave];
     __syncthreads();
-    const long long gt = B.tile_off + lt;
-    const long long p0 = tbase[gt], p1 = p0 + thw[gt];
-    const double vmax = __longlong_as_double((long long)maxbits[3 * sg.box + comp]);
-    const int E = vmax > 0.0 ? ilogb(vmax) : 0;
-    for (long long p = p0 + threadIdx.x; p < p1; p += kBlock) {
-        const double px = x[p];
-        if (isnan(px)) continue;  // empty slot
-        double xint, yint, zint;
-        const int i = cic_index(px, B.plo[0], B.dxi[0], &xint);
-        const int j = cic_index(y[p], B.plo[1], B.dxi[1], &yint);
-        const int k = cic_index(z[p], B.plo[2], B.dxi[2], &zint);
-        const int iw = wrap_checked(i, B.n[0], err) - o0;
-        const int jw = wrap_checked(j, B.n[1], err) - o1;
-        const int kw = wrap_checked(k, B.n[2], err) - o2;
-        if (iw < 0 || iw >= bx || jw < 0 || jw >= by || kw < 0 || kw >= bz) {
-            atomicOr(err, 2);
-            continue;
-        }
-        const double sx[2] = {1.0 - xint, xint};
-        const double sy[2] = {1.0 - yint, yint};
-        const double sz[2] = {1.0 - zint, zint};
-        const double mp = B.has_mass ? m[p] : B.m_const;
-        const double vp = v[p];
-#pragma unroll
-        for (int kk = 0; kk < 2; ++kk)
-#pragma unroll
-            for (int jj = 0; jj < 2; ++jj)
-#pragma unroll
-                for (int ii = 0; ii < 2; ++ii) {
-                    const double w = sx[ii] * sy[jj] * sz[kk] * mp;
-                    const double s = ldexp(w * vp, 30 - E);  // |s| < 2^31
-                    const double hf = floor(s);
-                    const double lr = rint(ldexp(s - hf, 32));
-                    const bool carry = lr >= 4294967296.0;
-                    const long long hi = (long long)(int)hf + (carry ? 1 : 0);
-                    const unsigned long long lo = carry ? 0ull : (unsigned long long)(unsigned)lr;
-                    const int idx = ((kw + kk) * Ly + (jw + jj)) * Lx + (iw + ii);
-                    atomicAdd(&acc[idx], (unsigned long long)hi);
-                    atomicAdd(&acc[LC + idx], lo);
-                }
-    }
+    if ((threadIdx.x & (kWave - 1)) == 0) wmax[threadIdx.x / kWave] = v;
     __syncthreads();
-    for (int c = threadIdx.x; c < LC; c += kBlock) {
-        const int lx = c % Lx, ly = (c / Lx) % Ly, lz = c / (Lx * Ly);
-        const double val = ldexp((double)(long long)acc[c], E - 30) + ldexp((double)acc[LC + c], E - 62);
-        if (lx > 0 && ly > 0 && lz > 0)
-            own[B.cell_off + cidx(o0 + lx - 1, o1 + ly - 1, o2 + lz - 1, B.n[0], B.n[1])] = val;
-        else
-            halo[gt * B.halo_stride + halo_index(lx, ly, lz, bx, by, bz)] = val;
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < kBlock / kWave; ++w) v = max(v, wmax[w]);
+        if (v > __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(slot, v);
     }
 }
 
-// max |m v_d| per box and component (bit pattern, atomicMax) for k_deposit_mom.
+// max |m v_d| per box and component (bit patterns) for the momentum deposit.
 __global__ void __launch_bounds__(kBlock) k_max_mom(const BoxSeg* segs, int nseg, const BoxDev* boxes,
-                                                    const double* __restrict__ x, const double* __restrict__ m, const double* __restrict__ vx,
-                                                    const double* __restrict__ vy, const double* __restrict__ vz,
-                                                    unsigned long long* maxbits) {
+                                                    const double* __restrict__ x, const double* __restrict__ m,
+                                                    const double* __restrict__ vx, const double* __restrict__ vy,
+                                                    const double* __restrict__ vz, unsigned long long* maxbits) {
     const BoxSeg sg = segs[find_seg(segs, nseg, blockIdx.x)];
     const BoxDev B = boxes[__builtin_amdgcn_readfirstlane(sg.box)];
     const long long q = (long long)(blockIdx.x - sg.blk0) * kBlock + threadIdx.x;
-    if (q >= B.span) return;
     const long long p = B.part_off + q;
-    if (isnan(x[p])) return;
-    const double mp = B.has_mass ? m[p] : B.m_const;
-    atomicMax(maxbits + 3 * sg.box + 0, dbits(fabs(mp * vx[p])));
-    atomicMax(maxbits + 3 * sg.box + 1, dbits(fabs(mp * vy[p])));
-    atomicMax(maxbits + 3 * sg.box + 2, dbits(fabs(mp * vz[p])));
+    unsigned long long b0 = 0, b1 = 0, b2 = 0;
+    if (q < B.span && !isnan(x[p])) {
+        const double mp = B.has_mass ? m[p] : B.m_const;
+        b0 = dbits(fabs(mp * vx[p]));
+        b1 = dbits(fabs(mp * vy[p]));
+        b2 = dbits(fabs(mp * vz[p]));
+    }
+    block_max_to(b0, maxbits + 3 * sg.box + 0);
+    block_max_to(b1, maxbits + 3 * sg.box + 1);
+    block_max_to(b2, maxbits + 3 * sg.box + 2);
 }
 
 // Sum of a block's values in a fixed order (wave butterfly, then waves in order).
@@ -675,10 +648,15 @@ __device__ __forceinline__ void for_block_cells(const CellSeg& sg, const BoxDev&
 // values and face terms (x, y, z) are loaded before any is used, so a thread
 // has up to 4U loads in flight; the edge and corner terms (cells on two or
 // three top faces of a tile) follow them.  Coordinates advance by kBlock cells
-// with block-uniform carries instead of divisions.
-template <int U, class F>
-__device__ __forceinline__ void fold_walk(const CellSeg& sg, const BoxDev& B, const double* own,
-                                          const double* __restrict__ halo, F emit) {
+// with block-uniform carries instead of divisions.  C fields of the same tiles at
+// once (their addresses derived once): emit(q, v) gets the C values of a cell.
+template <int C>
+struct FoldFields {
+    const double* own[C];
+    const double* halo[C];
+};
+template <int U, int C, class F>
+__device__ __forceinline__ void fold_walk(const CellSeg& sg, const BoxDev& B, const FoldFields<C>& fields, F emit) {
     const int nx = B.n[0], ny = B.n[1], nz = B.n[2];
     const int T0 = B.tile[0], T1 = B.tile[1], T2 = B.tile[2];
     const int nt0 = B.ntile[0], nt1 = B.ntile[1], nt2 = B.ntile[2];
@@ -700,7 +678,7 @@ __device__ __forceinline__ void fold_walk(const CellSeg& sg, const BoxDev& B, co
     const long long hbase = B.tile_off;
     const long long hs = B.halo_stride;
     for (; c < c1; c += (long long)U * kBlock) {
-        double v[U], hx[U], hy[U], hz[U];
+        double v[U][C], hx[U][C], hy[U][C], hz[U][C];
         int cx[U], cy[U], cz[U];
         int fl[U];  // bit 0, 1, 2: on the tile's top x, y, z face; -1: past the block's cells
 #pragma unroll
@@ -709,9 +687,11 @@ __device__ __forceinline__ void fold_walk(const CellSeg& sg, const BoxDev& B, co
             cy[u] = j;
             cz[u] = k;
             fl[u] = -1;
-            hx[u] = hy[u] = hz[u] = 0.0;
+#pragma unroll
+            for (int f = 0; f < C; ++f) hx[u][f] = hy[u][f] = hz[u][f] = 0.0;
             if (c + (long long)u * kBlock < c1) {
-                v[u] = own[B.cell_off + c + (long long)u * kBlock];
+#pragma unroll
+                for (int f = 0; f < C; ++f) v[u][f] = fields.own[f][B.cell_off + c + (long long)u * kBlock];
                 const int tx = tile_div(i, B.tdiv[0]), ty = tile_div(j, B.tdiv[1]), tz = tile_div(k, B.tdiv[2]);
                 const int li = i - tx * T0, lj = j - ty * T1, lk = k - tz * T2;
                 const int bx = min(T0, nx - tx * T0), by = min(T1, ny - ty * T1), bz = min(T2, nz - tz * T2);
@@ -719,19 +699,25 @@ __device__ __forceinline__ void fold_walk(const CellSeg& sg, const BoxDev& B, co
                 fl[u] = (li == bx - 1 ? 1 : 0) | (lj == by - 1 ? 2 : 0) | (lk == bz - 1 ? 4 : 0);
                 if (li == bx - 1) {  // x face of tile tx + 1 (same rows and planes)
                     const int nlt = tx + 1 == nt0 ? lt - tx : lt + 1;
-                    hx[u] = halo[(hbase + nlt) * hs + (lk + 1) * (by + 1) + (lj + 1)];
+                    const long long o = (hbase + nlt) * hs + (lk + 1) * (by + 1) + (lj + 1);
+#pragma unroll
+                    for (int f = 0; f < C; ++f) hx[u][f] = fields.halo[f][o];
                 }
                 if (lj == by - 1) {  // y face of tile ty + 1
                     const int nty = ty + 1 == nt1 ? 0 : ty + 1;
                     const int nby = min(T1, ny - nty * T1);
                     const int nlt = lt + (nty - ty) * nt0;
-                    hy[u] = halo[(hbase + nlt) * hs + (nby + 1) * (bz + 1) + (lk + 1) * bx + li];
+                    const long long o = (hbase + nlt) * hs + (nby + 1) * (bz + 1) + (lk + 1) * bx + li;
+#pragma unroll
+                    for (int f = 0; f < C; ++f) hy[u][f] = fields.halo[f][o];
                 }
                 if (lk == bz - 1) {  // z face of tile tz + 1
                     const int ntz = tz + 1 == nt2 ? 0 : tz + 1;
                     const int nbz = min(T2, nz - ntz * T2);
                     const int nlt = lt + (ntz - tz) * nt0 * nt1;
-                    hz[u] = halo[(hbase + nlt) * hs + (by + 1) * (nbz + 1) + bx * (nbz + 1) + lj * bx + li];
+                    const long long o = (hbase + nlt) * hs + (by + 1) * (nbz + 1) + bx * (nbz + 1) + lj * bx + li;
+#pragma unroll
+                    for (int f = 0; f < C; ++f) hz[u][f] = fields.halo[f][o];
                 }
             }
             i += di;
@@ -748,17 +734,23 @@ __device__ __forceinline__ void fold_walk(const CellSeg& sg, const BoxDev& B, co
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int f = fl[u];
-            if (f < 0) continue;
-            double w = v[u];
-            if (f & 1) w += hx[u];
-            if (f & 2) w += hy[u];
-            if (f & 4) w += hz[u];
-            if (__builtin_popcount(f) >= 2) {
+            const int top = fl[u];
+            if (top < 0) continue;
+            double w[C];
+#pragma unroll
+            for (int f = 0; f < C; ++f) {
+                w[f] = v[u][f];
+                if (top & 1) w[f] += hx[u][f];
+                if (top & 2) w[f] += hy[u][f];
+                if (top & 4) w[f] += hz[u][f];
+            }
+            if (__builtin_popcount(top) >= 2) {
                 const int tx = tile_div(cx[u], B.tdiv[0]), ty = tile_div(cy[u], B.tdiv[1]),
                           tz = tile_div(cz[u], B.tdiv[2]);
-                w = fold_edges(B, halo, w, tx, ty, tz, cx[u] - tx * T0, cy[u] - ty * T1, cz[u] - tz * T2, f & 1,
-                               f & 2, f & 4);
+#pragma unroll
+                for (int f = 0; f < C; ++f)
+                    w[f] = fold_edges(B, fields.halo[f], w[f], tx, ty, tz, cx[u] - tx * T0, cy[u] - ty * T1,
+                                      cz[u] - tz * T2, top & 1, top & 2, top & 4);
             }
             emit(B.cell_off + (size_t)(c + (long long)u * kBlock), w);
         }
@@ -781,8 +773,9 @@ __global__ void __launch_bounds__(kBlock) k_fold(const CellSeg* segs, int nseg, 
     const CellSeg& sg = segs[find_seg(segs, nseg, blockIdx.x)];
     const BoxDev B = boxes[__builtin_amdgcn_readfirstlane(sg.box)];
     double acc = 0.0;  // this thread's cells, in a fixed order
-    fold_walk<kFoldU>(sg, B, own, halo, [&](size_t q, double v) {
-        const double rv = v * B.inv_vol;
+    const FoldFields<1> fields{{own}, {halo}};
+    fold_walk<kFoldU, 1>(sg, B, fields, [&](size_t q, const double (&v)[1]) {
+        const double rv = v[0] * B.inv_vol;
         if (WRITE_RHO) rho[q] = rv;
         const double fv = rv + (-B.mass_offset);
         f[q] = fv;
@@ -792,33 +785,24 @@ __global__ void __launch_bounds__(kBlock) k_fold(const CellSeg* segs, int nseg, 
     if (threadIdx.x == 0) partial[blockIdx.x] = bs;
 }
 
-// out = own + halos (fold_walk, no scaling): the folded raw sums of a deposit.
-__global__ void __launch_bounds__(kBlock) k_fold_raw(const CellSeg* segs, int nseg, const BoxDev* boxes,
-                                                     const double* __restrict__ own,
-                                                     const double* __restrict__ halo, double* __restrict__ out) {
-    const CellSeg& sg = segs[find_seg(segs, nseg, blockIdx.x)];
+// AssignDensityAndVels for one box (segs: its piece): the folded mass and momenta,
+// rho = mass * 1/vol, v_d = mom_d / mass (0 without mass), written as 4 fields of the
+// box's cells.  One pass over the four deposits (a fold per field into its own sums
+// and a pass to divide them before: 5 launches, 80 B more per cell).
+__global__ void __launch_bounds__(kBlock) k_fold_vels(const CellSeg* segs, const BoxDev* boxes, FoldFields<4> fields,
+                                                      double* __restrict__ out) {
+    CellSeg sg = segs[0];
+    sg.blk0 = 0;
     const BoxDev B = boxes[__builtin_amdgcn_readfirstlane(sg.box)];
-    fold_walk<kFoldU>(sg, B, own, halo, [&](size_t q, double v) { out[q] = v; });
+    const size_t nc = (size_t)B.n[0] * B.n[1] * B.n[2];
+    fold_walk<2, 4>(sg, B, fields, [&](size_t q, const double (&v)[4]) {
+        double* o = out + (q - B.cell_off);
+        const double ms = v[0];
+        o[0] = ms * B.inv_vol;
+#pragma unroll
+        for (int d = 1; d < 4; ++d) o[d * nc] = ms != 0.0 ? v[d] / ms : 0.0;
+    });
 }
-
-// AssignDensityAndVels for box `box`: rho = mass * 1/vol, v_d = mom_d / mass (0
-// without mass), written as 4 fields of the box's cells.
-__global__ void __launch_bounds__(kBlock) k_vels_finish(const BoxDev* boxes, int box,
-                                                        const double* __restrict__ mass,
-                                                        const double* __restrict__ mom,
-                                                        long long mom_stride, double* __restrict__ out) {
-    const BoxDev B = boxes[box];
-    const long long nc = (long long)B.n[0] * B.n[1] * B.n[2];
-    const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
-    if (q >= nc) return;
-    const double ms = mass[B.cell_off + q];
-    out[q] = ms * B.inv_vol;
-    for (int d = 0; d < 3; ++d) {
-        const double md = mom[d * mom_stride + B.cell_off + q];
-        out[(d + 1) * nc + q] = ms != 0.0 ? md / ms : 0.0;
-    }
-}
-
 
 // sum = (S*dV)/ProbSize, as vol_weight_sum computes it (sum_utils.cpp:85-93).
 __global__ void __launch_bounds__(kBlock) k_rhs_sum(const CellSeg* segs, const double* __restrict__ partial,
@@ -1105,7 +1089,9 @@ __device__ __forceinline__ void block_min_to(double v, unsigned long long* slot)
     if (threadIdx.x == 0) {
         double m = wmin[0];
         for (int w = 1; w < kBlock / kWave; ++w) m = wmin[w] < m ? wmin[w] : m;
-        if (m < 1e50) atomicMin(slot, dbits(m));
+        // (the slot only falls: see block_max_to)
+        const unsigned long long b = dbits(m);
+        if (m < 1e50 && b < __hip_atomic_load(slot, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(slot, b);
     }
 }
 

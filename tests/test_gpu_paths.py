@@ -176,3 +176,42 @@ def test_split_tile_deposit(nyx, orc, npart, precision):
         tol = 1e-13 if precision == "fp64" else 4 * 2.0 ** -24
         assert np.abs(c.get_rhs() - rhs).max() <= tol * ref.max()
         assert np.array_equal(c.assign_density(), rho)
+
+
+@pytest.mark.parametrize("clump", [0, 6001])
+def test_density_and_vels_second_box_of_a_batch(nyx, orc, clump):
+    # the momentum deposits (three components in one launch, a clump's tile in parts)
+    # and the one-pass fold, for a box with partial tiles behind another one: the
+    # density is AssignDensity's, the velocities the oracle's to the rounding of a sum
+    # of its contributions (cells with mass), and a second call gives the same bits
+    r = np.random.default_rng(71)
+    n, hi = (36, 20, 24), (1.8, 1.0, 1.2)
+    npart = 5000
+    pos = [r.random(npart) * h for h in hi]
+    pos = [np.concatenate([p, 0.41 + 0.02 * r.random(clump)]) for p in pos]
+    vel = [r.standard_normal(npart + clump) * (d + 1) for d in range(3)]
+    m = 0.5 + r.random(npart + clump)
+    geoms = [nyx.BoxGeom((16, 16, 16)), nyx.BoxGeom(n, (0, 0, 0), hi)]
+    with nyx.PMContext(geoms) as c:
+        small = [r.random(100) for _ in range(3)]
+        c.upload(0, small, small, m=0.1 + r.random(100))
+        c.upload(1, pos, vel, m=m)
+        rho = c.assign_density(1)
+        out = c.assign_density_and_vels(1)
+        assert np.array_equal(c.assign_density_and_vels(1), out)
+        assert np.array_equal(c.assign_density(1), rho)
+        # the solver's pools held the momentum sums: a solve after it is unaffected
+        c.solve_for_phi(use_guess=False)
+        phi = c.get_phi(1)
+    with nyx.PMContext(geoms) as c:
+        c.upload(0, small, small, m=0.1 + r.random(100))
+        c.upload(1, pos, vel, m=m)
+        c.assign_density(want=False)
+        c.solve_for_phi(use_guess=False)
+        assert np.array_equal(c.get_phi(1), phi)
+    assert np.array_equal(out[0], rho)
+    ref = orc.deposit_vels(n, (0, 0, 0), hi, pos, vel, m=m)
+    big = ref[0] > 1e-3 * ref[0].max()
+    for d in range(3):
+        assert np.abs(out[d + 1] - ref[d + 1])[big].max() <= 1e-11 * (d + 1)
+        assert np.array_equal(out[d + 1] == 0, out[0] == 0)
