@@ -1242,6 +1242,8 @@ constexpr int kBottomStage = 1024;  // bottom cells up to which G is staged in L
 // division is ~25 instructions, each 16 cycles with 16 waves on one CU.)
 __device__ __forceinline__ int small_div(int q, float inv) { return (int)(((float)q + 0.5f) * inv); }
 
+constexpr int kBottomPiece = 10;
+
 // One smoothing level as its threads hold it (NP pairs per thread).
 template <typename T, int NP>
 struct CoarseLevel {
@@ -1450,11 +1452,14 @@ __global__ void __launch_bounds__(kCoarseThreads) k_coarse_vcycle(const CellSeg*
     const int nbx = bs.n[0], nby = bs.n[1], nbz = bs.n[2];
     const int nb = nbx * nby * nbz;
     const int tid = threadIdx.x;
-    // LDS: the bottom's r (FP64), its G where staged, its e, then the levels' arrays
+    // LDS: the bottom's r (FP64), its G where staged (each row written out over one
+    // period either side, so that an x difference indexes it without a wrap), its e,
+    // then the levels' arrays
     double* rb = coarse_smem;
-    const bool stage = nb <= kBottomStage;
+    const bool stage = nb <= kBottomStage && nbx <= kWave;
     double* gl = rb + nb;
-    T* ebot = reinterpret_cast<T*>(gl + (stage ? nb : 0));
+    const int gw = 2 * nbx - 1;
+    T* ebot = reinterpret_cast<T*>(gl + (stage ? nby * nbz * gw : 0));
     T* lds = ebot + nb;
     const double* Gb = G + bs.coff;
     CoarseLevel<T, 2> L0;
@@ -1463,7 +1468,11 @@ __global__ void __launch_bounds__(kCoarseThreads) k_coarse_vcycle(const CellSeg*
         L0.setup(top, lds);
         L0.load_r(r + top.off);
     }
-    if (stage && tid < nb) gl[tid] = Gb[tid];
+    if (stage)
+        for (int q = tid; q < nby * nbz * gw; q += kCoarseThreads) {
+            const int row = small_div(q, 1.0f / (float)gw), k = q - row * gw;
+            gl[q] = Gb[row * nbx + (k < nbx - 1 ? k + 1 : k - (nbx - 1))];
+        }
     if (ns > 1) L1.setup(segs[l0 + 1], lds + 2 * L0.np);
     if (ns > 2) L2.setup(segs[l0 + 2], lds + 2 * L0.np + 2 * L1.np);
     // down: zero guess (keep_top: on the box's own level, the e of the previous
@@ -1493,8 +1502,79 @@ __global__ void __launch_bounds__(kCoarseThreads) k_coarse_vcycle(const CellSeg*
                                    : L2.restricted(I, J, K));
     }
     __syncthreads();
-    {
-        const double* g = stage ? gl : Gb;
+    auto put = [&](int q, double acc) {
+        if (ns == 0)
+            e[bs.off + q] = T(acc);
+        else
+            ebot[q] = T(acc);
+    };
+    if (stage) {
+        // two x-adjacent outputs per thread: at input qx the second one needs the G
+        // the first needed at qx - 1, so one LDS read serves two products; r is the
+        // same for all threads and comes from the lanes of a wave that read its row
+        // once.  A row goes in pieces of at most kBottomPiece inputs whose operands
+        // are read while the piece before is added up: with 7-12 waves on the CU the
+        // sums are otherwise chains of LDS latencies (115 cycles an input).  Whole
+        // kernel, us: 7 x 6 x 9 bottom 34 -> 25, 9^3 54 -> 37 (129 and 59 with one
+        // output per thread, operands through the caches and a wrap per product).
+        const int lane = tid & (kWave - 1);
+        const int px = (nbx + 1) >> 1, units = px * nby * nbz;
+        // whole waves take part (readlane reads lanes without an output too)
+        if ((tid & ~(kWave - 1)) < units) {
+            const int u = min(tid, units - 1);
+            const int t = small_div(u, 1.0f / (float)px), c0 = 2 * (u - t * px);
+            const int cz = small_div(t, 1.0f / (float)nby), cy = t - cz * nby;
+            const int npc = (nbx + kBottomPiece - 1) / kBottomPiece;
+            double a0 = 0.0, a1 = 0.0;
+            // the piece being read: row (qz, qy), inputs from xs.  g[i]: G of output
+            // c0 + 1 at input xs + i, of c0 at xs + i - 1.  Inputs past the row have
+            // r = 0 (lanes past nbx): they add a zero times some finite word (G of
+            // another row or the r before it) to a sum that is never -0.
+            int qz = 0, qy = 0, xs = 0;
+            auto read = [&](double (&g)[kBottomPiece + 1], double& rv) {
+                const int dz = cz - qz < 0 ? cz - qz + nbz : cz - qz;
+                const int dy = cy - qy < 0 ? cy - qy + nby : cy - qy;
+                const double* gr = gl + (dz * nby + dy) * gw + c0 + nbx - xs;
+                const double v = rb[(qz * nby + qy) * nbx + min(xs + lane, nbx - 1)];
+                rv = xs + lane < nbx ? v : 0.0;
+#pragma unroll
+                for (int i = 0; i <= kBottomPiece; ++i) g[i] = gr[-i];
+                xs += kBottomPiece;
+                if (xs >= nbx) {
+                    xs = 0;
+                    if (++qy == nby) {
+                        qy = 0;
+                        ++qz;
+                    }
+                }
+            };
+            auto add = [&](const double (&g)[kBottomPiece + 1], double rv) {
+                const int rlo = __double2loint(rv), rhi = __double2hiint(rv);
+#pragma unroll
+                for (int i = 0; i < kBottomPiece; ++i) {
+                    const double rr = __hiloint2double(__builtin_amdgcn_readlane(rhi, i),
+                                                       __builtin_amdgcn_readlane(rlo, i));
+                    a0 += g[i + 1] * rr;
+                    a1 += g[i] * rr;
+                }
+            };
+            const int np = npc * nby * nbz;
+            double ga[kBottomPiece + 1], gb[kBottomPiece + 1], ra, rc;
+            read(ga, ra);
+            for (int k = 0; k + 1 < np; k += 2) {
+                read(gb, rc);
+                add(ga, ra);
+                if (k + 2 < np) read(ga, ra);
+                add(gb, rc);
+            }
+            if (np & 1) add(ga, ra);
+            if (tid < units) {
+                const int q = t * nbx + c0;
+                put(q, a0);
+                if (c0 + 1 < nbx) put(q + 1, a1);
+            }
+        }
+    } else {
         for (int q = tid; q < nb; q += kCoarseThreads) {
             const int cx = q % nbx, t = q / nbx;
             const int cy = t % nby, cz = t / nby;
@@ -1503,7 +1583,7 @@ __global__ void __launch_bounds__(kCoarseThreads) k_coarse_vcycle(const CellSeg*
                 int dz = cz - qz; dz = dz < 0 ? dz + nbz : dz;
                 for (int qy = 0; qy < nby; ++qy) {
                     int dy = cy - qy; dy = dy < 0 ? dy + nby : dy;
-                    const double* gr = g + (dz * nby + dy) * nbx;
+                    const double* gr = Gb + (dz * nby + dy) * nbx;
                     const double* rr = rb + (qz * nby + qy) * nbx;
                     for (int qx = 0; qx < nbx; ++qx) {
                         int dxx = cx - qx; dxx = dxx < 0 ? dxx + nbx : dxx;
@@ -1511,10 +1591,7 @@ __global__ void __launch_bounds__(kCoarseThreads) k_coarse_vcycle(const CellSeg*
                     }
                 }
             }
-            if (ns == 0)
-                e[bs.off + q] = T(acc);
-            else
-                ebot[q] = T(acc);
+            put(q, acc);
         }
     }
     if (ns == 0) return;

@@ -857,8 +857,10 @@ int build_tables(nyxpm_ctx* c) {
             }
             // the bottom's r and, where staged, G in FP64 (a bottom without levels
             // above it keeps no e)
-            const long long nb = B.lev[B.nlev - 1].nc;
-            const long long fp64 = nb * (nb <= kBottomStage ? 2 : 1);
+            const Level& LB = B.lev[B.nlev - 1];
+            const bool stage = LB.nc <= kBottomStage && LB.n[0] <= kWave;
+            // (one word more: an odd row's last pair reads G of an output past it)
+            const long long fp64 = LB.nc + (stage ? (long long)LB.n[1] * LB.n[2] * (2 * LB.n[0] - 1) + 1 : 0);
             if (B.dc == B.nlev - 1) cells = 0;
             for (int pr = 0; pr < 2; ++pr)
                 c->cc_lds[pr] = std::max(c->cc_lds[pr], (size_t)(fp64 * 8 + cells * (pr == 0 ? 8 : 4)));
