@@ -40,6 +40,8 @@ def test_residual_chunks_bitwise(nyx, orc, n):
     (9, 5, 7),       # a bottom alone
     (14, 12, 13),    # a bottom too large to be staged (2184 cells)
     (36, 40, 48),    # finer levels above a 9 x 10 x 12 workgroup level
+    (36, 36, 36),                 # a 9^3 bottom: odd rows of one piece
+    (44, 20, 12),                 # an 11 x 5 x 3 bottom: rows of two pieces
 ])
 def test_coarse_workgroup_equals_per_level(nyx, orc, n, precision):
     # the one-workgroup coarse cycle against one launch per level and step, bit for
