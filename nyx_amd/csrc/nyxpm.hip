@@ -1782,6 +1782,17 @@ int solve_results(nyxpm_ctx* c, int* iters, double* final_res, bool allow_active
     return NYXPM_OK;
 }
 
+// LDS of the kernels that stage g per tile (stage_g): phi of the tile with a halo of 2,
+// and the three components of g on its (tile+1)^3 cells, written over the staged phi
+// where a thread's share of g fits in registers, else beside it.
+template <typename G>
+size_t stage_lds(const nyxpm_ctx* c) {
+    const size_t lds_phi = sizeof(double) * (c->tile[0] + 3) * (c->tile[1] + 3) * (c->tile[2] + 3);
+    const long long ng = (long long)(c->tile[0] + 1) * (c->tile[1] + 1) * (c->tile[2] + 1);
+    const size_t lds_g = sizeof(G) * 3 * ng;
+    return ng <= (long long)kBlock * kKickG ? std::max(lds_phi, lds_g) : lds_phi + lds_g;
+}
+
 template <int MODE>
 int phase_kick(nyxpm_ctx* c, double dt, double a_prev, double a_cur, double a_prev2 = 1.0, double a_cur2 = 1.0);
 
@@ -1798,13 +1809,7 @@ int phase_kick_g(nyxpm_ctx* c, double dt, double a_prev, double a_cur, double a_
     if ((rc = ensure_idle_buffer(c))) return rc;
     PartPtrs& A = c->P[c->cur];
     constexpr bool MOVE = MODE != kKick;
-    // staged phi tile with a halo of 2, and the three components of g on the
-    // (tile+1)^3 cells its particles interpolate from: written over the staged
-    // phi where a thread's share of g fits in registers, else beside it
-    const size_t lds_phi = sizeof(double) * (c->tile[0] + 3) * (c->tile[1] + 3) * (c->tile[2] + 3);
-    const long long ng = (long long)(c->tile[0] + 1) * (c->tile[1] + 1) * (c->tile[2] + 1);
-    const size_t lds_g = sizeof(G) * 3 * ng;
-    const size_t lds = ng <= (long long)kBlock * kKickG ? std::max(lds_phi, lds_g) : lds_phi + lds_g;
+    const size_t lds = stage_lds<G>(c);
     if (c->items_valid && !c->untiled_kick && lds <= 64 * 1024) {
         Timed t(c, MODE == kKickPair ? "kick_pair" : MOVE ? "kick_drift" : "kick");
         // incremental re-sort: the kick-drift lists the particles that change tile
@@ -2012,11 +2017,40 @@ int bind_scratch(nyxpm_ctx* c) {
     return NYXPM_OK;
 }
 
-// Accelerations of box `box`'s particles (k_gather) into `out`, device memory of
-// 3*np doubles; stream-ordered, no synchronisation.
+template <typename G>
+void launch_gather_tiled(nyxpm_ctx* c, int box, double* out, double* rec) {
+    PartPtrs& A = c->P[c->cur];
+    const Box& B = c->boxes[box];
+    auto kern = rec ? k_gather_tiled<G, true> : k_gather_tiled<G, false>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)c->items_cap), dim3(kBlock), stage_lds<G>(c), c->stream, c->tseg,
+                       c->tseg_n, c->dboxes, box, c->items, c->nitems, c->phi, A.x, A.y, A.z, A.id, rec ? rec : out,
+                       c->err_flag);
+    if (rec)
+        hipLaunchKernelGGL(k_unpack_accel, dim3(nblocks(B.np)), dim3(kBlock), 0, c->stream, B.np, rec, out);
+}
+
+// Accelerations of box `box`'s particles into `out`, device memory of 3*np doubles;
+// stream-ordered, no synchronisation, no allocation.  From the staged tiles above
+// kUnsortDirect particles (at 2^18 the thread-per-particle kernel takes 45 us, the
+// staged one 49) where they are binned and the box holds most of the context's slots
+// (the launch walks every box's items), through records in the idle buffer where that
+// exists and holds no list of moves (9 of the 64 KB of LDS are the records).
 int launch_gather(nyxpm_ctx* c, int box, double* out) {
     const Box& B = c->boxes[box];
     PartPtrs& A = c->P[c->cur];
+    const bool mixed = c->precision == NYXPM_MIXED;
+    const size_t lds = mixed ? stage_lds<float>(c) : stage_lds<double>(c);
+    if (c->items_valid && B.np > kUnsortDirect && 2 * B.span >= c->part_cap && lds <= 48 * 1024) {
+        PartPtrs& I = c->P[1 - c->cur];
+        const bool room = I.x && I.bytes >= (size_t)B.np * kAccelRec * sizeof(double);
+        double* rec = room && !c->moves_pending ? I.x : nullptr;
+        if (mixed)
+            launch_gather_tiled<float>(c, box, out, rec);
+        else
+            launch_gather_tiled<double>(c, box, out, rec);
+        LAUNCHCK(c);
+        return NYXPM_OK;
+    }
     hipLaunchKernelGGL(c->precision == NYXPM_MIXED ? k_gather<float> : k_gather<double>, dim3(nblocks(B.span)),
                        dim3(kBlock), 0, c->stream, c->dboxes, box, c->phi, A.x, A.y, A.z, A.id, out, c->err_flag);
     LAUNCHCK(c);

@@ -1134,83 +1134,17 @@ __device__ __forceinline__ long long defer_entry(long long p, int box) {
     return p | ((long long)box << 40);
 }
 
-// Tile-staged gather + kick(-drift).  phi over the tile plus a halo of 2 is
-// staged in LDS once per item (rows of the staged box spread over the lanes of a
-// wave, so the index arithmetic is per row), and g (the average of the face
-// gradients, the three components of a cell side by side) is formed there on the
-// (tile+1)^3 cells the CIC stencils of the tile's particles touch.  Same
-// arithmetic as k_kick, bit for bit.
-//
-// kKickPair runs the closing kick of step n (a_prev, a_cur) and the opening
-// kick-drift of step n+1 (a_prev2, a_cur2) in one pass: both use g from the same
-// phi at the same position.  A particle moved by the periodic shift in between
-// has its kick stored and its kick-drift deferred (to be interpolated again at
-// the shifted position, as the separate kernels would); so is any particle whose
-// cell falls outside the item's tile (binning older than a shift).  Deferral
-// keeps those rare paths out of this kernel's registers.
-//
-// Binning for the next deposit (kick-drifts): with inc, the particles whose new
-// tile differs from the item's are listed for k_migrate; otherwise every
-// particle gets its key, and the tile counts are summed per block for the
-// particles that stay in the item's tile (one atomic), counted individually
-// for the others.
-//
-// EST (closing kicks only): also NyxParticleContainer::estTimestep of the kicked
-// particles (cfl, a = a_cur) into dtmin, from the staged g; a compile-time
-// variant so that the kernels without it keep their register budget.
-template <int MODE, bool EST, typename G>
-__global__ void __launch_bounds__(kBlock) k_kick_tiled(const BoxSeg* tsegs, int ntseg, const BoxDev* boxes,
-                                                       const TileItem* __restrict__ items, const int* nitems,
-                                                       const double* __restrict__ phi, double* __restrict__ x,
-                                                       double* __restrict__ y, double* __restrict__ z,
-                                                       double* __restrict__ vx, double* __restrict__ vy,
-                                                       double* __restrict__ vz, double dt, double a_prev,
-                                                       double a_cur, double a_prev2, double a_cur2,
-                                                       int* __restrict__ key, int* counts,
-                                                       long long* __restrict__ defer, int* ndefer, double cfl,
-                                                       unsigned long long* dtmin, int inc,
-                                                       long long* __restrict__ moves, int* nmove, int* err) {
-    extern __shared__ __align__(16) unsigned char kick_smem[];
-    double* sphi = reinterpret_cast<double*>(kick_smem);
-    __shared__ int s_same[kBlock / kWave];
-    // items are in (roughly) tile order; giving each XCD a contiguous range of them
-    // lets neighbouring tiles share the phi halo lines in that XCD's L2
-    const int n_items = *nitems;
-    if ((int)blockIdx.x >= n_items) return;
-    const TileItem it = items[xcd_block(blockIdx.x, n_items)];
-    const int sgi = find_seg(tsegs, ntseg, it.tile);
-    const int box = __builtin_amdgcn_readfirstlane(tsegs[sgi].box);
-    // the box's fields as block-uniform values in registers: read through a
-    // reference they would be re-read from memory (and waited for, behind the
-    // particle stores) after every store or atomic of the particle loop
-    const BoxDev B = boxes[box];
-    const int lt = it.tile - tsegs[sgi].blk0;
+// g (the average of the face gradients) on the (tile+1)^3 cells that the particles of
+// the tile at (o0, o1, o2), bx x by x bz cells, interpolate from, in LDS: phi of the tile
+// and a halo of 2 staged at sphi, then the three components of a cell side by side.
+// Returns g's place (over the staged phi or behind it); the caller's barrier follows.
+template <typename G>
+__device__ __forceinline__ const G* stage_g(const BoxDev& B, const double* __restrict__ P, double* sphi, int o0, int o1,
+                                            int o2, int bx, int by, int bz) {
     const int nx = B.n[0], ny = B.n[1], nz = B.n[2];
-    const int tx = lt % B.ntile[0], ty = (lt / B.ntile[0]) % B.ntile[1], tz = lt / (B.ntile[0] * B.ntile[1]);
-    const int o0 = tx * B.tile[0], o1 = ty * B.tile[1], o2 = tz * B.tile[2];
-    const int bx = min(B.tile[0], nx - o0), by = min(B.tile[1], ny - o1), bz = min(B.tile[2], nz - o2);
     const int SX = bx + 3, SY = by + 3, SZ = bz + 3;
-    const double* P = phi + B.cell_off;
+    const int GX = bx + 1, GY = by + 1, GZ = bz + 1;
     const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-    // the item's particles through block-uniform base pointers and 32-bit
-    // indices (scalar base + vector offset addressing)
-    double* __restrict__ X = x + it.p0;
-    double* __restrict__ Y = y + it.p0;
-    double* __restrict__ Z = z + it.p0;
-    double* __restrict__ VX = vx + it.p0;
-    double* __restrict__ VY = vy + it.p0;
-    double* __restrict__ VZ = vz + it.p0;
-    int* __restrict__ KEY = key + it.p0;
-    // one particle per thread at a time, the first loaded before the staging of
-    // phi so that its latency overlaps the staging.  (Two per thread in flight
-    // need 12-27 more VGPRs, one wave per SIMD fewer: 2% slower in mixed
-    // precision, 14% in FP64.)
-    double ax = 0.0, ay = 0.0, az = 0.0, aux = 0.0, auy = 0.0, auz = 0.0;
-    auto load1 = [&](int q) {
-        ax = X[q]; ay = Y[q]; az = Z[q];
-        aux = VX[q]; auy = VY[q]; auz = VZ[q];
-    };
-    if ((int)threadIdx.x < it.np) load1(threadIdx.x);
     {
         // rows of SX cells: a wave takes rpw rows per pass (SX <= 35 < 64).  The
         // passes go in batches of kStageBatch: every load of a batch is issued
@@ -1257,7 +1191,6 @@ __global__ void __launch_bounds__(kBlock) k_kick_tiled(const BoxSeg* tsegs, int 
     // there and, after a barrier, written over the staged phi, which it no
     // longer needs: the block holds the larger of the two arrays instead of both
     // (more blocks per CU); otherwise g goes beside the staged phi.
-    const int GX = bx + 1, GY = by + 1, GZ = bz + 1;
     const int ng = GX * GY * GZ;
     const bool alias = ng <= kBlock * kKickG;
     G* sg = reinterpret_cast<G*>(alias ? sphi : sphi + SX * SY * SZ);
@@ -1321,6 +1254,88 @@ __global__ void __launch_bounds__(kBlock) k_kick_tiled(const BoxSeg* tsegs, int 
             }
         }
     }
+    return sg;
+}
+
+// Tile-staged gather + kick(-drift).  phi over the tile plus a halo of 2 is
+// staged in LDS once per item (rows of the staged box spread over the lanes of a
+// wave, so the index arithmetic is per row), and g (the average of the face
+// gradients, the three components of a cell side by side) is formed there on the
+// (tile+1)^3 cells the CIC stencils of the tile's particles touch.  Same
+// arithmetic as k_kick, bit for bit.
+//
+// kKickPair runs the closing kick of step n (a_prev, a_cur) and the opening
+// kick-drift of step n+1 (a_prev2, a_cur2) in one pass: both use g from the same
+// phi at the same position.  A particle moved by the periodic shift in between
+// has its kick stored and its kick-drift deferred (to be interpolated again at
+// the shifted position, as the separate kernels would); so is any particle whose
+// cell falls outside the item's tile (binning older than a shift).  Deferral
+// keeps those rare paths out of this kernel's registers.
+//
+// Binning for the next deposit (kick-drifts): with inc, the particles whose new
+// tile differs from the item's are listed for k_migrate; otherwise every
+// particle gets its key, and the tile counts are summed per block for the
+// particles that stay in the item's tile (one atomic), counted individually
+// for the others.
+//
+// EST (closing kicks only): also NyxParticleContainer::estTimestep of the kicked
+// particles (cfl, a = a_cur) into dtmin, from the staged g; a compile-time
+// variant so that the kernels without it keep their register budget.
+template <int MODE, bool EST, typename G>
+__global__ void __launch_bounds__(kBlock) k_kick_tiled(const BoxSeg* tsegs, int ntseg, const BoxDev* boxes,
+                                                       const TileItem* __restrict__ items, const int* nitems,
+                                                       const double* __restrict__ phi, double* __restrict__ x,
+                                                       double* __restrict__ y, double* __restrict__ z,
+                                                       double* __restrict__ vx, double* __restrict__ vy,
+                                                       double* __restrict__ vz, double dt, double a_prev,
+                                                       double a_cur, double a_prev2, double a_cur2,
+                                                       int* __restrict__ key, int* counts,
+                                                       long long* __restrict__ defer, int* ndefer, double cfl,
+                                                       unsigned long long* dtmin, int inc,
+                                                       long long* __restrict__ moves, int* nmove, int* err) {
+    extern __shared__ __align__(16) unsigned char kick_smem[];
+    double* sphi = reinterpret_cast<double*>(kick_smem);
+    __shared__ int s_same[kBlock / kWave];
+    // items are in (roughly) tile order; giving each XCD a contiguous range of them
+    // lets neighbouring tiles share the phi halo lines in that XCD's L2
+    const int n_items = *nitems;
+    if ((int)blockIdx.x >= n_items) return;
+    const TileItem it = items[xcd_block(blockIdx.x, n_items)];
+    const int sgi = find_seg(tsegs, ntseg, it.tile);
+    const int box = __builtin_amdgcn_readfirstlane(tsegs[sgi].box);
+    // the box's fields as block-uniform values in registers: read through a
+    // reference they would be re-read from memory (and waited for, behind the
+    // particle stores) after every store or atomic of the particle loop
+    const BoxDev B = boxes[box];
+    const int lt = it.tile - tsegs[sgi].blk0;
+    const int nx = B.n[0], ny = B.n[1], nz = B.n[2];
+    const int tx = lt % B.ntile[0], ty = (lt / B.ntile[0]) % B.ntile[1], tz = lt / (B.ntile[0] * B.ntile[1]);
+    const int o0 = tx * B.tile[0], o1 = ty * B.tile[1], o2 = tz * B.tile[2];
+    const int bx = min(B.tile[0], nx - o0), by = min(B.tile[1], ny - o1), bz = min(B.tile[2], nz - o2);
+    const double* P = phi + B.cell_off;
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    // the item's particles through block-uniform base pointers and 32-bit
+    // indices (scalar base + vector offset addressing)
+    double* __restrict__ X = x + it.p0;
+    double* __restrict__ Y = y + it.p0;
+    double* __restrict__ Z = z + it.p0;
+    double* __restrict__ VX = vx + it.p0;
+    double* __restrict__ VY = vy + it.p0;
+    double* __restrict__ VZ = vz + it.p0;
+    int* __restrict__ KEY = key + it.p0;
+    // one particle per thread at a time, the first loaded before the staging of
+    // phi so that its latency overlaps the staging.  (Two per thread in flight
+    // need 12-27 more VGPRs, one wave per SIMD fewer: 2% slower in mixed
+    // precision, 14% in FP64.)
+    double ax = 0.0, ay = 0.0, az = 0.0, aux = 0.0, auy = 0.0, auz = 0.0;
+    auto load1 = [&](int q) {
+        ax = X[q]; ay = Y[q]; az = Z[q];
+        aux = VX[q]; auy = VY[q]; auz = VZ[q];
+    };
+    if ((int)threadIdx.x < it.np) load1(threadIdx.x);
+    const int GX = bx + 1, GY = by + 1;
+    const double dxi0 = B.dxi[0], dxi1 = B.dxi[1], dxi2 = B.dxi[2];
+    const G* sg = stage_g<G>(B, P, sphi, o0, o1, o2, bx, by, bz);
     __syncthreads();
     const double half_dt = 0.5 * dt;
     const double a_cur_inv = 1.0 / a_cur;
@@ -1813,6 +1828,136 @@ __global__ void __launch_bounds__(kBlock) k_gather(const BoxDev* boxes, int box,
     out[o] = val[0];
     out[B.np + o] = val[1];
     out[2 * B.np + o] = val[2];
+}
+
+// The same from the tiles' staged g (k_kick_tiled's items and arithmetic: the values of
+// k_gather bit for bit), for one box of a context: a block stages g of an item's tile
+// once where k_gather reads 32 phi values per particle through the caches.  A particle
+// whose cell is not one of the tile's (the binning is older than its position) is
+// interpolated from global phi.  REC: the values go out as records of kAccelRec doubles
+// at the upload index (rec, spread over the components by k_unpack_accel), for outputs
+// the caches do not hold: a scattered 8-byte write costs a line.  A wave passes its
+// values through LDS so that adjacent lanes write a record.
+// Measured, whole call: 9 10^6 clustered particles in random upload order 1144 -> 552 us
+// mixed, 1047 -> 555 us FP64; 2^24 in lattice order 674 -> 529 us (records of 64 bytes
+// 604, 622 and 733 us; 32-byte records written by one lane each 605 us, the first).
+constexpr int kAccelRec = 4;
+template <typename G, bool REC>
+__global__ void __launch_bounds__(kBlock) k_gather_tiled(const BoxSeg* tsegs, int ntseg, const BoxDev* boxes, int box,
+                                                         const TileItem* __restrict__ items, const int* nitems,
+                                                         const double* __restrict__ phi,
+                                                         const double* __restrict__ x, const double* __restrict__ y,
+                                                         const double* __restrict__ z, const int* __restrict__ id,
+                                                         double* __restrict__ out, int* err) {
+    extern __shared__ __align__(16) unsigned char gather_smem[];
+    const int n_items = *nitems;
+    if ((int)blockIdx.x >= n_items) return;
+    const TileItem it = items[xcd_block(blockIdx.x, n_items)];
+    const int sgi = find_seg(tsegs, ntseg, it.tile);
+    if (tsegs[sgi].box != box) return;
+    const BoxDev B = boxes[box];
+    const int lt = it.tile - tsegs[sgi].blk0;
+    const int tx = lt % B.ntile[0], ty = (lt / B.ntile[0]) % B.ntile[1], tz = lt / (B.ntile[0] * B.ntile[1]);
+    const int o0 = tx * B.tile[0], o1 = ty * B.tile[1], o2 = tz * B.tile[2];
+    const int bx = min(B.tile[0], B.n[0] - o0), by = min(B.tile[1], B.n[1] - o1), bz = min(B.tile[2], B.n[2] - o2);
+    const double* __restrict__ X = x + it.p0;
+    const double* __restrict__ Y = y + it.p0;
+    const double* __restrict__ Z = z + it.p0;
+    const int* __restrict__ ID = id + it.p0;
+    // one particle per thread at a time, the next one loaded before this one's value
+    double ax = 0.0, ay = 0.0, az = 0.0;
+    int aid = 0;
+    auto load = [&](int q) {
+        ax = X[q];
+        ay = Y[q];
+        az = Z[q];
+        aid = ID[q];
+    };
+    if ((int)threadIdx.x < it.np) load(threadIdx.x);
+    const int GX = bx + 1, GY = by + 1;
+    const G* sg = stage_g<G>(B, phi + B.cell_off, reinterpret_cast<double*>(gather_smem), o0, o1, o2, bx, by, bz);
+    __syncthreads();
+    constexpr int RL = kAccelRec / 2;  // lanes per record
+    __shared__ __align__(16) double sval[REC ? kBlock * 4 : 2];
+    __shared__ int sid[REC ? kBlock : 1];
+    const int lane = threadIdx.x & (kWave - 1), w0 = threadIdx.x - lane;
+    // whole waves together (the lanes past the item's particles hold none)
+    for (int q = threadIdx.x; q - lane < it.np; q += kBlock) {
+        const double px = q < it.np ? ax : empty_slot(), py = ay, pz = az;
+        const long long o = aid;
+        if (q + kBlock < it.np) load(q + kBlock);
+        const bool valid = !isnan(px);
+        if (REC) sid[threadIdx.x] = valid ? (int)o : -1;
+        if (valid) {
+        double xint, yint, zint;
+        const int li = cic_index(px, B.plo[0], B.dxi[0], &xint) - o0;
+        const int lj = cic_index(py, B.plo[1], B.dxi[1], &yint) - o1;
+        const int lk = cic_index(pz, B.plo[2], B.dxi[2], &zint) - o2;
+        double val[3];
+        if ((unsigned)li < (unsigned)bx && (unsigned)lj < (unsigned)by && (unsigned)lk < (unsigned)bz) {
+            const G fx = G(xint), fy = G(yint), fz = G(zint);
+            const G mx = G(1) - fx, my = G(1) - fy, mz = G(1) - fz;
+            G g0 = G(0), g1 = G(0), g2 = G(0);
+#pragma unroll
+            for (int kk = 0; kk <= 1; ++kk) {
+                const G wz = kk ? mz : fz;
+#pragma unroll
+                for (int jj = 0; jj <= 1; ++jj) {
+                    const G wy = jj ? my : fy;
+                    const G* g = sg + 3 * (((lk + 1 - kk) * GY + (lj + 1 - jj)) * GX + li);
+                    const G w0 = fx * wy * wz;  // cell i
+                    g0 += w0 * g[3];
+                    g1 += w0 * g[4];
+                    g2 += w0 * g[5];
+                    const G w1 = mx * wy * wz;  // cell i-1
+                    g0 += w1 * g[0];
+                    g1 += w1 * g[1];
+                    g2 += w1 * g[2];
+                }
+            }
+            val[0] = double(g0);
+            val[1] = double(g1);
+            val[2] = double(g2);
+        } else {
+            gather_grad<G>(B, phi + B.cell_off, px, py, pz, val, err);
+        }
+        if (REC) {
+            double2* sv = reinterpret_cast<double2*>(sval + 4 * threadIdx.x);
+            sv[0] = make_double2(val[0], val[1]);
+            sv[1] = make_double2(val[2], 0.0);
+        } else {
+            out[o] = val[0];
+            out[B.np + o] = val[1];
+            out[2 * B.np + o] = val[2];
+        }
+        }
+        if (REC) {
+            // LDS operations of one wave complete in order: no barrier
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+#pragma unroll
+            for (int k = 0; k < RL; ++k) {
+                const int rr = w0 + k * (kWave / RL) + lane / RL, part = lane % RL;
+                const int d = sid[rr];
+                if (d >= 0)
+                    reinterpret_cast<double2*>(out)[(size_t)d * RL + part] =
+                        reinterpret_cast<const double2*>(sval + 4 * rr)[part & 1];
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        }
+    }
+}
+
+__global__ void __launch_bounds__(kBlock) k_unpack_accel(long long np, const double* __restrict__ rec,
+                                                         double* __restrict__ out) {
+    const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
+    if (q >= np) return;
+    const double2* r = reinterpret_cast<const double2*>(rec) + (kAccelRec / 2) * q;
+    const double2 a = r[0], b = r[1];
+    out[q] = a.x;
+    out[np + q] = a.y;
+    out[2 * np + q] = b.x;
 }
 
 }  // namespace nyxpm

@@ -217,3 +217,39 @@ def test_density_and_vels_second_box_of_a_batch(nyx, orc, clump):
     for d in range(3):
         assert np.abs(out[d + 1] - ref[d + 1])[big].max() <= 1e-11 * (d + 1)
         assert np.array_equal(out[d + 1] == 0, out[0] == 0)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("npart", [3000, 2 ** 18 + 5])
+def test_tiled_gather_equals_thread_per_particle(nyx, npart, precision):
+    # the staged gather (written directly, and as records above 2^18 particles) against
+    # the thread-per-particle kernel, which a context that has not binned its particles
+    # takes: after the deposit, after a kick-drift whose moves still wait (particles
+    # outside their tile and outside the box) and after its periodic shift
+    r = np.random.default_rng(81)
+    n, hi = (40, 24, 36), (2.0, 1.2, 1.8)
+    pos = [r.random(npart) * h for h in hi]
+    vel = [r.standard_normal(npart) for _ in range(3)]
+    phi = r.standard_normal((n[2], n[1], n[0]))
+    with ctx1(nyx, n, hi=hi, precision=precision) as c:
+        c.upload(0, pos, vel, m_const=1.0)
+        c.set_phi(phi)
+
+        def unbinned():
+            p, v = c.download()
+            with ctx1(nyx, n, hi=hi, precision=precision) as c2:
+                c2.upload(0, p, v, m_const=1.0)
+                c2.set_phi(phi)
+                return c2.gather_accel()
+
+        assert np.array_equal(c.gather_accel(), unbinned())
+        c.assign_density(want=False)
+        assert np.array_equal(c.gather_accel(), unbinned())
+        c.move_kick_drift(0.05)
+        assert np.array_equal(c.gather_accel(), unbinned())
+        c.assign_density(want=False)
+        assert np.array_equal(c.gather_accel(), unbinned())
+        c.redistribute()
+        assert np.array_equal(c.gather_accel(), unbinned())
+        if npart <= 2 ** 20:
+            assert np.array_equal(c.gather_accel_noalloc(), unbinned())
