@@ -1756,11 +1756,13 @@ __global__ void __launch_bounds__(kBlock) k_update0(const CellSeg* segs, int nse
 //   iter: iters++, active = |r| > target && iters < limit
 // state: [0] resnorm0 [1] rhsnorm [2] final [3] target
 // One wave per box: its lanes take the norm slots (one lane reading them in turn
-// was a chain of 64 loads, 5 us a launch).
+// was a chain of 64 loads, 5 us a launch).  The box's flags and state also go to the
+// host's mirror (pinned memory), so that reading them takes a wait for the stream and
+// no copies (a copy is a launch of its own, 3-4 us and its gap; a step read five).
 __global__ void __launch_bounds__(kWave) k_check(int init, int fixed_iters, int max_iter, double rel_tol,
                                                  double abs_tol, int* active, int* iters, int* failed,
                                                  unsigned long long* nr, unsigned long long* nf, double* state,
-                                                 int inc) {
+                                                 int inc, int nbox, int* h_flags, double* h_state) {
     static_assert(kNormSlots == kWave, "one lane per norm slot");
     const int b = blockIdx.x;
     const int slot = b * kNormSlots + threadIdx.x;
@@ -1799,6 +1801,11 @@ __global__ void __launch_bounds__(kWave) k_check(int init, int fixed_iters, int 
             failed[b] = (more && it >= max_iter) ? 1 : 0;
         }
     }
+    auto put = [](auto* p, auto v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
+    put(&h_flags[b], active[b]);
+    put(&h_flags[nbox + b], iters[b]);
+    put(&h_flags[2 * nbox + b], failed[b]);
+    for (int q = 0; q < 4; ++q) put(&h_state[4 * b + q], state[4 * b + q]);
 }
 
 // After the recorded V-cycles of a captured solve: a box still active has not

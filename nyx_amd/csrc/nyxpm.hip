@@ -223,9 +223,10 @@ struct nyxpm_ctx {
     bool inc_suspended = false;   // no incremental re-sort (graph capture)
     long long holes = 0;          // slots emptied since the last full sort
     long long n_full_sorts = 0, n_inc_sorts = 0, n_moved = 0;
-    int* nmove = nullptr;
+    int* nmove = nullptr;         // of the last kick: [0] moves, [1] ndefer, [2..3] mig
     int* mig = nullptr;           // k_migrate flags: overflow, moved
     int* h_mig = nullptr;         // pinned mirror
+    int* hd_mig = nullptr;        // its device address
     long long* bsum = nullptr;
     // AssignDensityAndVels: halo slots of the three momentum deposits (allocated by the
     // first call, with the tile's size) and the per-box maxima
@@ -262,9 +263,12 @@ struct nyxpm_ctx {
     unsigned long long *nr = nullptr, *nf = nullptr;
     double *state = nullptr, *solv = nullptr, *dv_size = nullptr;
     BoxDev* dboxes = nullptr;
-    // host mirror of per-box flags
-    int* h_flags = nullptr;  // pinned: active[nbox] iters[nbox] failed[nbox] err
+    // host mirror of per-box flags and state (pinned), written by k_check
+    int* h_flags = nullptr;  // active[nbox] iters[nbox] failed[nbox] err
     double* h_state = nullptr;
+    int* hd_flags = nullptr;     // their device addresses
+    double* hd_state = nullptr;
+    bool results_ready = false;  // the mirror holds the last solve's results (no wait needed)
 
     // launch tables
     CellSeg* seg_pool = nullptr;
@@ -1024,8 +1028,9 @@ int alloc_fields(nyxpm_ctx* c) {
     if ((rc = dalloc(c, &c->phi, c->ncell_total))) return rc;
     if ((rc = alloc_tile_buffers(c))) return rc;
     if ((rc = dalloc(c, &c->partial, (size_t)c->t_l0.blocks))) return rc;
-    if ((rc = dalloc(c, &c->nmove, 1))) return rc;
-    if ((rc = dalloc(c, &c->mig, 2))) return rc;
+    if ((rc = dalloc(c, &c->nmove, 4))) return rc;
+    c->ndefer = c->nmove + 1;
+    c->mig = c->nmove + 2;
     if ((rc = dalloc(c, &c->guess_ok, 1))) return rc;
     HIPCK(c, hipMemset(c->guess_ok, 0, sizeof(int)));
     HIPCK(c, hipHostMalloc((void**)&c->h_mig, 2 * sizeof(int), hipHostMallocDefault));
@@ -1041,7 +1046,6 @@ int alloc_fields(nyxpm_ctx* c) {
     c->nheavy = c->nitems + 1;
     c->nsplit = c->nitems + 2;
     HIPCK(c, hipMemset(c->nitems, 0, 3 * sizeof(int)));
-    if ((rc = dalloc(c, &c->ndefer, 1))) return rc;
     if ((rc = dalloc(c, &c->dtmin, nbox))) return rc;
     if ((rc = dalloc(c, &c->mom_max, 3 * nbox))) return rc;
     if ((rc = dalloc(c, &c->nr, (size_t)nbox * kNormSlots))) return rc;
@@ -1054,6 +1058,9 @@ int alloc_fields(nyxpm_ctx* c) {
     HIPCK(c, hipHostMalloc((void**)&c->h_gstat, 2 * nbox * sizeof(int), hipHostMallocDefault));
     HIPCK(c, hipHostMalloc((void**)&c->h_flags, (3 * nbox + 1) * sizeof(int), hipHostMallocDefault));
     HIPCK(c, hipHostMalloc((void**)&c->h_state, 4 * nbox * sizeof(double), hipHostMallocDefault));
+    HIPCK(c, hipHostGetDevicePointer((void**)&c->hd_flags, c->h_flags, 0));
+    HIPCK(c, hipHostGetDevicePointer((void**)&c->hd_state, c->h_state, 0));
+    HIPCK(c, hipHostGetDevicePointer((void**)&c->hd_mig, c->h_mig, 0));
     HIPCK(c, hipMemset(c->phi, 0, c->ncell_total * sizeof(double)));
     HIPCK(c, hipMemset(c->nr, 0, (size_t)nbox * kNormSlots * sizeof(unsigned long long)));
     HIPCK(c, hipMemset(c->nf, 0, (size_t)nbox * kNormSlots * sizeof(unsigned long long)));
@@ -1115,14 +1122,15 @@ int ensure_idle_buffer(nyxpm_ctx* c) {
 // device phases
 // ---------------------------------------------------------------------------
 
+// Waits for the stream and reports the kernels' error flags.
 int err_check(nyxpm_ctx* c) {
-    int e = 0;
-    HIPCK(c, hipMemcpyAsync(&e, c->err_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    int* e = c->h_flags + 3 * c->boxes.size();
+    HIPCK(c, hipMemcpyAsync(e, c->err_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCK(c, hipStreamSynchronize(c->stream));
-    if (e) {
+    if (*e) {
         hipMemsetAsync(c->err_flag, 0, sizeof(int), c->stream);
         FAIL(c, NYXPM_ERR_STATE,
-             "particle outside one periodic image of its box or binning inconsistent (flags 0x%x)", e);
+             "particle outside one periodic image of its box or binning inconsistent (flags 0x%x)", *e);
     }
     return NYXPM_OK;
 }
@@ -1194,14 +1202,14 @@ void set_items(nyxpm_ctx* c, const ItemTables& t) {
     c->split_cap = (int)t.split_cap;
 }
 
-int make_items(nyxpm_ctx* c) {
+int make_items(nyxpm_ctx* c, const int* mig = nullptr) {
     Timed t(c, "items");
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nitems, 3LL, 0);
     const long long split_min = std::max((long long)kSplitTile, c->npart_total / kSplitShare);
     const int split_part = (int)std::max((long long)kSplitPart, c->npart_total / kSplitParts);
     hipLaunchKernelGGL(k_make_items, dim3(nblocks(c->ntiles_total)), dim3(kBlock), 0, c->stream, c->tbase,
                        c->cursor, c->ntiles_total, c->items, c->nitems, c->kick_chunk, c->heavy, c->nheavy,
-                       c->nsplit, split_min, split_part, c->split_cap);
+                       c->nsplit, split_min, split_part, c->split_cap, mig, c->hd_mig);
     LAUNCHCK(c);
     c->items_valid = true;
     return NYXPM_OK;
@@ -1216,18 +1224,19 @@ int phase_migrate(nyxpm_ctx* c, bool* done) {
     const long long* moves = reinterpret_cast<const long long*>(c->P[1 - c->cur].y);
     {
         Timed t(c, "migrate");
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->mig, 2LL, 0);
         hipLaunchKernelGGL(k_migrate, dim3(1024), dim3(kBlock), 0, c->stream, moves, c->nmove, c->dboxes, c->tbase,
                            c->tcap, c->cursor, A, c->mig, c->err_flag);
     }
     LAUNCHCK(c);
-    HIPCK(c, hipMemcpyAsync(c->h_mig, c->mig, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    // the items of the layout as migrated (made again if a full sort follows); the
+    // kernel also passes the flags to the host
+    int rc;
+    if ((rc = make_items(c, c->mig))) return rc;
     HIPCK(c, hipStreamSynchronize(c->stream));
     c->holes += c->h_mig[1];
     c->n_moved += c->h_mig[1];
     *done = c->h_mig[0] == 0 && c->holes * 1024 <= c->npart_total * (long long)c->hole_num;
     if (*done) ++c->n_inc_sorts;
-    if (*done) return make_items(c);
     return NYXPM_OK;
 }
 
@@ -1342,14 +1351,15 @@ int phase_rhs(nyxpm_ctx* c, double a, double four_pi_G) {
     return NYXPM_OK;
 }
 
+bool guess_wanted(const nyxpm_ctx* c) { return c->phi_guess == 2; }
+
 // Initial guess of a step's solve (nyxpm_pm_steps): phi_n as Nyx uses it, or on
 // request the linear extrapolation 2 phi_n - phi_{n-1} in time.  The stopping rule
 // is the same either way.
 void invalidate_guess(nyxpm_ctx* c) {
-    if (c->guess_ok) hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->guess_ok, 1LL, 0);
+    // (the flag is read only where the extrapolation is wanted)
+    if (c->guess_ok && guess_wanted(c)) hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->guess_ok, 1LL, 0);
 }
-
-bool guess_wanted(const nyxpm_ctx* c) { return c->phi_guess == 2; }
 
 // phi_{n-1}'s buffer; allocated before any graph capture (no hipMalloc inside one).
 int ensure_guess_buffer(nyxpm_ctx* c) {
@@ -1672,14 +1682,14 @@ int update(nyxpm_ctx* c) {
 int check(nyxpm_ctx* c, bool init, int fixed_iters, double rel, double abs_tol, int inc = 1) {
     const int nbox = (int)c->boxes.size();
     hipLaunchKernelGGL(k_check, dim3(nbox), dim3(kWave), 0, c->stream, init ? 1 : 0, fixed_iters, c->max_iter, rel,
-                       abs_tol, c->active, c->iters, c->failed, c->nr, c->nf, c->state, inc);
+                       abs_tol, c->active, c->iters, c->failed, c->nr, c->nf, c->state, inc, nbox,
+                       c->hd_flags, c->hd_state);
     LAUNCHCK(c);
     return NYXPM_OK;
 }
 
 int read_flags(nyxpm_ctx* c, bool* any_active) {
     const int nbox = (int)c->boxes.size();
-    HIPCK(c, hipMemcpyAsync(c->h_flags, c->active, nbox * sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCK(c, hipStreamSynchronize(c->stream));
     bool a = false;
     for (int b = 0; b < nbox; ++b) a = a || c->h_flags[b];
@@ -1743,6 +1753,7 @@ int solve_impl(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int gr
     for (int it = 0, g = g0; it <= limit; it += g, g = 1) {
         bool any;
         if ((rc = read_flags(c, &any))) return rc;
+        c->results_ready = !any;
         if (!any) break;
         if ((rc = vcycle_group<T>(c, g, rs))) return rc;
         if ((rc = res(false))) return rc;
@@ -1753,6 +1764,7 @@ int solve_impl(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int gr
 
 int solve(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int graph_cycles) {
     c->dt_valid = false;  // phi changes
+    c->results_ready = false;
     if (c->precision == NYXPM_MIXED) {
         int rc = ensure_mixed_pools(c);
         if (rc) return rc;
@@ -1764,11 +1776,9 @@ int solve(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int graph_c
 // Per-box results of the last solve; NYXPM_ERR_NOT_CONVERGED if any box failed.
 int solve_results(nyxpm_ctx* c, int* iters, double* final_res, bool allow_active) {
     const int nbox = (int)c->boxes.size();
-    HIPCK(c, hipMemcpyAsync(c->h_flags, c->active, nbox * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCK(c, hipMemcpyAsync(c->h_flags + nbox, c->iters, nbox * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCK(c, hipMemcpyAsync(c->h_flags + 2 * nbox, c->failed, nbox * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    HIPCK(c, hipMemcpyAsync(c->h_state, c->state, 4 * nbox * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCK(c, hipStreamSynchronize(c->stream));
+    // (a solve run eagerly ended with a wait behind its last check)
+    if (!c->results_ready) HIPCK(c, hipStreamSynchronize(c->stream));
+    c->results_ready = false;
     int bad = -1;
     for (int b = 0; b < nbox; ++b) {
         c->iters_seen = std::max(c->iters_seen, c->h_flags[nbox + b]);
@@ -1816,9 +1826,8 @@ int phase_kick_g(nyxpm_ctx* c, double dt, double a_prev, double a_cur, double a_
         // (the list lives in the idle buffer's y array, like the deferred list in x)
         const int inc = MOVE && c->slack_num > 0 && !c->inc_suspended ? 1 : 0;
         long long* moves = reinterpret_cast<long long*>(c->P[1 - c->cur].y);
-        if (inc)
-            hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nmove, 1LL, 0);
-        else if (MOVE)
+        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nmove, 4LL, 0);
+        if (MOVE && !inc)
             hipLaunchKernelGGL(k_fill_int, dim3(nblocks(c->ntiles_total)), dim3(kBlock), 0, c->stream, c->counts,
                                c->ntiles_total, 0);
         // the deferred-particle list lives in the sort target's x array (as many
@@ -1829,7 +1838,6 @@ int phase_kick_g(nyxpm_ctx* c, double dt, double a_prev, double a_cur, double a_
         if (cfl > 0)
             hipLaunchKernelGGL(k_fill_dbl, dim3(1), dim3(kBlock), 0, c->stream, reinterpret_cast<double*>(c->dtmin),
                                (long long)c->boxes.size(), 1e50);
-        hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->ndefer, 1LL, 0);
         auto kern = cfl > 0 ? k_kick_tiled<MODE, MODE != kKickDrift, G> : k_kick_tiled<MODE, false, G>;
         hipLaunchKernelGGL(kern, dim3((unsigned)c->items_cap), dim3(kBlock), lds, c->stream, c->tseg, c->tseg_n,
                            c->dboxes, c->items, c->nitems, c->phi, A.x, A.y, A.z, A.vx, A.vy, A.vz, dt, a_prev,
@@ -2146,7 +2154,7 @@ int nyxpm_destroy(nyxpm_ctx* c) {
     if (c->graph) hipGraphDestroy(c->graph);
     free_particles(c);
     dfree(c->counts); dfree(c->cursor); dfree(c->tstart); dfree(c->bsum);
-    dfree(c->tbase); dfree(c->tcap); dfree(c->mom_halo); dfree(c->mom_max); dfree(c->nmove); dfree(c->mig); dfree(c->phi_prev); dfree(c->guess_ok);
+    dfree(c->tbase); dfree(c->tcap); dfree(c->mom_halo); dfree(c->mom_max); dfree(c->nmove); dfree(c->phi_prev); dfree(c->guess_ok);
     if (c->h_mig) hipHostFree(c->h_mig);
     c->rho = nullptr;
     dfree(c->own); dfree(c->halo); dfree(c->f); dfree(c->phi); dfree(c->partial);
@@ -2154,7 +2162,7 @@ int nyxpm_destroy(nyxpm_ctx* c) {
     dfree(c->r64); dfree(c->e64); dfree(c->e64b); dfree(c->G64);
     dfree(c->r32); dfree(c->e32); dfree(c->e32b);
     dfree(c->active); dfree(c->iters); dfree(c->failed); dfree(c->err_flag); dfree(c->nitems); dfree(c->nr); dfree(c->nf);
-    dfree(c->ndefer); dfree(c->dtmin);
+    dfree(c->dtmin);
     dfree(c->state); dfree(c->solv); dfree(c->dv_size); dfree(c->dboxes);
     dfree(c->seg_pool); dfree(c->pseg); dfree(c->tseg); dfree(c->cc_first);
     dfree(c->gstat);
@@ -2184,7 +2192,6 @@ int nyxpm_set_stream(nyxpm_ctx* c, void* s) {
 
 int nyxpm_sync(nyxpm_ctx* c) {
     if (!c) return NYXPM_ERR_ARG;
-    HIPCK(c, hipStreamSynchronize(c->stream));
     return err_check(c);
 }
 
@@ -2508,7 +2515,6 @@ static int shift_into_box(nyxpm_ctx* c) {
                        A.y, A.z, c->err_flag);
     LAUNCHCK(c);
     c->keys_valid = c->sorted_valid = c->density_valid = false;
-    HIPCK(c, hipStreamSynchronize(c->stream));
     return err_check(c);
 }
 
@@ -2742,7 +2748,6 @@ int nyxpm_assign_density(nyxpm_ctx* c, int box, double* rho_out) {
         HIPCK(c, hipMemcpyAsync(rho_out, c->rho + B.cell_off, B.lev[0].nc * sizeof(double), hipMemcpyDefault,
                                 c->stream));
     }
-    HIPCK(c, hipStreamSynchronize(c->stream));
     return err_check(c);
 }
 
@@ -2933,7 +2938,6 @@ int nyxpm_gather_accel_noalloc(nyxpm_ctx* c, int box, double* g_out) {
     if ((rc = launch_gather(c, box, dev ? g_out : c->scratch_dev))) return rc;
     if (!dev)
         HIPCK(c, hipMemcpyAsync(g_out, c->scratch_dev, 3 * B.np * sizeof(double), hipMemcpyDeviceToHost, c->stream));
-    HIPCK(c, hipStreamSynchronize(c->stream));
     return err_check(c);
 }
 

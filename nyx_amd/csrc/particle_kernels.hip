@@ -983,8 +983,11 @@ __global__ void __launch_bounds__(kBlock) k_make_items(const long long* __restri
                                                        const int* __restrict__ thw, long long ntiles,
                                                        TileItem* __restrict__ items, int* nitems, int chunk,
                                                        HeavyItem* __restrict__ heavy, int* nheavy, int* nsplit,
-                                                       long long split_min, int split_part, int split_cap) {
+                                                       long long split_min, int split_part, int split_cap,
+                                                       const int* mig, int* h_mig) {
     const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
+    // the migration's flags to the host's mirror (pinned memory) along the way
+    if (mig && t < 2) __hip_atomic_store(&h_mig[t], mig[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     int nc = 0;
     long long p0 = 0, cnt = 0;
     if (t < ntiles) {
