@@ -176,6 +176,7 @@ struct nyxpm_ctx {
     int force_tx[2] = {0, 0}, force_ty[2] = {8, 8};  // fixed sweep shape per precision (0: chosen)
     bool fuse_update = true;    // phi += e in the last finest-level sweep
     int kick_chunk = kChunk;    // particles per work item of the tile-staged kicks
+    int kick_chunk_opt = 0;     // set in the options (0: chosen with the slots, choose_chunk)
     hipStream_t stream = nullptr;
     bool own_stream = false;
     std::vector<Box> boxes;
@@ -1160,11 +1161,31 @@ struct ItemTables {
     unsigned long long* split_acc = nullptr;
     int* split_done = nullptr;
     long long items_cap = 0, heavy_cap = 0, split_cap = 0;
+    int chunk = 0;
 };
+
+// Particles per work item of the tile-staged kernels for `slots` slots.  An item stages
+// its tile's phi once, so large items cost least in all (kChunk), but an item is a
+// serial loop of ~2 us per 256 particles: halved down to a block's threads while the
+// slots make fewer than kItemsMin items, and, while there are fewer than kItemsMany,
+// at most the power of two from 1.5 times the average tile, so that ordinary tiles stay
+// whole and a clump's tiles are cut.
+// Paired kick, us, 4096 everywhere -> the rule: 32^3 FP64 22 -> 17, 112x96x144 with 10^6
+// clustered particles 66 -> 59, 160^3 with 3 10^6 132 -> 122; 64^3 (29), 128^3 (63) and
+// 256^3 (500) as before.
+constexpr long long kItemsMin = 512, kItemsMany = 4096;
+int choose_chunk(const nyxpm_ctx* c, long long slots) {
+    if (c->kick_chunk_opt) return c->kick_chunk_opt;
+    int chunk = kChunk;
+    while (chunk > kBlock && slots / chunk < kItemsMin) chunk /= 2;
+    while (slots / kChunk < kItemsMany && chunk > kBlock && chunk / 2 * c->ntiles_total * 2 >= slots * 3) chunk /= 2;
+    return chunk;
+}
 
 // New tables for `slots` particle slots (the context's stay until set_items).
 int alloc_items(nyxpm_ctx* c, long long slots, ItemTables* t) {
-    t->items_cap = c->ntiles_total + slots / c->kick_chunk + 1;
+    t->chunk = choose_chunk(c, slots);
+    t->items_cap = c->ntiles_total + slots / t->chunk + 1;
     if (t->items_cap > 0x7fffffffLL) FAIL(c, NYXPM_ERR_ARG, "too many tile chunks");
     // a heavy tile's whole block stands for more than kHeavyTile slots, a part of a
     // split one for at least 2/3 kSplitPart on average (three parts from 4097 slots,
@@ -1195,6 +1216,7 @@ int alloc_items(nyxpm_ctx* c, long long slots, ItemTables* t) {
 void set_items(nyxpm_ctx* c, const ItemTables& t) {
     c->items = t.items;
     c->items_cap = t.items_cap;
+    c->kick_chunk = t.chunk;
     c->heavy = t.heavy;
     c->heavy_cap = (int)t.heavy_cap;
     c->split_acc = t.split_acc;
@@ -2096,7 +2118,7 @@ int nyxpm_create_batch(nyxpm_ctx** out, int nbox, const nyxpm_geom* geoms, const
             c->force_ty[0] = c->force_ty[1] = opts->sweep_ty > 0 ? opts->sweep_ty : 8;
         }
         if (opts->sweep_zchunk > 0) c->sweep_zchunk = opts->sweep_zchunk;
-        if (opts->kick_chunk > 0) c->kick_chunk = std::max(kBlock, opts->kick_chunk);
+        if (opts->kick_chunk > 0) c->kick_chunk_opt = std::max(kBlock, opts->kick_chunk);
         if (opts->phi_guess >= 0 && opts->phi_guess <= 2) c->phi_guess = opts->phi_guess;
         c->fuse_res = opts->residual == 1;
         if (opts->graph_cycles > 0) c->graph_cycles = opts->graph_cycles;
