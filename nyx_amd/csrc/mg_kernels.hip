@@ -1736,6 +1736,76 @@ __global__ void __launch_bounds__(kResTX * kResTY) k_residual0(const CellSeg* se
     }
 }
 
+// The same for small boxes, a thread per pair of x-adjacent cells: a box that does not
+// fill the chip is bound by the latency of the march above (8.7 us up to 64^3), not by
+// reading a plane's neighbours from the caches.  Needs even nx.
+// Whole solves, us per V-cycle FP64 / mixed, against the march: 32^3 58 / 44 -> 53 / 42,
+// 64^3 78 / 60 -> 74 / 58, 96^3 107 / 83 -> 103 / 81, 128^3 130 / 96 -> 128 / 94;
+// 160x192x224 252 / 180 -> 254 / 182.
+template <typename T>
+__global__ void __launch_bounds__(kResTX * kResTY) k_residual_cells(const CellSeg* segs, int nseg, const int* active,
+                                                                   const double* __restrict__ f,
+                                                                   const double* __restrict__ solv, double Ggravity,
+                                                                   double inv_a, const double* __restrict__ phi,
+                                                                   T* __restrict__ r, unsigned long long* nr,
+                                                                   unsigned long long* nf) {
+    constexpr int NT = kResTX * kResTY;
+    const CellSeg& sg = segs[find_seg(segs, nseg, blockIdx.x)];
+    if (!active[sg.box]) return;
+    const int nx = sg.n[0], ny = sg.n[1], nz = sg.n[2];
+    const unsigned hx = nx >> 1, np = hx * ny * nz;
+    const unsigned q = (blockIdx.x - sg.blk0) * NT + threadIdx.x;
+    double ar = 0.0, af = 0.0;
+    if (q < np) {
+        const unsigned t = q / hx, k = t / ny;
+        const int m = q - t * hx, j = t - k * ny;
+        const size_t o = 2 * (size_t)q, plane = (size_t)nx * ny;
+        const double* P = phi + sg.coff + o;
+        const long long xm = m == 0 ? nx - 1 : -1, xp = m == (int)hx - 1 ? 2 - nx : 2;
+        const long long ym = j == 0 ? (long long)(ny - 1) * nx : -nx, yp = j == ny - 1 ? -(long long)(ny - 1) * nx : nx;
+        const long long zm = k == 0 ? (long long)(nz - 1) * plane : -(long long)plane;
+        const long long zp = (int)k == nz - 1 ? -(long long)(nz - 1) * plane : (long long)plane;
+        auto pair = [](const double* p) { return *reinterpret_cast<const CellPair<double>*>(p); };
+        const CellPair<double> c = pair(P), y0 = pair(P + ym), y1 = pair(P + yp), z0 = pair(P + zm), z1 = pair(P + zp);
+        const double l = P[xm], rt = P[xp];
+        CellPair<double> fv = pair(f + sg.coff + o);
+        const double dhx = sg.dh[0], dhy = sg.dh[1], dhz = sg.dh[2];
+        if (solv) {
+            const double ns = -solv[sg.box];
+            const double ta = fv.a + ns, tb = fv.b + ns;
+            fv.a = (ta * Ggravity) * inv_a;
+            fv.b = (tb * Ggravity) * inv_a;
+        }
+        const double axv = dhx * (l - 2.0 * c.a + c.b), bxv = dhx * (c.a - 2.0 * c.b + rt);
+        const double ayv = dhy * (y0.a - 2.0 * c.a + y1.a), byv = dhy * (y0.b - 2.0 * c.b + y1.b);
+        const double azv = dhz * (z0.a - 2.0 * c.a + z1.a), bzv = dhz * (z0.b - 2.0 * c.b + z1.b);
+        const double va = fv.a - (axv + ayv + azv), vb = fv.b - (bxv + byv + bzv);
+        *reinterpret_cast<CellPair<T>*>(r + sg.off + o) = CellPair<T>{T(va), T(vb)};
+        ar = fmax(fabs(va), fabs(vb));
+        af = fmax(fabs(fv.a), fabs(fv.b));
+    }
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        ar = fmax(ar, __shfl_xor(ar, o));
+        af = fmax(af, __shfl_xor(af, o));
+    }
+    __shared__ double wr[NT / kWave], wf[NT / kWave];
+    if ((threadIdx.x & (kWave - 1)) == 0) {
+        wr[threadIdx.x / kWave] = ar;
+        wf[threadIdx.x / kWave] = af;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double mr = wr[0], mf = wf[0];
+        for (int w = 1; w < NT / kWave; ++w) {
+            mr = fmax(mr, wr[w]);
+            mf = fmax(mf, wf[w]);
+        }
+        const int slot = sg.box * kNormSlots + (blockIdx.x & (kNormSlots - 1));
+        atomicMax(&nr[slot], dbits(mr));
+        if (nf) atomicMax(&nf[slot], dbits(mf));
+    }
+}
+
 // phi += e (level 0).
 template <typename T>
 __global__ void __launch_bounds__(kBlock) k_update0(const CellSeg* segs, int nseg, const int* active,

@@ -313,6 +313,7 @@ struct nyxpm_ctx {
     int* cc_first = nullptr;
     size_t cc_lds[2] = {0, 0};
     Table t_resz;                 // level 0, z-marching residual columns
+    Table t_resc;                 // or, where all boxes are small, a thread per pair of cells
     BoxSeg* pseg = nullptr;
     int pseg_n = 0, pseg_blocks = 0;
     BoxSeg* tseg = nullptr;
@@ -589,6 +590,10 @@ double sw2_model(int pr, int tx, int ty, int zc, const std::vector<const Level*>
     const double march = 3.0 + rounds * planes * (pr == 0 ? 0.33 + 0.034 * w : 0.27 + 0.022 * w);
     return std::max(march, lines / 1e7);
 }
+
+// Cells of all boxes up to which the residual takes a thread per pair of cells (figures
+// at k_residual_cells).
+constexpr long long kResCells = 1ll << 21;
 
 // Cells of a depth's levels (all boxes) up to which its V-cycle legs run as one launch
 // each (k_leg); above, a paired pass and a restriction, whose halos cost less.
@@ -916,6 +921,20 @@ int build_tables(nyxpm_ctx* c) {
         while (res_pieces(rzc) < 512 && rzc > 4) rzc /= 2;
         c->t_res = add_table(vr);
         c->t_resz = add_table(vz);
+        std::vector<CellSeg> vc;
+        long long cells = 0;
+        bool even = true;
+        for (int b = 0; b < nbox; ++b) {
+            const Level& L = c->boxes[b].lev[0];
+            CellSeg s = mk(b, 0, 1);
+            s.coff = c->boxes[b].cell_off;
+            s.nblk = nblocks((L.nc + 1) / 2, kResTX * kResTY);
+            cells += L.nc;
+            even = even && L.n[0] % 2 == 0;
+            vc.push_back(s);
+        }
+        if (!even || cells > kResCells) vc.clear();
+        c->t_resc = add_table(vc);
     }
     int rc = dalloc(c, &c->seg_pool, S.size());
     if (rc) return rc;
@@ -1686,9 +1705,12 @@ int residual_sweep0(nyxpm_ctx* c, bool with_f) {
 template <typename T>
 int residual(nyxpm_ctx* c, bool with_f) {
     Timed t(c, "residual");
-    hipLaunchKernelGGL(k_residual0<T>, dim3(c->t_resz.blocks), dim3(kResTX * kResTY), 0, c->stream,
-                       c->segs(c->t_resz), c->t_resz.count, c->active, c->f, c->f_raw ? c->solv : nullptr,
-                       c->f_G, c->f_inv_a, c->phi, Pools<T>::r(c), c->nr, with_f ? c->nf : nullptr);
+    const bool small = c->t_resc.count > 0;
+    const auto& tab = small ? c->t_resc : c->t_resz;
+    auto kern = small ? k_residual_cells<T> : k_residual0<T>;
+    hipLaunchKernelGGL(kern, dim3(tab.blocks), dim3(kResTX * kResTY), 0, c->stream, c->segs(tab), tab.count,
+                       c->active, c->f, c->f_raw ? c->solv : nullptr, c->f_G, c->f_inv_a, c->phi, Pools<T>::r(c),
+                       c->nr, with_f ? c->nf : nullptr);
     return NYXPM_OK;
 }
 

@@ -14,11 +14,13 @@ def mean_free(n, seed):
     return f - f.mean()
 
 
-@pytest.mark.parametrize("n", [(32, 32, 32), (66, 18, 10), (130, 34, 6), (40, 24, 18)])
+@pytest.mark.parametrize("n", [(32, 32, 32), (66, 18, 10), (130, 34, 6), (40, 24, 18), (15, 16, 14),
+                               (144, 112, 144)])
 def test_residual_chunks_bitwise(nyx, orc, n):
-    # the level-0 residual in short z-chunks (small boxes), chunks that do not
-    # divide the box and columns that pass its edge: iterates and norms of two
-    # V-cycles from a non-zero guess, bit for bit
+    # the level-0 residual by pairs of cells (small boxes of even nx, blocks past the
+    # last pair), and by marched columns that pass its edge (odd nx, and above 2^21
+    # cells): iterates and norms of two V-cycles from a
+    # non-zero guess, bit for bit
     f = mean_free(n, 31)
     guess = mean_free(n, 32)
     dx = [1.0 / 32] * 3
@@ -26,9 +28,12 @@ def test_residual_chunks_bitwise(nyx, orc, n):
     with ctx1(nyx, n, hi=hi) as c:
         phi, it, norms = c.solve_poisson(f, guess, fixed_iters=2)
     ref, it2, st, _ = orc.mg_solve(n, dx, f, guess, fixed_iters=2)
+    assert np.array_equal(norms[:2], st[:2])
+    if n[0] % 2:  # a bottom alone, solved exactly: only the first residual compares in bits
+        return
     assert it == it2 == 2
     assert np.array_equal(phi, ref)
-    assert np.array_equal(norms[:3], st[:3])
+    assert norms[2] == st[2]
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
