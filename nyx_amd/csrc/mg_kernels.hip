@@ -1034,8 +1034,9 @@ __global__ void __launch_bounds__(kBlock) k_resid_restrict(const CellSeg* segs, 
 // coarse plane K in LDS, the next planes fetched into registers during the
 // compute.  Each fine value is read once per block (plus the x-y halo), where the
 // thread-per-cell kernel fetched the e planes between coarse planes twice.  Same
-// arithmetic (lap7's, children summed k, j, i) bit for bit.  Needs nx % 2CX ==
-// ny % 2CY == nz % 2 == 0.
+// arithmetic (lap7's, children summed k, j, i) bit for bit.  Needs even nx >= 2CX,
+// ny >= 2CY and nz; the last column of a row is moved back to end at the level's edge
+// and writes the same values as its neighbour where they overlap.
 template <typename T, int CX, int CY>
 __global__ void __launch_bounds__(CX * CY) k_resid_restrict_z(const CellSeg* segs, int nseg, const int* active,
                                                               const T* __restrict__ e, T* __restrict__ r) {
@@ -1052,10 +1053,10 @@ __global__ void __launch_bounds__(CX * CY) k_resid_restrict_z(const CellSeg* seg
     if (!active[sg.box]) return;
     const int nx = sg.n[0], ny = sg.n[1], nz = sg.n[2];
     const int cx = nx >> 1, cy = ny >> 1, cz = nz >> 1;
-    const int ntx = nx / RX, nty = ny / RY;
+    const int ntx = (nx + RX - 1) / RX, nty = (ny + RY - 1) / RY;
     const int b = bid - sg.blk0;
     const int tx = b % ntx, ty = (b / ntx) % nty, tz = b / (ntx * nty);
-    const int x0 = tx * RX, y0 = ty * RY;
+    const int x0 = min(tx * RX, nx - RX), y0 = min(ty * RY, ny - RY);
     const int K0 = tz * sg.zchunk, K1 = min(cz, K0 + sg.zchunk);
     const T dhx = T(sg.dh[0]), dhy = T(sg.dh[1]), dhz = T(sg.dh[2]);
     const T* E = e + sg.off;

@@ -132,6 +132,7 @@ def test_device_download_equals_host_download(nyx, npart, slack):
     [(16, 8, 40)],                # the smallest shape
     [(5, 5, 5), (100, 36, 28)],   # a batch whose first box has no smoothing level
     [(144, 80, 48), (48, 64, 40)],
+    [(160, 80, 96)],              # restrictions by narrow marched tiles
 ])
 def test_paired_smoothing_equals_half_sweeps(nyx, boxes, precision, sweep2):
     # whole cycle legs in one launch (sweep2 = 0, these sizes) and smoothing pairs as
