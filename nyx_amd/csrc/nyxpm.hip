@@ -308,6 +308,7 @@ struct nyxpm_ctx {
     std::vector<int> pre_buf;    // buffer holding e after pre-smoothing, per depth
     std::vector<int> fin_buf;    // buffer holding e after post-smoothing, per depth
     Table t_bottom, t_l0, t_res;  // t_res: level 0, at most kReduceBlocks blocks per box
+    Table t_fold;                 // k_fold's blocks, each one or more of t_res's
     // one-workgroup coarse V-cycle: per box, levels dc..nlev-1 (cc_first[b] ..
     // cc_first[b+1]-1 of table t_cc) and the LDS it needs per precision
     Table t_cc;
@@ -950,6 +951,17 @@ int build_tables(nyxpm_ctx* c) {
         int rzc = 64;
         while (res_pieces(rzc) < 512 && rzc > 4) rzc /= 2;
         c->t_res = add_table(vr);
+        // k_fold: kFoldU of t_res's blocks each where those have one cell per thread
+        std::vector<CellSeg> vf;
+        for (int b = 0; b < nbox; ++b) {
+            CellSeg s = S[c->t_res.first + b];
+            s.coff = s.blk0;
+            s.ebuf = s.nblk;
+            s.zchunk = (c->boxes[b].lev[0].nc + s.nblk - 1) / s.nblk <= kBlock ? kFoldU : 1;
+            s.nblk = (s.nblk + s.zchunk - 1) / s.zchunk;
+            vf.push_back(s);
+        }
+        c->t_fold = add_table(vf);
         c->t_resz = add_table(vz);
         std::vector<CellSeg> vc;
         long long cells = 0;
@@ -1386,11 +1398,11 @@ int phase_deposit(nyxpm_ctx* c, bool want_rho, bool f32 = false) {
     {
         Timed t(c, "fold");
         if (want_rho)
-            hipLaunchKernelGGL(k_fold<true>, dim3(c->t_res.blocks), dim3(kBlock), 0, c->stream, c->segs(c->t_res),
-                               c->t_res.count, c->dboxes, c->own, c->halo, c->rho, c->f, c->partial);
+            hipLaunchKernelGGL(k_fold<true>, dim3(c->t_fold.blocks), dim3(kBlock), 0, c->stream, c->segs(c->t_fold),
+                               c->t_fold.count, c->dboxes, c->own, c->halo, c->rho, c->f, c->partial);
         else
-            hipLaunchKernelGGL(k_fold<false>, dim3(c->t_res.blocks), dim3(kBlock), 0, c->stream,
-                               c->segs(c->t_res), c->t_res.count, c->dboxes, c->own, c->halo, c->rho, c->f,
+            hipLaunchKernelGGL(k_fold<false>, dim3(c->t_fold.blocks), dim3(kBlock), 0, c->stream,
+                               c->segs(c->t_fold), c->t_fold.count, c->dboxes, c->own, c->halo, c->rho, c->f,
                                c->partial);
     }
     LAUNCHCK(c);

@@ -649,22 +649,26 @@ __device__ __forceinline__ void for_block_cells(const CellSeg& sg, const BoxDev&
 // has up to 4U loads in flight; the edge and corner terms (cells on two or
 // three top faces of a tile) follow them.  Coordinates advance by kBlock cells
 // with block-uniform carries instead of divisions.  C fields of the same tiles at
-// once (their addresses derived once): emit(q, v) gets the C values of a cell.
+// once (their addresses derived once): emit(q, v, u) gets the C values of a cell, the
+// u-th of the thread's U in flight.  V consecutive shares of the piece's nv in one block
+// (its block b takes shares b*V ..): with shares of kBlock cells and V <= U, the u-th
+// cell of a thread is its one cell of share b*V + u.
 template <int C>
 struct FoldFields {
     const double* own[C];
     const double* halo[C];
 };
 template <int U, int C, class F>
-__device__ __forceinline__ void fold_walk(const CellSeg& sg, const BoxDev& B, const FoldFields<C>& fields, F emit) {
+__device__ __forceinline__ void fold_walk(const CellSeg& sg, int nv, int V, const BoxDev& B,
+                                          const FoldFields<C>& fields, F emit) {
     const int nx = B.n[0], ny = B.n[1], nz = B.n[2];
     const int T0 = B.tile[0], T1 = B.tile[1], T2 = B.tile[2];
     const int nt0 = B.ntile[0], nt1 = B.ntile[1], nt2 = B.ntile[2];
     const long long N = (long long)nx * ny * nz;
-    long long per = (N + sg.nblk - 1) / sg.nblk;
+    long long per = (N + nv - 1) / nv;
     per = (per + kBlock - 1) / kBlock * kBlock;
-    const long long c0 = (long long)(blockIdx.x - sg.blk0) * per;
-    const long long c1 = min(N, c0 + per);
+    const long long c0 = (long long)(blockIdx.x - sg.blk0) * V * per;
+    const long long c1 = min(N, c0 + V * per);
     long long c = c0 + threadIdx.x;
     if (c >= c1) return;
     const long long plane = (long long)nx * ny;
@@ -752,7 +756,7 @@ __device__ __forceinline__ void fold_walk(const CellSeg& sg, const BoxDev& B, co
                     w[f] = fold_edges(B, fields.halo[f], w[f], tx, ty, tz, cx[u] - tx * T0, cy[u] - ty * T1,
                                       cz[u] - tz * T2, top & 1, top & 2, top & 4);
             }
-            emit(B.cell_off + (size_t)(c + (long long)u * kBlock), w);
+            emit(B.cell_off + (size_t)(c + (long long)u * kBlock), w, u);
         }
     }
 }
@@ -760,10 +764,14 @@ __device__ __forceinline__ void fold_walk(const CellSeg& sg, const BoxDev& B, co
 // Cells per thread in flight in the fold.
 constexpr int kFoldU = 4;
 
-// rho = (own + halos, fold_walk) * 1/vol; f = rho + (-mass_offset); per-block sum
-// of f for the solvability correction.  Cells in row-major order (coalesced reads
-// of own and writes of f, whole cache lines).  rho itself is written only when the
-// caller wants the density (AssignDensity); the step needs only f.
+// rho = (own + halos, fold_walk) * 1/vol; f = rho + (-mass_offset); sum of f per share
+// for the solvability correction.  Cells in row-major order (coalesced reads of own and
+// writes of f, whole cache lines).  rho itself is written only when the caller wants the
+// density (AssignDensity); the step needs only f.
+// The shares (and so the order of the sums) are the reducing table's blocks: piece s has
+// s.ebuf of them from partial[s.coff] on, s.zchunk per block of this launch.  In boxes
+// of up to 2^21 cells a share is one cell per thread, too little to have loads in
+// flight: four shares per block took 52M cells of 64^3-128^3 boxes from 0.54 to 0.31 ms.
 template <bool WRITE_RHO>
 __global__ void __launch_bounds__(kBlock) k_fold(const CellSeg* segs, int nseg, const BoxDev* boxes,
                                                  const double* own, const double* __restrict__ halo,
@@ -772,17 +780,37 @@ __global__ void __launch_bounds__(kBlock) k_fold(const CellSeg* segs, int nseg, 
     // rho may be own itself (each cell is read, then written, by one thread)
     const CellSeg& sg = segs[find_seg(segs, nseg, blockIdx.x)];
     const BoxDev B = boxes[__builtin_amdgcn_readfirstlane(sg.box)];
-    double acc = 0.0;  // this thread's cells, in a fixed order
+    const int V = sg.zchunk, nv = sg.ebuf;
+    double acc[kFoldU];  // this thread's cells of each share, in a fixed order
+#pragma unroll
+    for (int u = 0; u < kFoldU; ++u) acc[u] = 0.0;
     const FoldFields<1> fields{{own}, {halo}};
-    fold_walk<kFoldU, 1>(sg, B, fields, [&](size_t q, const double (&v)[1]) {
+    fold_walk<kFoldU, 1>(sg, nv, V, B, fields, [&](size_t q, const double (&v)[1], int u) {
         const double rv = v[0] * B.inv_vol;
         if (WRITE_RHO) rho[q] = rv;
         const double fv = rv + (-B.mass_offset);
         f[q] = fv;
-        acc += fv;
+        if (V == 1)
+            acc[0] += fv;
+        else
+            acc[u] += fv;
     });
-    const double bs = block_sum_fixed(acc);
-    if (threadIdx.x == 0) partial[blockIdx.x] = bs;
+    const int b0 = (int)(blockIdx.x - sg.blk0) * V;
+    // each share's sum as block_sum_fixed forms it: a butterfly per wave, then the waves
+    // in order
+    __shared__ double ws[kFoldU][kBlock / kWave];
+#pragma unroll
+    for (int u = 0; u < kFoldU; ++u) {
+        if (u >= V) break;
+        for (int o = kWave / 2; o > 0; o >>= 1) acc[u] += __shfl_xor(acc[u], o);
+        if ((threadIdx.x & (kWave - 1)) == 0) ws[u][threadIdx.x / kWave] = acc[u];
+    }
+    __syncthreads();
+    if ((int)threadIdx.x < V && b0 + (int)threadIdx.x < nv) {
+        double t = 0.0;
+        for (int w = 0; w < kBlock / kWave; ++w) t += ws[threadIdx.x][w];
+        partial[sg.coff + b0 + threadIdx.x] = t;
+    }
 }
 
 // AssignDensityAndVels for one box (segs: its piece): the folded mass and momenta,
@@ -795,7 +823,7 @@ __global__ void __launch_bounds__(kBlock) k_fold_vels(const CellSeg* segs, const
     sg.blk0 = 0;
     const BoxDev B = boxes[__builtin_amdgcn_readfirstlane(sg.box)];
     const size_t nc = (size_t)B.n[0] * B.n[1] * B.n[2];
-    fold_walk<2, 4>(sg, B, fields, [&](size_t q, const double (&v)[4]) {
+    fold_walk<2, 4>(sg, sg.nblk, 1, B, fields, [&](size_t q, const double (&v)[4], int) {
         double* o = out + (q - B.cell_off);
         const double ms = v[0];
         o[0] = ms * B.inv_vol;
@@ -809,7 +837,16 @@ __global__ void __launch_bounds__(kBlock) k_rhs_sum(const CellSeg* segs, const d
                                                     const double* __restrict__ dv_size, double* __restrict__ solv) {
     const CellSeg& sg = segs[blockIdx.x];
     double s = 0.0;
-    for (int b = threadIdx.x; b < sg.nblk; b += kBlock) s += partial[sg.blk0 + b];
+    // eight loads in flight, added in order (a load at a time: 12 us for 8192 shares)
+    constexpr int U = 8;
+    for (int b = threadIdx.x; b < sg.nblk; b += U * kBlock) {
+        double v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) v[u] = partial[sg.blk0 + min(b + u * kBlock, sg.nblk - 1)];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (b + u * kBlock < sg.nblk) s += v[u];
+    }
     const double S = block_sum_fixed(s);
     if (threadIdx.x == 0) {
         double sum = S * dv_size[2 * sg.box];
