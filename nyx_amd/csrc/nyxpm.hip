@@ -221,7 +221,10 @@ struct nyxpm_ctx {
     int slack_num = 256, slack_pad = 16;
     int hole_num = 64;            // full sort once the emptied slots exceed np * hole_num / 1024
     bool moves_pending = false;
-    bool inc_suspended = false;   // no incremental re-sort (graph capture)
+    bool capturing = false;       // a step is being recorded: nothing is read back
+    long long* resort = nullptr;  // a replay's re-sort state (Resort::state) and its pinned mirror
+    long long* h_resort = nullptr;
+    long long* hd_resort = nullptr;
     long long holes = 0;          // slots emptied since the last full sort
     long long n_full_sorts = 0, n_inc_sorts = 0, n_moved = 0;
     int* nmove = nullptr;         // of the last kick: [0] moves, [1] ndefer, [2..3] mig
@@ -1096,6 +1099,9 @@ int alloc_fields(nyxpm_ctx* c) {
     if ((rc = dalloc(c, &c->guess_ok, 1))) return rc;
     HIPCK(c, hipMemset(c->guess_ok, 0, sizeof(int)));
     HIPCK(c, hipHostMalloc((void**)&c->h_mig, 2 * sizeof(int), hipHostMallocDefault));
+    if ((rc = dalloc(c, &c->resort, 4))) return rc;
+    HIPCK(c, hipHostMalloc((void**)&c->h_resort, 4 * sizeof(long long), hipHostMallocDefault));
+    HIPCK(c, hipHostGetDevicePointer((void**)&c->hd_resort, c->h_resort, 0));
     if ((rc = dalloc(c, &c->r64, c->mg_total))) return rc;
     if ((rc = dalloc(c, &c->e64, c->mg_total))) return rc;
     if ((rc = dalloc(c, &c->e64b, c->mg_total))) return rc;
@@ -1285,14 +1291,14 @@ void set_items(nyxpm_ctx* c, const ItemTables& t) {
     c->split_cap = (int)t.split_cap;
 }
 
-int make_items(nyxpm_ctx* c, const int* mig = nullptr) {
+int make_items(nyxpm_ctx* c, const int* mig = nullptr, const Resort& resort = {}) {
     Timed t(c, "items");
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nitems, 3LL, 0);
     const long long split_min = std::max((long long)kSplitTile, c->npart_total / kSplitShare);
     const int split_part = (int)std::max((long long)kSplitPart, c->npart_total / kSplitParts);
     hipLaunchKernelGGL(k_make_items, dim3(nblocks(c->ntiles_total)), dim3(kBlock), 0, c->stream, c->tbase,
                        c->cursor, c->ntiles_total, c->items, c->nitems, c->kick_chunk, c->heavy, c->nheavy,
-                       c->nsplit, split_min, split_part, c->split_cap, mig, c->hd_mig);
+                       c->nsplit, split_min, split_part, c->split_cap, mig, c->hd_mig, resort, c->hd_resort);
     LAUNCHCK(c);
     c->items_valid = true;
     return NYXPM_OK;
@@ -1323,6 +1329,29 @@ int phase_migrate(nyxpm_ctx* c, bool* done) {
     return NYXPM_OK;
 }
 
+// The same in a captured step: the migration, and the full sort that it may ask for
+// decided on the device, in place (see Resort).
+int captured_resort(nyxpm_ctx* c) {
+    PartPtrs& A = c->P[c->cur];
+    PartPtrs& I = c->P[1 - c->cur];
+    const long long* moves = reinterpret_cast<const long long*>(I.y);
+    const Resort r{c->mig, c->resort, c->npart_total, c->hole_num};
+    const dim3 grid(std::min(c->pseg_blocks, 2048));
+    hipLaunchKernelGGL(k_fill_int, dim3(nblocks(c->ntiles_total)), dim3(kBlock), 0, c->stream, c->counts,
+                       c->ntiles_total, 0);
+    hipLaunchKernelGGL(k_migrate, dim3(1024), dim3(kBlock), 0, c->stream, moves, c->nmove, c->dboxes, c->tbase,
+                       c->tcap, c->cursor, A, c->mig, c->err_flag);
+    hipLaunchKernelGGL(k_resort_keys, grid, dim3(kBlock), 0, c->stream, r, c->pseg_blocks, c->pseg, c->pseg_n,
+                       c->dboxes, A, c->key, c->counts, c->err_flag, I);
+    hipLaunchKernelGGL(k_resort_scan, dim3(1), dim3(1024), 0, c->stream, r, c->tseg, c->tseg_n, c->dboxes, c->counts,
+                       c->ntiles_total, c->slack_num, c->slack_pad, c->tcap, c->tstart, c->tbase, c->cursor);
+    hipLaunchKernelGGL(k_resort_scatter, grid, dim3(kBlock), 0, c->stream, r, c->pseg_blocks, c->pseg, c->pseg_n,
+                       c->dboxes, c->key, c->tbase, c->cursor, A, I);
+    hipLaunchKernelGGL(k_resort_copy, grid, dim3(kBlock), 0, c->stream, r, c->part_cap, I, A);
+    LAUNCHCK(c);
+    return make_items(c, nullptr, r);
+}
+
 // Brings the particles into tile order for the deposit and the tile-staged
 // kicks: incrementally after a kick-drift that listed its tile changes, else by
 // a full counting sort into the other buffer (tiles with slack when slack_num > 0).
@@ -1330,8 +1359,8 @@ int phase_sort(nyxpm_ctx* c) {
     int rc;
     if (c->moves_pending) {
         c->moves_pending = false;
-        bool done = false;
-        if ((rc = phase_migrate(c, &done))) return rc;
+        bool done = c->capturing;
+        if ((rc = c->capturing ? captured_resort(c) : phase_migrate(c, &done))) return rc;
         if (done) {
             c->sorted_valid = true;
             c->keys_valid = false;
@@ -1372,6 +1401,9 @@ int phase_sort(nyxpm_ctx* c) {
     LAUNCHCK(c);
     c->cur = 1 - c->cur;
     c->holes = 0;
+    if (c->capturing)
+        hipLaunchKernelGGL(k_fill_dbl, dim3(1), dim3(kBlock), 0, c->stream, reinterpret_cast<double*>(c->resort), 1LL,
+                           0.0);
     ++c->n_full_sorts;
     if ((rc = make_items(c))) return rc;
     c->sorted_valid = true;
@@ -1914,7 +1946,7 @@ int phase_kick_g(nyxpm_ctx* c, double dt, double a_prev, double a_cur, double a_
         Timed t(c, MODE == kKickPair ? "kick_pair" : MOVE ? "kick_drift" : "kick");
         // incremental re-sort: the kick-drift lists the particles that change tile
         // (the list lives in the idle buffer's y array, like the deferred list in x)
-        const int inc = MOVE && c->slack_num > 0 && !c->inc_suspended ? 1 : 0;
+        const int inc = MOVE && c->slack_num > 0 ? 1 : 0;
         long long* moves = reinterpret_cast<long long*>(c->P[1 - c->cur].y);
         hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nmove, 4LL, 0);
         if (MOVE && !inc)
@@ -2246,6 +2278,8 @@ int nyxpm_destroy(nyxpm_ctx* c) {
     dfree(c->counts); dfree(c->cursor); dfree(c->tstart); dfree(c->bsum);
     dfree(c->tbase); dfree(c->tcap); dfree(c->mom_halo); dfree(c->mom_max); dfree(c->nmove); dfree(c->phi_prev); dfree(c->guess_ok);
     if (c->h_mig) hipHostFree(c->h_mig);
+    dfree(c->resort);
+    if (c->h_resort) hipHostFree(c->h_resort);
     c->rho = nullptr;
     dfree(c->own); dfree(c->halo); dfree(c->f); dfree(c->phi); dfree(c->partial);
 
@@ -3148,17 +3182,7 @@ int nyxpm_pm_steps(nyxpm_ctx* c, int nsteps, double dt, double a_old, double a_n
     // run as one particle pass (bit-identical to the separate kernels).
     const bool fused = !nyx_faithful && !c->separate_kicks;
     const double a_half = 0.5 * (a_old + a_new);
-    // a captured step cannot read back k_migrate's flags: full sorts throughout
-    struct Suspend {
-        nyxpm_ctx* c;
-        bool old;
-        ~Suspend() { c->inc_suspended = old; }
-    } suspend{c, c->inc_suspended};
-    if (use_graph) {
-        if (c->moves_pending && (rc = phase_sort(c))) return rc;
-        if ((rc = ensure_guess_buffer(c))) return rc;
-        c->inc_suspended = true;
-    }
+    if (use_graph && (rc = ensure_guess_buffer(c))) return rc;
     c->iters_seen = 0;
     if (fused && nsteps > 0 && (rc = phase_kick<kKickDrift>(c, dt, a_old, a_half))) return rc;
     auto one_step = [&](int s) -> int {
@@ -3198,11 +3222,15 @@ int nyxpm_pm_steps(nyxpm_ctx* c, int nsteps, double dt, double a_old, double a_n
             // their starting roles
             HIPCK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
             int cur0 = c->cur;
+            const long long holes0 = c->holes;
+            c->capturing = true;
             for (int r = 0; r < 2 && !rc; ++r)
                 rc = fused ? step_tail(c, dt, a_old, a_new, four_pi_G, rel_tol, abs_tol, cycles, a_old, a_new)
                            : step_body(c, dt, a_old, a_new, four_pi_G, rel_tol, abs_tol, nyx_faithful, cycles);
             hipGraph_t g = nullptr;
             hipError_t ee = hipStreamEndCapture(c->stream, &g);
+            c->capturing = false;
+            c->holes = holes0;
             c->timing = was_timing;
             if (rc) return rc;
             if (ee != hipSuccess) FAIL(c, NYXPM_ERR_HIP, "hipStreamEndCapture: %s", hipGetErrorString(ee));
@@ -3217,12 +3245,20 @@ int nyxpm_pm_steps(nyxpm_ctx* c, int nsteps, double dt, double a_old, double a_n
         }
         const int nbox = (int)c->boxes.size();
         hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->gstat, 2LL * nbox, 0);
+        hipLaunchKernelGGL(k_resort_state, dim3(1), dim3(1), 0, c->stream, c->resort, c->holes);
+        c->h_resort[0] = c->holes;
+        c->h_resort[1] = c->h_resort[2] = c->h_resort[3] = 0;
         HIPCK(c, hipGraphLaunch(c->gexec, c->stream));
         ++s;
         // every solve of the replay: a box still active after the recorded cycles
         // has not converged (the last solve's flags alone would hide an earlier one)
         HIPCK(c, hipMemcpyAsync(c->h_gstat, c->gstat, 2 * nbox * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-        if ((rc = solve_results(c, iters, nullptr, true))) return rc;
+        rc = solve_results(c, iters, nullptr, true);
+        c->holes = c->h_resort[0];
+        c->n_full_sorts += c->h_resort[1];
+        c->n_inc_sorts += c->h_resort[2];
+        c->n_moved += c->h_resort[3];
+        if (rc) return rc;
         for (int b = 0; b < nbox; ++b) {
             c->iters_seen = std::max(c->iters_seen, c->h_gstat[nbox + b]);
             if (c->h_gstat[b])

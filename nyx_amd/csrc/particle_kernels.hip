@@ -122,13 +122,15 @@ __device__ __forceinline__ int tile_of(const BoxDev& B, double x, double y, doub
 // binning: keys + counts, exclusive scan, scatter
 // ---------------------------------------------------------------------------
 
-__global__ void __launch_bounds__(kBlock) k_keys(const BoxSeg* segs, int nseg, const BoxDev* boxes,
-                                                 const double* __restrict__ x, const double* __restrict__ y,
-                                                 const double* __restrict__ z, int* __restrict__ key,
-                                                 int* counts, int* err) {
-    const BoxSeg sg = segs[find_seg(segs, nseg, blockIdx.x)];
+// Block blk's slots: keys and tile counts; empty_x (may be null): their x in the other
+// buffer emptied.
+__device__ __forceinline__ void keys_block(int blk, const BoxSeg* segs, int nseg, const BoxDev* boxes,
+                                           const double* __restrict__ x, const double* __restrict__ y,
+                                           const double* __restrict__ z, int* __restrict__ key, int* counts, int* err,
+                                           double* __restrict__ empty_x) {
+    const BoxSeg sg = segs[find_seg(segs, nseg, blk)];
     const BoxDev B = boxes[__builtin_amdgcn_readfirstlane(sg.box)];
-    const long long q = (long long)(blockIdx.x - sg.blk0) * kBlock + threadIdx.x;
+    const long long q = (long long)(blk - sg.blk0) * kBlock + threadIdx.x;
     bool valid = false;
     int t = 0;
     if (q < B.span) {
@@ -137,8 +139,16 @@ __global__ void __launch_bounds__(kBlock) k_keys(const BoxSeg* segs, int nseg, c
         valid = !isnan(px);  // NaN: an empty slot, keyed -1
         if (valid) t = tile_of(B, px, y[p], z[p], err);
         key[p] = valid ? t : -1;
+        if (empty_x) empty_x[p] = empty_slot();
     }
     agg_atomic_add(counts, t, valid);
+}
+
+__global__ void __launch_bounds__(kBlock) k_keys(const BoxSeg* segs, int nseg, const BoxDev* boxes,
+                                                 const double* __restrict__ x, const double* __restrict__ y,
+                                                 const double* __restrict__ z, int* __restrict__ key,
+                                                 int* counts, int* err) {
+    keys_block(blockIdx.x, segs, nseg, boxes, x, y, z, key, counts, err, nullptr);
 }
 
 // Slot capacity of each tile for a sort with slack: cnt + floor(cnt * num / 1024)
@@ -249,15 +259,14 @@ struct PartPtrs {
     size_t bytes;
 };
 
-// Move every particle to its tile's slot range (order inside a tile is
+// Move block blk's particles to their tiles' slot ranges (order inside a tile is
 // arbitrary); cursor[t] ends as the tile's particle count.
-__global__ void __launch_bounds__(kBlock) k_scatter(const BoxSeg* segs, int nseg, const BoxDev* boxes,
-                                                    const int* __restrict__ key,
-                                                    const long long* __restrict__ tbase, int* cursor,
-                                                    PartPtrs src, PartPtrs dst) {
-    const BoxSeg sg = segs[find_seg(segs, nseg, blockIdx.x)];
+__device__ __forceinline__ void scatter_block(int blk, const BoxSeg* segs, int nseg, const BoxDev* boxes,
+                                              const int* __restrict__ key, const long long* __restrict__ tbase,
+                                              int* cursor, const PartPtrs& src, const PartPtrs& dst) {
+    const BoxSeg sg = segs[find_seg(segs, nseg, blk)];
     const BoxDev B = boxes[__builtin_amdgcn_readfirstlane(sg.box)];
-    const long long q = (long long)(blockIdx.x - sg.blk0) * kBlock + threadIdx.x;
+    const long long q = (long long)(blk - sg.blk0) * kBlock + threadIdx.x;
     const long long p = B.part_off + q;
     // occupied slots only (a kick-drift keys the slots it visits, not the free ones)
     bool valid = false;
@@ -279,6 +288,106 @@ __global__ void __launch_bounds__(kBlock) k_scatter(const BoxSeg* segs, int nseg
         if (src.m) dst.m[d] = src.m[p];
         dst.id[d] = src.id[p];
     }
+}
+
+__global__ void __launch_bounds__(kBlock) k_scatter(const BoxSeg* segs, int nseg, const BoxDev* boxes,
+                                                    const int* __restrict__ key,
+                                                    const long long* __restrict__ tbase, int* cursor,
+                                                    PartPtrs src, PartPtrs dst) {
+    scatter_block(blockIdx.x, segs, nseg, boxes, key, tbase, cursor, src, dst);
+}
+
+// The full sort of a captured step, decided on the device: a replay cannot read
+// k_migrate's flags back, so it records the incremental re-sort and behind it these
+// kernels, which do nothing unless a tile ran out of slack or the emptied slots pass
+// their limit.  They sort into the idle buffer and copy back (the buffers' roles are
+// baked into the recorded launches).  Few, persistent blocks: skipped, the four cost ~2 us
+// each; a full sort per captured step took 1.6 ms for 5.2 10^7 particles.
+struct Resort {
+    const int* mig;    // of k_migrate: overflow, particles moved
+    long long* state;  // [0] emptied slots, [1] full sorts, [2] incremental ones, [3] particles moved
+    long long np;      // particles and the share (of 1024) of emptied slots that asks for a full sort
+    int hole_num;
+};
+__device__ __forceinline__ bool resort_full(const Resort& r) {
+    return r.mig[0] != 0 || (r.state[0] + r.mig[1]) * 1024 > r.np * r.hole_num;
+}
+
+__global__ void __launch_bounds__(kBlock) k_resort_keys(Resort r, int nblk, const BoxSeg* segs, int nseg,
+                                                        const BoxDev* boxes, PartPtrs A, int* __restrict__ key,
+                                                        int* counts, int* err, PartPtrs idle) {
+    if (!resort_full(r)) return;
+    for (int b = blockIdx.x; b < nblk; b += gridDim.x)
+        keys_block(b, segs, nseg, boxes, A.x, A.y, A.z, key, counts, err, idle.x);
+}
+
+// Capacities, slot ranges (per box from its first slot) and empty cursors of all tiles,
+// one block.
+__global__ void __launch_bounds__(1024) k_resort_scan(Resort r, const BoxSeg* tsegs, int ntseg, const BoxDev* boxes,
+                                                      const int* __restrict__ counts, long long ntiles, int num,
+                                                      int pad, int* __restrict__ cap, long long* start,
+                                                      long long* __restrict__ tbase, int* __restrict__ cursor) {
+    if (!resort_full(r)) return;
+    __shared__ long long sh[1024];
+    long long carry = 0;
+    for (long long base = 0; base < ntiles; base += 1024) {
+        const long long t = base + threadIdx.x;
+        long long v = 0;
+        if (t < ntiles) {
+            const long long c = counts[t];
+            v = c + ((c * num) >> 10) + pad;
+            cap[t] = (int)v;
+            cursor[t] = 0;
+        }
+        sh[threadIdx.x] = v;
+        __syncthreads();
+        for (int o = 1; o < 1024; o <<= 1) {
+            const long long u = (int)threadIdx.x >= o ? sh[threadIdx.x - o] : 0;
+            __syncthreads();
+            sh[threadIdx.x] += u;
+            __syncthreads();
+        }
+        if (t < ntiles) start[t] = carry + sh[threadIdx.x] - v;
+        carry += sh[1023];
+        __syncthreads();
+    }
+    __threadfence_block();
+    __syncthreads();
+    for (long long t = threadIdx.x; t < ntiles; t += 1024) {
+        const BoxDev& B = boxes[tsegs[find_seg(tsegs, ntseg, (int)t)].box];
+        tbase[t] = start[t] - start[B.tile_off] + B.part_off;
+    }
+}
+
+__global__ void __launch_bounds__(kBlock) k_resort_scatter(Resort r, int nblk, const BoxSeg* segs, int nseg,
+                                                           const BoxDev* boxes, const int* __restrict__ key,
+                                                           const long long* __restrict__ tbase, int* cursor,
+                                                           PartPtrs src, PartPtrs dst) {
+    if (!resort_full(r)) return;
+    for (int b = blockIdx.x; b < nblk; b += gridDim.x)
+        scatter_block(b, segs, nseg, boxes, key, tbase, cursor, src, dst);
+}
+
+__global__ void __launch_bounds__(kBlock) k_resort_copy(Resort r, long long slots, PartPtrs src, PartPtrs dst) {
+    if (!resort_full(r)) return;
+    for (long long p = (long long)blockIdx.x * kBlock + threadIdx.x; p < slots; p += (long long)gridDim.x * kBlock) {
+        const double px = src.x[p];
+        dst.x[p] = px;
+        if (isnan(px)) continue;  // an empty slot
+        dst.y[p] = src.y[p];
+        dst.z[p] = src.z[p];
+        dst.vx[p] = src.vx[p];
+        dst.vy[p] = src.vy[p];
+        dst.vz[p] = src.vz[p];
+        if (src.m) dst.m[p] = src.m[p];
+        dst.id[p] = src.id[p];
+    }
+}
+
+// The state a replay starts from.
+__global__ void k_resort_state(long long* state, long long holes) {
+    state[0] = holes;
+    state[1] = state[2] = state[3] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1021,10 +1130,21 @@ __global__ void __launch_bounds__(kBlock) k_make_items(const long long* __restri
                                                        TileItem* __restrict__ items, int* nitems, int chunk,
                                                        HeavyItem* __restrict__ heavy, int* nheavy, int* nsplit,
                                                        long long split_min, int split_part, int split_cap,
-                                                       const int* mig, int* h_mig) {
+                                                       const int* mig, int* h_mig, Resort resort,
+                                                       long long* h_resort) {
     const long long t = (long long)blockIdx.x * kBlock + threadIdx.x;
-    // the migration's flags to the host's mirror (pinned memory) along the way
+    // the migration's flags to the host's mirror (pinned memory) along the way, or in a
+    // captured step the outcome of the re-sort
     if (mig && t < 2) __hip_atomic_store(&h_mig[t], mig[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    if (resort.state && t == 0) {
+        long long* st = resort.state;
+        const bool full = resort_full(resort);
+        st[0] = full ? 0 : st[0] + resort.mig[1];
+        st[full ? 1 : 2] += 1;
+        st[3] += resort.mig[1];
+        for (int q = 0; q < 4; ++q)
+            __hip_atomic_store(&h_resort[q], st[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
     int nc = 0;
     long long p0 = 0, cnt = 0;
     if (t < ntiles) {

@@ -259,3 +259,38 @@ def test_tiled_gather_equals_thread_per_particle(nyx, npart, precision):
         assert np.array_equal(c.gather_accel(), unbinned())
         if npart <= 2 ** 20:
             assert np.array_equal(c.gather_accel_noalloc(), unbinned())
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("slack,speed", [(0.25, 0.02), (0.002, 1.0), (0.5, 6.0)])
+def test_captured_resort_equals_eager(nyx, precision, slack, speed):
+    # captured steps re-sort incrementally and decide on the device about the full sort
+    # (few particles moving; tiles that run out of slack; emptied slots past their
+    # limit), over several replays and calls with eager steps between them, against
+    # eager steps bit for bit, with per-particle masses, and with what the host counts
+    r = np.random.default_rng(91)
+    sizes, npart = [(32, 32, 32), (24, 24, 24)], 20000
+    parts = [([r.random(npart) for _ in range(3)], [speed * 0.3 * r.standard_normal(npart) for _ in range(3)],
+              0.5 / npart + r.random(npart) / npart) for _ in sizes]
+    res = []
+    for graph in (False, True):
+        with nyx.PMContext([nyx.BoxGeom(n) for n in sizes], precision=precision, resort_slack=slack) as c:
+            for b, (pos, vel, m) in enumerate(parts):
+                c.upload(b, pos, vel, m=m)
+            c.pm_init()
+            states = []
+            for nsteps in (8, 5, 10):
+                c.pm_steps(nsteps, 1e-3, use_graph=graph)
+                for b in range(2):
+                    p, v = c.download(b)
+                    states += list(p) + list(v) + [c.get_phi(b)]
+            st = c.sort_stats()
+            res.append(states)
+            print("sorts", graph, st, flush=True)
+            if speed < 0.1:
+                assert st["full"] == 1 and st["incremental"] == 23 and st["moved"] > 0
+            else:
+                assert st["full"] > 3
+                assert speed > 2 or st["incremental"] > 3
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
