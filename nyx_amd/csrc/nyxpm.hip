@@ -312,6 +312,7 @@ struct nyxpm_ctx {
     std::vector<int> fin_buf;    // buffer holding e after post-smoothing, per depth
     Table t_bottom, t_l0, t_res;  // t_res: level 0, at most kReduceBlocks blocks per box
     Table t_fold;                 // k_fold's blocks, each one or more of t_res's
+    bool fold_shares = false;     // more than one for some piece
     // one-workgroup coarse V-cycle: per box, levels dc..nlev-1 (cc_first[b] ..
     // cc_first[b+1]-1 of table t_cc) and the LDS it needs per precision
     Table t_cc;
@@ -954,14 +955,19 @@ int build_tables(nyxpm_ctx* c) {
         int rzc = 64;
         while (res_pieces(rzc) < 512 && rzc > 4) rzc /= 2;
         c->t_res = add_table(vr);
-        // k_fold: kFoldU of t_res's blocks each where those have one cell per thread
+        // k_fold: kFoldU of t_res's blocks each where those have one cell per thread and
+        // leave four blocks per CU (us, one share -> four: 64^3 alone 7.3 -> 9.6, 112x96x144
+        // 18.6 -> 15.8)
+        const bool many = c->t_res.blocks >= 1024 * kFoldU;
         std::vector<CellSeg> vf;
+        c->fold_shares = false;
         for (int b = 0; b < nbox; ++b) {
             CellSeg s = S[c->t_res.first + b];
             s.coff = s.blk0;
             s.ebuf = s.nblk;
-            s.zchunk = (c->boxes[b].lev[0].nc + s.nblk - 1) / s.nblk <= kBlock ? kFoldU : 1;
+            s.zchunk = many && (c->boxes[b].lev[0].nc + s.nblk - 1) / s.nblk <= kBlock ? kFoldU : 1;
             s.nblk = (s.nblk + s.zchunk - 1) / s.zchunk;
+            c->fold_shares |= s.zchunk > 1;
             vf.push_back(s);
         }
         c->t_fold = add_table(vf);
@@ -1254,11 +1260,10 @@ int alloc_items(nyxpm_ctx* c, long long slots, ItemTables* t) {
     t->chunk = choose_chunk(c, slots);
     t->items_cap = c->ntiles_total + slots / t->chunk + 1;
     if (t->items_cap > 0x7fffffffLL) FAIL(c, NYXPM_ERR_ARG, "too many tile chunks");
-    // a heavy tile's whole block stands for more than kHeavyTile slots, a part of a
-    // split one for at least 2/3 kSplitPart on average (three parts from 4097 slots,
-    // at least 4/5 of a longer part from four times its length)
-    t->heavy_cap = slots / (kSplitPart * 2 / 3) + 1;
+    // a heavy tile's whole block stands for more than kHeavyTile slots, and so does a
+    // part of a split one but for the tile's last
     t->split_cap = std::min<long long>(kSplitShare, slots / kSplitTile);
+    t->heavy_cap = slots / kHeavyTile + t->split_cap + 1;
     // (three accumulators per split tile: the momentum deposit's components)
     const size_t words = (size_t)t->split_cap * 3 * split_words(c);
     int rc = dalloc(c, &t->items, t->items_cap);
@@ -1429,13 +1434,10 @@ int phase_deposit(nyxpm_ctx* c, bool want_rho, bool f32 = false) {
     }
     {
         Timed t(c, "fold");
-        if (want_rho)
-            hipLaunchKernelGGL(k_fold<true>, dim3(c->t_fold.blocks), dim3(kBlock), 0, c->stream, c->segs(c->t_fold),
-                               c->t_fold.count, c->dboxes, c->own, c->halo, c->rho, c->f, c->partial);
-        else
-            hipLaunchKernelGGL(k_fold<false>, dim3(c->t_fold.blocks), dim3(kBlock), 0, c->stream,
-                               c->segs(c->t_fold), c->t_fold.count, c->dboxes, c->own, c->halo, c->rho, c->f,
-                               c->partial);
+        auto fold = c->fold_shares ? (want_rho ? k_fold<true, true> : k_fold<false, true>)
+                                   : (want_rho ? k_fold<true, false> : k_fold<false, false>);
+        hipLaunchKernelGGL(fold, dim3(c->t_fold.blocks), dim3(kBlock), 0, c->stream, c->segs(c->t_fold),
+                           c->t_fold.count, c->dboxes, c->own, c->halo, c->rho, c->f, c->partial);
     }
     LAUNCHCK(c);
     c->density_valid = want_rho;
