@@ -82,15 +82,14 @@ __device__ __forceinline__ double empty_slot() { return __longlong_as_double(0x7
 // Slots above which a tile's deposit block is launched ahead of the others.
 constexpr int kHeavyTile = 2048;
 // A tile with more than kSplitTile slots and more than 1/kSplitShare of all particles
-// (so about kSplitShare tiles at most) is deposited by several blocks, which add their
-// fixed-point sums in global memory: one block takes ~3.7 ns a slot, the whole chip
-// ~17 ps, so such a tile alone holds the launch for about as long as everything else
-// (131 us for a clump of 35000 in 10^6 particles).  Below that share the blocks of the
-// other tiles hide it, and the parts' additions (2754 64-bit atomics each, ~30 per ns)
-// cost more than they save; parts of at least kSplitPart slots and 1/kSplitParts of
-// all particles keep them to ~100 us at the most.  At 2 10^7 particles, splitting the
-// tiles above 1/1024 into parts of 2048 took 900 us, none 340 us.
-constexpr int kSplitTile = 4096, kSplitPart = 2048, kSplitShare = 256, kSplitParts = 1024;
+// is deposited by several blocks, which add their fixed-point sums in global memory: a
+// CU holds seven blocks of 16x8x8 tiles, so one with more than 1/1792 of the work
+// outlasts the others.  Parts of at least kSplitPart slots and 1/kSplitParts of all
+// particles: the additions are at most 2754 64-bit atomics a part, ~30 per ns in all.
+// 1/256 and 1/1024 -> 1/2048 and 1/2048, us: 128^3 with 2 10^6 clustered particles,
+// density and velocities, 250 -> 236; 256^3 with 2 10^7, density, 465 -> 382 (parts of
+// 1/4096 and tiles above 1/4096 the same within 2%).
+constexpr int kSplitTile = 4096, kSplitPart = 2048, kSplitShare = 2048, kSplitParts = 2048;
 
 // One block of the deposit ahead of the ordinary tiles: `len` slots from `off` of a
 // heavy tile, one of nparts pieces (1: the whole tile); split: the tile's accumulator.
@@ -420,20 +419,33 @@ __device__ __forceinline__ unsigned fx32_units(float w, float scale) {
 // The parts of a split tile: adds the block's LDS words to the tile's accumulator
 // (integers: exact in any order); the last part to arrive takes the sums back into
 // LDS, leaving the accumulator and its counter at zero for the next deposit, and
-// returns true.
+// returns true.  Everything shared between the parts is touched by device-scope atomics
+// alone, which are performed where all XCDs see them: a part waits for its additions to
+// be performed, then arrives.  (A fence instead of the wait writes back the XCD's whole
+// L2 for each part: with it 128^3 with 2 10^6 clustered particles took 121 us instead of
+// 43, the three momenta 376 instead of 86, 10^6 in 112x96x144 FP32 66 instead of 19.)
 __device__ __forceinline__ bool split_combine(unsigned long long* acc, int words, const HeavyItem& hv,
                                               unsigned long long* split_acc, int split_words, int* split_done) {
     __shared__ int s_last;
     unsigned long long* g = split_acc + (size_t)hv.split * split_words;
-    for (int c = threadIdx.x; c < words; c += blockDim.x)
+    for (int c = threadIdx.x; c < words; c += kBlock)
         if (acc[c]) atomicAdd(&g[c], acc[c]);
-    __threadfence();  // every addition before the arrival
+    __builtin_amdgcn_s_waitcnt(0);  // every addition before the arrival
     __syncthreads();
     if (threadIdx.x == 0) s_last = atomicAdd(&split_done[hv.split], 1) == hv.nparts - 1;
     __syncthreads();
     if (!s_last) return false;
-    __threadfence();
-    for (int c = threadIdx.x; c < words; c += blockDim.x) acc[c] = atomicExch(&g[c], 0ull);
+    // several exchanges in flight per thread: each is a round trip past the L2
+    constexpr int U = 6;
+    for (int c0 = threadIdx.x; c0 < words; c0 += U * kBlock) {
+        unsigned long long v[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (c0 + u * kBlock < words) v[u] = atomicExch(&g[c0 + u * kBlock], 0ull);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (c0 + u * kBlock < words) acc[c0 + u * kBlock] = v[u];
+    }
     if (threadIdx.x == 0) atomicExch(&split_done[hv.split], 0);
     __syncthreads();
     return true;
