@@ -1829,20 +1829,27 @@ __global__ void __launch_bounds__(kBlock) k_update0(const CellSeg* segs, int nse
 // One wave per box: its lanes take the norm slots (one lane reading them in turn
 // was a chain of 64 loads, 5 us a launch).  The box's flags and state also go to the
 // host's mirror (pinned memory), so that reading them takes a wait for the stream and
-// no copies (a copy is a launch of its own, 3-4 us and its gap; a step read five).
+// no copies (a copy is a launch of its own, 3-4 us and its gap; a step read five), but
+// only when the host is about to look (`mirror`) or the box has stopped: the launch ends
+// with its stores' way across the bus.  Everything is loaded before anything is decided,
+// one round trip to memory.
 __global__ void __launch_bounds__(kWave) k_check(int init, int fixed_iters, int max_iter, double rel_tol,
                                                  double abs_tol, int* active, int* iters, int* failed,
                                                  unsigned long long* nr, unsigned long long* nf, double* state,
-                                                 int inc, int nbox, int* h_flags, double* h_state) {
+                                                 int inc, int nbox, int mirror, int* h_flags, double* h_state) {
     static_assert(kNormSlots == kWave, "one lane per norm slot");
     const int b = blockIdx.x;
     const int slot = b * kNormSlots + threadIdx.x;
-    unsigned long long br = nr[slot], bf = nf[slot];
+    unsigned long long br = nr[slot], bf = init ? nf[slot] : 0ull;
+    int act = active[b], it = iters[b], fail = failed[b];
+    double st[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) st[q] = state[4 * b + q];
     nr[slot] = 0ull;
-    nf[slot] = 0ull;
+    if (init) nf[slot] = 0ull;
     for (int o = kWave / 2; o > 0; o >>= 1) {
         br = max(br, (unsigned long long)__shfl_xor((long long)br, o));
-        bf = max(bf, (unsigned long long)__shfl_xor((long long)bf, o));
+        if (init) bf = max(bf, (unsigned long long)__shfl_xor((long long)bf, o));
     }
     if (threadIdx.x != 0) return;
     if (init) {
@@ -1852,31 +1859,36 @@ __global__ void __launch_bounds__(kWave) k_check(int init, int fixed_iters, int 
         const double rt = rel_tol > 1e-16 ? rel_tol : 1e-16;
         double target = rt * mx;
         if (abs_tol > target) target = abs_tol;
-        state[4 * b + 0] = r0;
-        state[4 * b + 1] = fn;
-        state[4 * b + 2] = r0;
-        state[4 * b + 3] = target;
-        iters[b] = 0;
-        failed[b] = 0;
-        active[b] = fixed_iters > 0 ? 1 : (r0 > target ? 1 : 0);
-    } else if (active[b]) {
+        st[0] = r0;
+        st[1] = fn;
+        st[2] = r0;
+        st[3] = target;
+        it = 0;
+        fail = 0;
+        act = fixed_iters > 0 ? 1 : (r0 > target ? 1 : 0);
+    } else if (act) {
         const double rn = __longlong_as_double((long long)br);
-        const int it = iters[b] + inc;  // the V-cycles run since the last check
-        iters[b] = it;
-        state[4 * b + 2] = rn;
+        it += inc;  // the V-cycles run since the last check
+        st[2] = rn;
         if (fixed_iters > 0) {
-            active[b] = it < fixed_iters ? 1 : 0;
+            act = it < fixed_iters ? 1 : 0;
         } else {
-            const int more = rn > state[4 * b + 3];
-            active[b] = (more && it < max_iter) ? 1 : 0;
-            failed[b] = (more && it >= max_iter) ? 1 : 0;
+            const int more = rn > st[3];
+            act = (more && it < max_iter) ? 1 : 0;
+            fail = (more && it >= max_iter) ? 1 : 0;
         }
     }
+    active[b] = act;
+    iters[b] = it;
+    failed[b] = fail;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) state[4 * b + q] = st[q];
+    if (!mirror && act) return;
     auto put = [](auto* p, auto v) { __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM); };
-    put(&h_flags[b], active[b]);
-    put(&h_flags[nbox + b], iters[b]);
-    put(&h_flags[2 * nbox + b], failed[b]);
-    for (int q = 0; q < 4; ++q) put(&h_state[4 * b + q], state[4 * b + q]);
+    put(&h_flags[b], act);
+    put(&h_flags[nbox + b], it);
+    put(&h_flags[2 * nbox + b], fail);
+    for (int q = 0; q < 4; ++q) put(&h_state[4 * b + q], st[q]);
 }
 
 // After the recorded V-cycles of a captured solve: a box still active has not

@@ -167,6 +167,7 @@ struct nyxpm_ctx {
     // first FP64 residual check (the correction carried over, phi updated once)
     int ir_first = kIrFirstDefault;
     int iters_seen = 0;  // most V-cycles of a box in the solves of the current call
+    int cycles_last = 0; // most V-cycles of a box in the last solve
     bool no_fused = false;  // force half-sweep smoothing (for comparisons)
     bool untiled_kick = false;  // force the thread-per-particle kick (for comparisons)
     bool separate_kicks = false;  // nyxpm_pm_steps without the kick / kick-drift pairing
@@ -1802,12 +1803,13 @@ int update(nyxpm_ctx* c) {
     return NYXPM_OK;
 }
 
-// inc: the V-cycles run since the previous check (added to the per-box count)
-int check(nyxpm_ctx* c, bool init, int fixed_iters, double rel, double abs_tol, int inc = 1) {
+// inc: the V-cycles run since the previous check (added to the per-box count); look: the
+// host reads the flags before the next check
+int check(nyxpm_ctx* c, bool init, int fixed_iters, double rel, double abs_tol, int inc, bool look) {
     const int nbox = (int)c->boxes.size();
     hipLaunchKernelGGL(k_check, dim3(nbox), dim3(kWave), 0, c->stream, init ? 1 : 0, fixed_iters, c->max_iter, rel,
                        abs_tol, c->active, c->iters, c->failed, c->nr, c->nf, c->state, inc, nbox,
-                       c->hd_flags, c->hd_state);
+                       look ? 1 : 0, c->hd_flags, c->hd_state);
     LAUNCHCK(c);
     return NYXPM_OK;
 }
@@ -1858,13 +1860,13 @@ int solve_impl(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int gr
     const int g0 = first_group<T>(c, fixed_iters);
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->active, (long long)nbox, 1);
     if ((rc = res(true))) return rc;
-    if ((rc = check(c, true, fixed_iters, rel, abs_tol))) return rc;
     if (graph_cycles > 0) {
+        if ((rc = check(c, true, fixed_iters, rel, abs_tol, 0, false))) return rc;
         // the same schedule as eagerly, graph_cycles V-cycles in all
         for (int done = 0, g = std::min(g0, graph_cycles); done < graph_cycles; done += g, g = 1) {
             if ((rc = vcycle_group<T>(c, g, rs))) return rc;
             if ((rc = res(false))) return rc;
-            if ((rc = check(c, false, fixed_iters, rel, abs_tol, g))) return rc;
+            if ((rc = check(c, false, fixed_iters, rel, abs_tol, g, done + g >= graph_cycles))) return rc;
         }
         // a box still active now did not converge within the recorded cycles:
         // kept in gstat, which the next solve of the replay does not reset
@@ -1874,14 +1876,27 @@ int solve_impl(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int gr
         return NYXPM_OK;
     }
     const int limit = fixed_iters > 0 ? fixed_iters : c->max_iter;
+    // V-cycles issued before the host first waits for a check.  A wait empties the
+    // stream: 10-15 us until the next cycle's first kernel, of ~45 us a cycle at 32^3.
+    // The previous solve's count less one: solves of one program differ little, and a
+    // cycle too many, with every box stopped, still costs its launches (~25 us).
+    const int ahead = fixed_iters > 0 ? fixed_iters : std::min(c->cycles_last - 1, limit);
+    auto look = [&](int it, int g) { return it + g > ahead; };
+    if ((rc = check(c, true, fixed_iters, rel, abs_tol, 0, look(0, g0)))) return rc;
     for (int it = 0, g = g0; it <= limit; it += g, g = 1) {
-        bool any;
-        if ((rc = read_flags(c, &any))) return rc;
-        c->results_ready = !any;
-        if (!any) break;
+        if (look(it, g)) {
+            bool any;
+            if ((rc = read_flags(c, &any))) return rc;
+            c->results_ready = !any;
+            if (!any) break;
+        }
         if ((rc = vcycle_group<T>(c, g, rs))) return rc;
         if ((rc = res(false))) return rc;
-        if ((rc = check(c, false, fixed_iters, rel, abs_tol, g))) return rc;
+        if ((rc = check(c, false, fixed_iters, rel, abs_tol, g, look(it + g, 1)))) return rc;
+    }
+    if (c->results_ready && fixed_iters == 0) {
+        c->cycles_last = 0;
+        for (int b = 0; b < nbox; ++b) c->cycles_last = std::max(c->cycles_last, c->h_flags[nbox + b]);
     }
     return NYXPM_OK;
 }

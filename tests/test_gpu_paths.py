@@ -294,3 +294,38 @@ def test_captured_resort_equals_eager(nyx, precision, slack, speed):
                 assert speed > 2 or st["incremental"] > 3
     for a, b in zip(*res):
         assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_cycles_issued_ahead(nyx, precision):
+    # V-cycles issued before the host looks at a check (one fewer than the last solve
+    # took): solves that need fewer, none, more or a fixed number of cycles than the one
+    # before give the bits, counts and norms of a context that has solved nothing else
+    n = (40, 24, 32)
+    f = mean_free(n, 91)
+    hard = dict(rel_tol=1e-12)
+    def runs(c, phi):
+        return [lambda: c.solve_poisson(f, **hard), lambda: c.solve_poisson(f, rel_tol=1e-3),
+                lambda: c.solve_poisson(f, phi, rel_tol=1e-6), lambda: c.solve_poisson(f, **hard),
+                lambda: c.solve_poisson(f, fixed_iters=3), lambda: c.solve_poisson(0 * f),
+                lambda: c.solve_poisson(f, phi, **hard)]
+    with ctx1(nyx, n, precision=precision) as c:
+        phi = c.solve_poisson(f, **hard)[0]
+        together = [g() for g in runs(c, phi)]
+    for i, (p, it, norms) in enumerate(together):
+        with ctx1(nyx, n, precision=precision) as c:
+            p1, it1, norms1 = runs(c, phi)[i]()
+        assert it == it1 and np.array_equal(norms, norms1) and np.array_equal(p, p1)
+    assert together[2][1] == together[5][1] == 0 and together[4][1] == 3
+
+
+def test_cycles_issued_ahead_up_to_the_limit(nyx):
+    # ... and a solve that runs into max_iter raises with its count, whatever was issued
+    n = (32, 32, 32)
+    f = mean_free(n, 92)
+    with ctx1(nyx, n, max_iter=4) as c:
+        assert c.solve_poisson(f, rel_tol=1e-2)[1] <= 4
+        for _ in range(2):
+            with pytest.raises(nyx.NyxPMError, match="after 4 cycles"):
+                c.solve_poisson(f, rel_tol=1e-14)
+        assert c.solve_poisson(f, rel_tol=1e-2)[1] <= 4
