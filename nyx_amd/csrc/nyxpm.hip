@@ -264,12 +264,13 @@ struct nyxpm_ctx {
     float *r32 = nullptr, *e32 = nullptr, *e32b = nullptr;
     double* G64 = nullptr;  // bottom Green's functions (FP64 in both precisions)
     // per-box device state
-    int *active = nullptr, *iters = nullptr, *failed = nullptr, *err_flag = nullptr;
+    int *active = nullptr, *iters = nullptr, *failed = nullptr;
+    int* err_flag = nullptr;  // kErrFlags words behind hd_flags' per-box ones (raise_err)
     unsigned long long *nr = nullptr, *nf = nullptr;
     double *state = nullptr, *solv = nullptr, *dv_size = nullptr;
     BoxDev* dboxes = nullptr;
     // host mirror of per-box flags and state (pinned), written by k_check
-    int* h_flags = nullptr;  // active[nbox] iters[nbox] failed[nbox] err
+    int* h_flags = nullptr;  // active[nbox] iters[nbox] failed[nbox] errors[kErrFlags]
     double* h_state = nullptr;
     int* hd_flags = nullptr;     // their device addresses
     double* hd_state = nullptr;
@@ -1116,7 +1117,6 @@ int alloc_fields(nyxpm_ctx* c) {
     if ((rc = dalloc(c, &c->active, nbox))) return rc;
     if ((rc = dalloc(c, &c->iters, nbox))) return rc;
     if ((rc = dalloc(c, &c->failed, nbox))) return rc;
-    if ((rc = dalloc(c, &c->err_flag, 1))) return rc;
     if ((rc = dalloc(c, &c->nitems, 3))) return rc;
     c->nheavy = c->nitems + 1;
     c->nsplit = c->nitems + 2;
@@ -1131,15 +1131,16 @@ int alloc_fields(nyxpm_ctx* c) {
     if ((rc = dalloc(c, &c->dboxes, nbox))) return rc;
     if ((rc = dalloc(c, &c->gstat, 2 * nbox))) return rc;
     HIPCK(c, hipHostMalloc((void**)&c->h_gstat, 2 * nbox * sizeof(int), hipHostMallocDefault));
-    HIPCK(c, hipHostMalloc((void**)&c->h_flags, (3 * nbox + 1) * sizeof(int), hipHostMallocDefault));
+    HIPCK(c, hipHostMalloc((void**)&c->h_flags, (3 * nbox + kErrFlags) * sizeof(int), hipHostMallocDefault));
     HIPCK(c, hipHostMalloc((void**)&c->h_state, 4 * nbox * sizeof(double), hipHostMallocDefault));
     HIPCK(c, hipHostGetDevicePointer((void**)&c->hd_flags, c->h_flags, 0));
     HIPCK(c, hipHostGetDevicePointer((void**)&c->hd_state, c->h_state, 0));
+    c->err_flag = c->hd_flags + 3 * nbox;
+    std::fill_n(c->h_flags + 3 * nbox, kErrFlags, 0);
     HIPCK(c, hipHostGetDevicePointer((void**)&c->hd_mig, c->h_mig, 0));
     HIPCK(c, hipMemset(c->phi, 0, c->ncell_total * sizeof(double)));
     HIPCK(c, hipMemset(c->nr, 0, (size_t)nbox * kNormSlots * sizeof(unsigned long long)));
     HIPCK(c, hipMemset(c->nf, 0, (size_t)nbox * kNormSlots * sizeof(unsigned long long)));
-    HIPCK(c, hipMemset(c->err_flag, 0, sizeof(int)));
     // bottom Green's functions
     std::vector<double> G(c->G_total);
     for (auto& B : c->boxes) {
@@ -1199,13 +1200,14 @@ int ensure_idle_buffer(nyxpm_ctx* c) {
 
 // Waits for the stream and reports the kernels' error flags.
 int err_check(nyxpm_ctx* c) {
-    int* e = c->h_flags + 3 * c->boxes.size();
-    HIPCK(c, hipMemcpyAsync(e, c->err_flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
     HIPCK(c, hipStreamSynchronize(c->stream));
-    if (*e) {
-        hipMemsetAsync(c->err_flag, 0, sizeof(int), c->stream);
+    int* e = c->h_flags + 3 * c->boxes.size();
+    int flags = 0;
+    for (int i = 0; i < kErrFlags; ++i) flags |= e[i] ? 1 << i : 0;
+    if (flags) {
+        std::fill_n(e, kErrFlags, 0);
         FAIL(c, NYXPM_ERR_STATE,
-             "particle outside one periodic image of its box or binning inconsistent (flags 0x%x)", *e);
+             "particle outside one periodic image of its box or binning inconsistent (flags 0x%x)", flags);
     }
     return NYXPM_OK;
 }
@@ -2302,7 +2304,7 @@ int nyxpm_destroy(nyxpm_ctx* c) {
 
     dfree(c->r64); dfree(c->e64); dfree(c->e64b); dfree(c->G64);
     dfree(c->r32); dfree(c->e32); dfree(c->e32b);
-    dfree(c->active); dfree(c->iters); dfree(c->failed); dfree(c->err_flag); dfree(c->nitems); dfree(c->nr); dfree(c->nf);
+    dfree(c->active); dfree(c->iters); dfree(c->failed); dfree(c->nitems); dfree(c->nr); dfree(c->nf);
     dfree(c->dtmin);
     dfree(c->state); dfree(c->solv); dfree(c->dv_size); dfree(c->dboxes);
     dfree(c->seg_pool); dfree(c->pseg); dfree(c->tseg); dfree(c->cc_first);

@@ -31,9 +31,17 @@ __device__ __forceinline__ int cic_index(double x, double plo, double dxi, doubl
     return i;
 }
 
+// Error flags 1, 2, 4, 8: a word each in pinned host memory, set by plain stores (rarely
+// any), so that the host reads them behind its wait for the stream without a copy.
+constexpr int kErrFlags = 4;
+__device__ __forceinline__ void raise_err(int* err, int flags) {
+    for (int i = 0; i < kErrFlags; ++i)
+        if (flags >> i & 1) __hip_atomic_store(&err[i], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Wrap an index known to lie within one period of [0, n); flags anything else.
 __device__ __forceinline__ int wrap_checked(int i, int n, int* err) {
-    if (i < -n || i >= 2 * n) { if (err) atomicOr(err, 1); }
+    if (i < -n || i >= 2 * n) { if (err) raise_err(err, 1); }
     return wrap1(i, n);
 }
 
@@ -111,7 +119,7 @@ __device__ __forceinline__ int tile_of(const BoxDev& B, double x, double y, doub
     // an index more than one period out: one flag branch for the three (rare)
     if ((unsigned)(ci + B.n[0]) >= (unsigned)(3 * B.n[0]) || (unsigned)(cj + B.n[1]) >= (unsigned)(3 * B.n[1]) ||
         (unsigned)(ck + B.n[2]) >= (unsigned)(3 * B.n[2]))
-        atomicOr(err, 1);
+        raise_err(err, 1);
     const int i = wrap1(ci, B.n[0]), j = wrap1(cj, B.n[1]), k = wrap1(ck, B.n[2]);
     const int tx = tile_div(i, B.tdiv[0]), ty = tile_div(j, B.tdiv[1]), tz = tile_div(k, B.tdiv[2]);
     return (int)(B.tile_off + ((long long)tz * B.ntile[1] + ty) * B.ntile[0] + tx);
@@ -569,7 +577,7 @@ __global__ void __launch_bounds__(kBlock) k_deposit(const BoxSeg* segs, int nseg
         const bool outside = (unsigned)iw >= (unsigned)bx || (unsigned)jw >= (unsigned)by ||
                              (unsigned)kw >= (unsigned)bz;
         if (far || outside) {
-            atomicOr(err, (far ? 1 : 0) | (outside ? 2 : 0));
+            raise_err(err, (far ? 1 : 0) | (outside ? 2 : 0));
             return;
         }
         if (F32) {
@@ -1015,7 +1023,7 @@ __global__ void __launch_bounds__(kBlock) k_rhs_final(const CellSeg* segs, int n
 // instead of looping.
 __device__ __forceinline__ double periodic_shift(double v, double lo, double rhi, double len, int* err) {
     if (!(v >= lo - 2.0 * len && v <= rhi + 2.0 * len)) {
-        if (err) atomicOr(err, 8);
+        if (err) raise_err(err, 8);
         return (v < lo) ? lo : rhi;  // NaN compares false: goes to rhi
     }
     if (v > rhi) {
@@ -1045,7 +1053,7 @@ __device__ __forceinline__ void gather_grad(const BoxDev& B, const double* __res
     const int j = cic_index(y, B.plo[1], B.dxi[1], &yint);
     const int k = cic_index(z, B.plo[2], B.dxi[2], &zint);
     if (i < -nx + 2 || i >= 2 * nx - 1 || j < -ny + 2 || j >= 2 * ny - 1 || k < -nz + 2 || k >= 2 * nz - 1)
-        atomicOr(err, 4);
+        raise_err(err, 4);
     int ix[4], iy[4], iz[4];
 #pragma unroll
     for (int mm = 0; mm < 4; ++mm) {
