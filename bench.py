@@ -594,9 +594,9 @@ def _stage_of_kernel(name):
         mode = int(mt.group(4)) if mt else -1
         return {1: "sweep0", 2: "sweep_p", 4: "sweep_u", 6: "sweep_p", 0: "sweep"}.get(mode, "sweep?"), \
             (mt.group(1) if mt else "?")
-    for k, v in (("k_residual0", "residual"), ("k_kick_tiled", None), ("k_deposit_mom", "deposit_mom"),
-                 ("k_deposit", "deposit"), ("k_fold", "fold"), ("k_resid_restrict_z", "resid_restrict"),
-                 ("k_resid_restrict", "resid_restrict"), ("k_coarse_vcycle", "coarse"), ("k_migrate", "migrate"),
+    for k, v in (("k_residual", "residual"), ("k_leg", "leg"), ("k_kick_tiled", None), ("k_deposit", "deposit"),
+                 ("k_fold", "fold"), ("k_resid_restrict_z", "resid_restrict"), ("k_resid_restrict", "resid_restrict"),
+                 ("k_coarse_vcycle", "coarse"), ("k_migrate", "migrate"), ("k_resort", "resort"),
                  ("k_scatter", "scatter"), ("k_keys", "keys"), ("k_make_items", "items"),
                  ("k_rhs_sum", "rhs"), ("k_check", "check"), ("k_update0", "update"),
                  ("k_kick_deferred", "kick_deferred"), ("k_fill", "fill"), ("k_scan", "scan"),

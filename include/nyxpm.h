@@ -88,7 +88,8 @@ typedef struct nyxpm_opts {
                           it (128x8, 64x16, 64x8, 32x8, 16x8); 0 = chosen per level */
     int sweep_zchunk;  /* z-planes per fused-sweep block; 0 = chosen per level */
     int kick_chunk;    /* particles per work item of the tile-staged kick (>= 256);
-                          0 = default (4096) */
+                          0 = default (4096, fewer where the slots make few
+                          items or a clump's tiles would hold the launch) */
     int separate_kicks; /* 0 = nyxpm_pm_steps runs the closing kick of a step and
                            the next step's kick-drift as one particle pass
                            (bit-identical); 1 = separate passes */

@@ -247,6 +247,8 @@ struct nyxpm_ctx {
     unsigned long long* split_acc = nullptr;  // their accumulators (zero between deposits)
     int* split_done = nullptr;                // parts arrived
     int split_cap = 0;
+    long long split_min = 0;  // tiles above are cut into parts of split_part slots
+    int split_part = 0;
     int* ndefer = nullptr;  // entries of the list handed from the tile-staged kick to k_kick_deferred
     // particle time step (estTimestep): per-box minimum as bits, kept by the closing
     // kicks when cfl > 0; valid for the state after the last such kick (a = dt_a)
@@ -1236,8 +1238,8 @@ struct ItemTables {
     HeavyItem* heavy = nullptr;
     unsigned long long* split_acc = nullptr;
     int* split_done = nullptr;
-    long long items_cap = 0, heavy_cap = 0, split_cap = 0;
-    int chunk = 0;
+    long long items_cap = 0, heavy_cap = 0, split_cap = 0, split_min = 0;
+    int chunk = 0, split_part = 0;
 };
 
 // Particles per work item of the tile-staged kernels for `slots` slots.  An item stages
@@ -1258,15 +1260,19 @@ int choose_chunk(const nyxpm_ctx* c, long long slots) {
     return chunk;
 }
 
-// New tables for `slots` particle slots (the context's stay until set_items).
-int alloc_items(nyxpm_ctx* c, long long slots, ItemTables* t) {
+// New tables for `slots` slots of `np` particles (the context's stay until set_items).
+int alloc_items(nyxpm_ctx* c, long long slots, long long np, ItemTables* t) {
     t->chunk = choose_chunk(c, slots);
     t->items_cap = c->ntiles_total + slots / t->chunk + 1;
     if (t->items_cap > 0x7fffffffLL) FAIL(c, NYXPM_ERR_ARG, "too many tile chunks");
-    // a heavy tile's whole block stands for more than kHeavyTile slots, and so does a
-    // part of a split one but for the tile's last
     t->split_cap = std::min<long long>(kSplitShare, slots / kSplitTile);
-    t->heavy_cap = slots / kHeavyTile + t->split_cap + 1;
+    t->split_min = std::max((long long)kSplitTile, np / kSplitShare);
+    t->split_part = (int)std::max((long long)kSplitPart, np / kSplitParts);
+    // a heavy tile's whole block stands for more than kHeavyTile slots, and so does a
+    // part of a split one but for the tile's last; with parts of twice as many, tiles of
+    // more than one part make fewer parts than that, the last included
+    t->heavy_cap = slots / kHeavyTile + 1;
+    if (std::min<long long>(t->split_part, t->split_min) < 2 * kHeavyTile) t->heavy_cap += t->split_cap;
     // (three accumulators per split tile: the momentum deposit's components)
     const size_t words = (size_t)t->split_cap * 3 * split_words(c);
     int rc = dalloc(c, &t->items, t->items_cap);
@@ -1297,16 +1303,16 @@ void set_items(nyxpm_ctx* c, const ItemTables& t) {
     c->split_acc = t.split_acc;
     c->split_done = t.split_done;
     c->split_cap = (int)t.split_cap;
+    c->split_min = t.split_min;
+    c->split_part = t.split_part;
 }
 
 int make_items(nyxpm_ctx* c, const int* mig = nullptr, const Resort& resort = {}) {
     Timed t(c, "items");
     hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nitems, 3LL, 0);
-    const long long split_min = std::max((long long)kSplitTile, c->npart_total / kSplitShare);
-    const int split_part = (int)std::max((long long)kSplitPart, c->npart_total / kSplitParts);
     hipLaunchKernelGGL(k_make_items, dim3(nblocks(c->ntiles_total)), dim3(kBlock), 0, c->stream, c->tbase,
                        c->cursor, c->ntiles_total, c->items, c->nitems, c->kick_chunk, c->heavy, c->nheavy,
-                       c->nsplit, split_min, split_part, c->split_cap, mig, c->hd_mig, resort, c->hd_resort);
+                       c->nsplit, c->split_min, c->split_part, c->split_cap, mig, c->hd_mig, resort, c->hd_resort);
     LAUNCHCK(c);
     c->items_valid = true;
     return NYXPM_OK;
@@ -2175,7 +2181,7 @@ void launch_gather_tiled(nyxpm_ctx* c, int box, double* out, double* rec) {
                        c->tseg_n, c->dboxes, box, c->items, c->nitems, c->phi, A.x, A.y, A.z, A.id, rec ? rec : out,
                        c->err_flag);
     if (rec)
-        hipLaunchKernelGGL(k_unpack_accel, dim3(nblocks(B.np)), dim3(kBlock), 0, c->stream, B.np, rec, out);
+        hipLaunchKernelGGL(k_unpack_accel<G>, dim3(nblocks(B.np)), dim3(kBlock), 0, c->stream, B.np, rec, out);
 }
 
 // Accelerations of box `box`'s particles into `out`, device memory of 3*np doubles;
@@ -2458,7 +2464,7 @@ static int upload_impl(nyxpm_ctx* c, int box, int64_t np, const double* x, const
     }
     HIPCK(c, hipStreamSynchronize(c->stream));
     ItemTables tables;
-    if ((rc = alloc_items(c, slots, &tables))) return rc;
+    if ((rc = alloc_items(c, slots, tot, &tables))) return rc;
     free_particles(c);
     c->P[0] = N[0];
     c->P[1] = N[1];
@@ -3480,7 +3486,7 @@ static int retile_from(nyxpm_ctx* c, const int t[3], const ParticleSnapshot& s) 
     }
     HIPCK(c, hipStreamSynchronize(c->stream));
     ItemTables tables;
-    if ((rc = alloc_items(c, slots, &tables))) return rc;
+    if ((rc = alloc_items(c, slots, c->npart_total, &tables))) return rc;
     free_particles(c);
     c->P[0] = N;
     c->P[1] = PartPtrs{};

@@ -2032,10 +2032,12 @@ __global__ void __launch_bounds__(kBlock) k_gather(const BoxDev* boxes, int box,
 // interpolated from global phi.  REC: the values go out as records of kAccelRec doubles
 // at the upload index (rec, spread over the components by k_unpack_accel), for outputs
 // the caches do not hold: a scattered 8-byte write costs a line.  A wave passes its
-// values through LDS so that adjacent lanes write a record.
+// values through LDS so that adjacent lanes write a record.  With G = float the values
+// are FP32 numbers, and a record is four of those, written by the particle's own lane.
 // Measured, whole call: 9 10^6 clustered particles in random upload order 1144 -> 552 us
 // mixed, 1047 -> 555 us FP64; 2^24 in lattice order 674 -> 529 us (records of 64 bytes
 // 604, 622 and 733 us; 32-byte records written by one lane each 605 us, the first).
+// FP32 records of 16 bytes, the first again: 616 -> 492 us.
 constexpr int kAccelRec = 4;
 template <typename G, bool REC>
 __global__ void __launch_bounds__(kBlock) k_gather_tiled(const BoxSeg* tsegs, int ntseg, const BoxDev* boxes, int box,
@@ -2072,9 +2074,11 @@ __global__ void __launch_bounds__(kBlock) k_gather_tiled(const BoxSeg* tsegs, in
     const int GX = bx + 1, GY = by + 1;
     const G* sg = stage_g<G>(B, phi + B.cell_off, reinterpret_cast<double*>(gather_smem), o0, o1, o2, bx, by, bz);
     __syncthreads();
+    constexpr bool F32 = std::is_same<G, float>::value;
+    constexpr bool EXCH = REC && !F32;
     constexpr int RL = kAccelRec / 2;  // lanes per record
-    __shared__ __align__(16) double sval[REC ? kBlock * 4 : 2];
-    __shared__ int sid[REC ? kBlock : 1];
+    __shared__ __align__(16) double sval[EXCH ? kBlock * 4 : 2];
+    __shared__ int sid[EXCH ? kBlock : 1];
     const int lane = threadIdx.x & (kWave - 1), w0 = threadIdx.x - lane;
     // whole waves together (the lanes past the item's particles hold none)
     for (int q = threadIdx.x; q - lane < it.np; q += kBlock) {
@@ -2082,7 +2086,7 @@ __global__ void __launch_bounds__(kBlock) k_gather_tiled(const BoxSeg* tsegs, in
         const long long o = aid;
         if (q + kBlock < it.np) load(q + kBlock);
         const bool valid = !isnan(px);
-        if (REC) sid[threadIdx.x] = valid ? (int)o : -1;
+        if (EXCH) sid[threadIdx.x] = valid ? (int)o : -1;
         if (valid) {
         double xint, yint, zint;
         const int li = cic_index(px, B.plo[0], B.dxi[0], &xint) - o0;
@@ -2116,7 +2120,9 @@ __global__ void __launch_bounds__(kBlock) k_gather_tiled(const BoxSeg* tsegs, in
         } else {
             gather_grad<G>(B, phi + B.cell_off, px, py, pz, val, err);
         }
-        if (REC) {
+        if (REC && F32) {
+            reinterpret_cast<float4*>(out)[o] = make_float4((float)val[0], (float)val[1], (float)val[2], 0.0f);
+        } else if (REC) {
             double2* sv = reinterpret_cast<double2*>(sval + 4 * threadIdx.x);
             sv[0] = make_double2(val[0], val[1]);
             sv[1] = make_double2(val[2], 0.0);
@@ -2126,7 +2132,7 @@ __global__ void __launch_bounds__(kBlock) k_gather_tiled(const BoxSeg* tsegs, in
             out[2 * B.np + o] = val[2];
         }
         }
-        if (REC) {
+        if (EXCH) {
             // LDS operations of one wave complete in order: no barrier
             __builtin_amdgcn_wave_barrier();
             __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -2144,10 +2150,18 @@ __global__ void __launch_bounds__(kBlock) k_gather_tiled(const BoxSeg* tsegs, in
     }
 }
 
+template <typename G>
 __global__ void __launch_bounds__(kBlock) k_unpack_accel(long long np, const double* __restrict__ rec,
                                                          double* __restrict__ out) {
     const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
     if (q >= np) return;
+    if (std::is_same<G, float>::value) {
+        const float4 a = reinterpret_cast<const float4*>(rec)[q];
+        out[q] = (double)a.x;
+        out[np + q] = (double)a.y;
+        out[2 * np + q] = (double)a.z;
+        return;
+    }
     const double2* r = reinterpret_cast<const double2*>(rec) + (kAccelRec / 2) * q;
     const double2 a = r[0], b = r[1];
     out[q] = a.x;
