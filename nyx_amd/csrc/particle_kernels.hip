@@ -39,12 +39,6 @@ __device__ __forceinline__ void raise_err(int* err, int flags) {
         if (flags >> i & 1) __hip_atomic_store(&err[i], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
-// Wrap an index known to lie within one period of [0, n); flags anything else.
-__device__ __forceinline__ int wrap_checked(int i, int n, int* err) {
-    if (i < -n || i >= 2 * n) { if (err) raise_err(err, 1); }
-    return wrap1(i, n);
-}
-
 // Wave-aggregated atomicAdd: lanes with equal keys share one atomic.  Returns, for
 // each valid lane, the counter's previous value plus the lane's rank among the
 // lanes with its key.  Must be called by every lane of the wave.
