@@ -1331,8 +1331,8 @@ int phase_migrate(nyxpm_ctx* c, bool* done) {
                            c->tcap, c->cursor, A, c->mig, c->err_flag);
     }
     LAUNCHCK(c);
-    // the items of the layout as migrated (made again if a full sort follows); the
-    // kernel also passes the flags to the host
+    // the items of the layout as migrated (none after an overflow; made again by the full
+    // sort that follows then); the kernel also passes the flags to the host
     int rc;
     if ((rc = make_items(c, c->mig))) return rc;
     HIPCK(c, hipStreamSynchronize(c->stream));
@@ -1340,6 +1340,7 @@ int phase_migrate(nyxpm_ctx* c, bool* done) {
     c->n_moved += c->h_mig[1];
     *done = c->h_mig[0] == 0 && c->holes * 1024 <= c->npart_total * (long long)c->hole_num;
     if (*done) ++c->n_inc_sorts;
+    c->items_valid = *done;
     return NYXPM_OK;
 }
 

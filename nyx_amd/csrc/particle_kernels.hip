@@ -1173,9 +1173,13 @@ __global__ void __launch_bounds__(kBlock) k_make_items(const long long* __restri
         for (int q = 0; q < 4; ++q)
             __hip_atomic_store(&h_resort[q], st[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
+    // a migration that ran out of slack has counted the particles it could not place in
+    // thw, whose sum then passes the slots that the lists are sized for: no lists (the
+    // full sort that follows makes them)
+    const bool overflow = mig && mig[0] != 0;
     int nc = 0;
     long long p0 = 0, cnt = 0;
-    if (t < ntiles) {
+    if (t < ntiles && !overflow) {
         p0 = tbase[t];
         cnt = thw[t];
         nc = (int)((cnt + chunk - 1) / chunk);

@@ -136,3 +136,31 @@ def test_timing_select_times_only_the_named_stages(nyx):
         for d_ in range(3):
             assert np.array_equal(a[0][d_], q[0][d_])
             assert np.array_equal(a[1][d_], q[1][d_])
+
+
+@pytest.mark.parametrize("n,per_cell,cells,slack", [
+    ((32, 32, 32), 1.0, 4.0, 0.0),          # default slack
+    ((32, 32, 32), 4.0, 4.0, 0.0),          # tiles above 2048 slots
+    ((64, 64, 64), 1.5, 2.0, 0.0),
+    ((32, 32, 32), 1.0, 1.0, 1.0 / 1024),
+])
+def test_overflowing_migration_makes_no_items(nyx, n, per_cell, cells, slack):
+    # a step after which the particles counted into the tiles (placed or not) would make
+    # more work items or heavy deposit blocks than the particle slots allow for
+    r = np.random.default_rng(71)
+    npart = int(per_cell * n[0] * n[1] * n[2])
+    pos = [r.random(npart) for _ in range(3)]
+    vel = [cells / n[0] / 1e-3 * r.standard_normal(npart) for _ in range(3)]
+    res = []
+    for s in (-1.0, slack):
+        with nyx.PMContext(nyx.BoxGeom(n), resort_slack=s) as c:
+            c.upload(0, pos, vel, m_const=1.0 / npart)
+            c.pm_init(1.0, 1.0, 1e-10)
+            its = list(c.pm_steps(3, 1e-3, rel_tol=1e-10))
+            c.move_kick_drift(1e-3)
+            rho = c.assign_density(0)
+            p, v = c.download(0)
+            res.append(list(p) + list(v) + [c.get_phi(0), rho, its])
+            assert c.sort_stats()["incremental"] == 0
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
