@@ -2190,13 +2190,23 @@ void launch_gather_tiled(nyxpm_ctx* c, int box, double* out, double* rec) {
 // kUnsortDirect particles (at 2^18 the thread-per-particle kernel takes 45 us, the
 // staged one 49) where they are binned and the box holds most of the context's slots
 // (the launch walks every box's items), through records in the idle buffer where that
-// exists and holds no list of moves (9 of the 64 KB of LDS are the records).
+// exists and holds no list of moves (9 of the 64 KB of LDS are the records).  Not where
+// the tiles hold few particles: the staged kernel reads phi of every tile that holds any,
+// the other one 32 values per particle.  At most 20 staged cells per particle in FP64, 32
+// in mixed precision (its records are half as wide); us, thread per particle / staged,
+// with 16x8x8 tiles: 512^3 cells and 2 particles per tile 136 / 1040 (139 / 870 mixed),
+// 30 per tile 925 / 1278 (986 / 1032), 122 per tile 2528 / 1567 (2750 / 1228), 256^3 and
+// 61 per tile 140 / 177 (152 / 151), 97 per tile 175 / 198 (188 / 160), 130 per tile 269 /
+// 214 (288 / 171).
+constexpr int kStagedPerParticle[2] = {20, 32};
 int launch_gather(nyxpm_ctx* c, int box, double* out) {
     const Box& B = c->boxes[box];
     PartPtrs& A = c->P[c->cur];
     const bool mixed = c->precision == NYXPM_MIXED;
     const size_t lds = mixed ? stage_lds<float>(c) : stage_lds<double>(c);
-    if (c->items_valid && B.np > kUnsortDirect && 2 * B.span >= c->part_cap && lds <= 48 * 1024) {
+    const long long staged = B.ntiles * (c->tile[0] + 3) * (c->tile[1] + 3) * (c->tile[2] + 3);
+    if (c->items_valid && B.np > kUnsortDirect && staged <= kStagedPerParticle[mixed] * B.np &&
+        2 * B.span >= c->part_cap && lds <= 48 * 1024) {
         PartPtrs& I = c->P[1 - c->cur];
         const bool room = I.x && I.bytes >= (size_t)B.np * kAccelRec * sizeof(double);
         double* rec = room && !c->moves_pending ? I.x : nullptr;

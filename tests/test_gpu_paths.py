@@ -262,6 +262,30 @@ def test_tiled_gather_equals_thread_per_particle(nyx, npart, precision):
 
 
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("per_tile", [71, 72, 114, 115])
+def test_gather_of_sparse_tiles(nyx, per_tile, precision):
+    # either side of the particles per tile from which the gather stages g per tile (115
+    # of 16x8x8 cells in FP64, 72 in mixed precision): the values of the
+    # thread-per-particle kernel of a context that has not binned them, bit for bit
+    n = (352, 160, 192)
+    npart = per_tile * (n[0] // 16) * (n[1] // 8) * (n[2] // 8)
+    hi = [v / 352 for v in n]
+    r = np.random.default_rng(83)
+    pos = [r.random(npart) * h for h in hi]
+    zero = np.zeros(npart)
+    phi = r.standard_normal((n[2], n[1], n[0]))
+    res = []
+    for binned in (False, True):
+        with ctx1(nyx, n, hi=hi, precision=precision) as c:
+            c.upload(0, pos, [zero] * 3, m_const=1.0)
+            if binned:
+                c.assign_density(want=False)
+            c.set_phi(phi)
+            res.append(c.gather_accel())
+    assert np.array_equal(*res)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("slack,speed", [(0.25, 0.02), (0.002, 1.0), (0.5, 6.0)])
 def test_captured_resort_equals_eager(nyx, precision, slack, speed):
     # captured steps re-sort incrementally and decide on the device about the full sort
