@@ -138,8 +138,12 @@ inline int nblocks(long long n, int per = kBlock) { return (int)((n + per - 1) /
 // components, particles in random upload order / in lattice order: 2^18 42 / 28 us
 // direct, 38 / 37 us records; 2^21 181 / 66 and 110 / 103; 2^24 3641 / 602 and 935 /
 // 737; 2^27 37.1 / 4.8 ms and 6.8 / 6.1 ms.  The order is not known here: above 2^18
-// records cost a lattice order up to 1.5x and save a random one up to 5x.  (One
-// launch and one copy per component before: 36.1 / 8.3 ms at 2^27.)
+// records cost a lattice order up to 1.5x and save a random one up to 5x.  One launch and
+// one copy per component, which remain where records find no room, against records, six /
+// three / two components: 2^27 random 35.7 -> 7.1 / 17.8 -> 8.0 / 11.8 -> 6.9 ms, lattice
+// 6.9 -> 5.9 / 3.4 -> 2.9 / 2.3 -> 1.7 ms, 2^24 lattice 1.07 -> 0.72 / 0.54 -> 0.41 / 0.36
+// -> 0.26 ms (with 64-byte records for any number of components three and two took 5.3 and
+// 5.1 ms in a lattice order at 2^27).
 constexpr long long kUnsortDirect = 1ll << 18;
 
 // V-cycles a captured solve records beyond the most a solve of the same call
@@ -2614,25 +2618,29 @@ int nyxpm_particles_download(nyxpm_ctx* c, int box, double* x, double* y, double
     double* src[6] = {A.x, A.y, A.z, A.vx, A.vy, A.vz};
     double* dst[6] = {x, y, z, vx, vy, vz};
     bool dev = true;
-    int wanted = 0;
-    for (double* p : dst) {
-        if (!p) continue;
-        ++wanted;
-        dev = dev && on_context_device(c, p);
+    UnsortCols cols{};
+    for (int q = 0; q < 6; ++q) {
+        if (!dst[q]) continue;
+        cols.in[cols.n] = src[q];
+        cols.out[cols.n++] = dst[q];
+        dev = dev && on_context_device(c, dst[q]);
     }
-    if (dev && wanted > 1) {
-        // destinations on this device are written in place: directly while the
-        // caches can merge the scattered writes, else through whole-line records in
-        // the idle buffer (free but for a list of moves waiting for the re-sort)
-        UnsortOut out{{x, y, z, vx, vy, vz}};
-        PartPtrs& I = c->P[1 - c->cur];
-        if (B.np <= kUnsortDirect || c->moves_pending || I.bytes < (size_t)B.np * kRecDoubles * sizeof(double)) {
+    // destinations on this device are written in place: directly while the caches can
+    // merge the scattered writes, else through records in the idle buffer where they fit
+    // there and no list of moves waits in it for the re-sort
+    PartPtrs& I = c->P[1 - c->cur];
+    const int rd = cols.n <= 2 ? 2 : cols.n <= 4 ? 4 : 8;
+    const bool records = !c->moves_pending && I.bytes >= (size_t)B.np * rd * sizeof(double);
+    if (dev && cols.n > 1 && (B.np <= kUnsortDirect || records)) {
+        if (B.np <= kUnsortDirect) {
             hipLaunchKernelGGL(k_unsort_all, dim3(nblocks(B.span)), dim3(kBlock), 0, c->stream, B.part_off, B.span,
-                               A, out);
+                               A.x, A.id, cols);
         } else {
-            hipLaunchKernelGGL(k_pack_records, dim3(nblocks(B.span)), dim3(kBlock), 0, c->stream, B.part_off, B.span,
-                               A, I.x);
-            hipLaunchKernelGGL(k_unpack_records, dim3(nblocks(B.np)), dim3(kBlock), 0, c->stream, B.np, I.x, out);
+            auto pack = rd == 2 ? k_pack_records<2> : rd == 4 ? k_pack_records<4> : k_pack_records<8>;
+            auto unpack = rd == 2 ? k_unpack_records<2> : rd == 4 ? k_unpack_records<4> : k_unpack_records<8>;
+            hipLaunchKernelGGL(pack, dim3(nblocks(B.span)), dim3(kBlock), 0, c->stream, B.part_off, B.span, A.x,
+                               A.id, cols, I.x);
+            hipLaunchKernelGGL(unpack, dim3(nblocks(B.np)), dim3(kBlock), 0, c->stream, B.np, I.x, cols);
         }
         LAUNCHCK(c);
         return err_check(c);

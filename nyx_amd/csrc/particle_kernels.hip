@@ -1869,90 +1869,101 @@ __global__ void __launch_bounds__(kBlock) k_unsort(long long p0, long long span,
     out[id[p0 + q]] = in[p0 + q];
 }
 
-// Destinations of a download: x y z vx vy vz in upload order (null: not wanted).
-struct UnsortOut {
-    double* p[6];
+// The wanted components of a download (n of x y z vx vy vz): the particles' arrays and
+// their destinations in upload order.
+struct UnsortCols {
+    const double* in[6];
+    double* out[6];
+    int n;
 };
 
-// All components of a box's particles to their destinations in upload order, one
+// The wanted components of a box's particles to their destinations in upload order, one
 // thread per slot: what the caches hold of the scattered 8-byte writes merges into
 // whole lines while the output is small.
-__global__ void __launch_bounds__(kBlock) k_unsort_all(long long p0, long long span, PartPtrs A, UnsortOut out) {
+__global__ void __launch_bounds__(kBlock) k_unsort_all(long long p0, long long span, const double* __restrict__ x,
+                                                       const int* __restrict__ id, UnsortCols cols) {
     const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
     if (q >= span) return;
     const long long p = p0 + q;
-    const double px = A.x[p];
-    if (isnan(px)) return;
-    const int d = A.id[p];
-    if (out.p[0]) out.p[0][d] = px;
-    if (out.p[1]) out.p[1][d] = A.y[p];
-    if (out.p[2]) out.p[2][d] = A.z[p];
-    if (out.p[3]) out.p[3][d] = A.vx[p];
-    if (out.p[4]) out.p[4][d] = A.vy[p];
-    if (out.p[5]) out.p[5][d] = A.vz[p];
+    if (isnan(x[p])) return;
+    const int d = id[p];
+#pragma unroll
+    for (int k = 0; k < 6; ++k)
+        if (k < cols.n) cols.out[k][d] = cols.in[k][p];
 }
 
 // The same in two passes for outputs the caches do not hold: k_pack_records writes
-// each particle's six components as one 64-byte record at its upload index (whole
-// lines instead of six scattered 8-byte writes, each of which costs a line), and
-// k_unpack_records spreads the records over the component arrays in order.  Both
-// go through LDS so that four lanes move a record as 16-byte pieces.
-// Bound by HBM: 60 + 64 B and 64 + 48 B per particle.
+// each particle's components as one record of RD doubles at its upload index (whole
+// lines, or fewer pieces of them, instead of scattered 8-byte writes, each of which
+// costs a line), and k_unpack_records spreads the records over the component arrays in
+// order.  RD is the smallest of 2, 4 and 8 that holds the wanted components.  Both go
+// through LDS so that RD / 2 lanes move a record as 16-byte pieces (a record of one
+// piece needs none).  Bound by HBM: 60 + 64 B and 64 + 48 B per particle for all six.
 // Measured: see kUnsortDirect.
-constexpr int kRecDoubles = 8;    // doubles per record
-constexpr int kRecStride = 10;    // its stride in LDS (16-byte aligned, spread over the banks)
-__global__ void __launch_bounds__(kBlock) k_pack_records(long long p0, long long span, PartPtrs A,
+template <int RD>
+__global__ void __launch_bounds__(kBlock) k_pack_records(long long p0, long long span, const double* __restrict__ x,
+                                                         const int* __restrict__ id, UnsortCols cols,
                                                          double* __restrict__ rec) {
-    __shared__ __align__(16) double sh[kBlock * kRecStride];
-    __shared__ int sid[kBlock];
+    constexpr int L = RD / 2, ST = RD + 2;  // pieces; LDS stride (16-byte aligned, spread over the banks)
+    __shared__ __align__(16) double sh[L > 1 ? kBlock * ST : 2];
+    __shared__ int sid[L > 1 ? kBlock : 1];
     const long long q = (long long)blockIdx.x * kBlock + threadIdx.x;
     const long long p = p0 + q;
-    int id = -1;
-    if (q < span) {
-        const double px = A.x[p];
-        if (!isnan(px)) {
-            id = A.id[p];
-            double2* s = reinterpret_cast<double2*>(sh + threadIdx.x * kRecStride);
-            s[0] = make_double2(px, A.y[p]);
-            s[1] = make_double2(A.z[p], A.vx[p]);
-            s[2] = make_double2(A.vy[p], A.vz[p]);
-            s[3] = make_double2(0.0, 0.0);
-        }
+    const bool valid = q < span && !isnan(x[p]);
+    double v[RD] = {};
+    int d = -1;
+    if (valid) {
+        d = id[p];
+#pragma unroll
+        for (int k = 0; k < (RD < 6 ? RD : 6); ++k)
+            if (k < cols.n) v[k] = cols.in[k][p];
     }
-    sid[threadIdx.x] = id;
+    double2* out = reinterpret_cast<double2*>(rec);
+    if (L == 1) {
+        if (valid) out[d] = make_double2(v[0], v[1]);
+        return;
+    }
+    double2* s = reinterpret_cast<double2*>(sh + threadIdx.x * ST);
+#pragma unroll
+    for (int c = 0; c < L; ++c) s[c] = make_double2(v[2 * c], v[2 * c + 1]);
+    sid[threadIdx.x] = d;
     __syncthreads();
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-        const int r = it * (kBlock / 4) + threadIdx.x / 4, c = threadIdx.x & 3;
-        const int d = sid[r];
-        if (d >= 0)
-            reinterpret_cast<double2*>(rec + (size_t)d * kRecDoubles)[c] =
-                reinterpret_cast<const double2*>(sh + r * kRecStride)[c];
+    for (int it = 0; it < L; ++it) {
+        const int r = it * (kBlock / L) + threadIdx.x / L, c = threadIdx.x & (L - 1);
+        const int dr = sid[r];
+        if (dr >= 0) out[(size_t)dr * L + c] = reinterpret_cast<const double2*>(sh + r * ST)[c];
     }
 }
 
+template <int RD>
 __global__ void __launch_bounds__(kBlock) k_unpack_records(long long np, const double* __restrict__ rec,
-                                                           UnsortOut out) {
-    __shared__ __align__(16) double sh[kBlock * kRecStride];
+                                                           UnsortCols cols) {
+    constexpr int L = RD / 2, ST = RD + 2, LU = RD < 6 ? L : 3;  // LU: pieces that can hold a component
+    __shared__ __align__(16) double sh[L > 1 ? kBlock * ST : 2];
     const long long base = (long long)blockIdx.x * kBlock;
-#pragma unroll
-    for (int it = 0; it < 4; ++it) {
-        const int r = it * (kBlock / 4) + threadIdx.x / 4, c = threadIdx.x & 3;
-        if (base + r < np && c < 3)
-            reinterpret_cast<double2*>(sh + r * kRecStride)[c] =
-                reinterpret_cast<const double2*>(rec + (size_t)(base + r) * kRecDoubles)[c];
-    }
-    __syncthreads();
     const long long d = base + threadIdx.x;
+    const double2* in = reinterpret_cast<const double2*>(rec);
+    double2 v[LU];
+    if (L == 1) {
+        if (d < np) v[0] = in[d];
+    } else {
+#pragma unroll
+        for (int it = 0; it < L; ++it) {
+            const int r = it * (kBlock / L) + threadIdx.x / L, c = threadIdx.x & (L - 1);
+            if (base + r < np && c < LU)
+                reinterpret_cast<double2*>(sh + r * ST)[c] = in[(size_t)(base + r) * L + c];
+        }
+        __syncthreads();
+#pragma unroll
+        for (int c = 0; c < LU; ++c) v[c] = reinterpret_cast<const double2*>(sh + threadIdx.x * ST)[c];
+    }
     if (d >= np) return;
-    const double2* s = reinterpret_cast<const double2*>(sh + threadIdx.x * kRecStride);
-    const double2 a = s[0], b = s[1], c = s[2];
-    if (out.p[0]) out.p[0][d] = a.x;
-    if (out.p[1]) out.p[1][d] = a.y;
-    if (out.p[2]) out.p[2][d] = b.x;
-    if (out.p[3]) out.p[3][d] = b.y;
-    if (out.p[4]) out.p[4][d] = c.x;
-    if (out.p[5]) out.p[5][d] = c.y;
+#pragma unroll
+    for (int c = 0; c < LU; ++c) {
+        if (2 * c < cols.n) cols.out[2 * c][d] = v[c].x;
+        if (2 * c + 1 < cols.n) cols.out[2 * c + 1][d] = v[c].y;
+    }
 }
 
 __global__ void __launch_bounds__(kBlock) k_iota(long long p0, long long np, int* __restrict__ id) {

@@ -122,6 +122,33 @@ def test_device_download_equals_host_download(nyx, npart, slack):
         check((0, 5))
 
 
+@pytest.mark.parametrize("slack", [0.0, -1.0])
+@pytest.mark.parametrize("use", [(0, 1), (3, 5), (0, 1, 2), (0, 2, 3, 5), (1, 2, 3, 4, 5), (0, 1, 2, 3, 4, 5)])
+def test_device_download_of_some_components(nyx, use, slack):
+    # records of two, four and eight doubles, and the launch per component where they find
+    # no room (no slack: the idle buffer is too small for eight) or a list of moves waits
+    import torch
+    npart = 2 ** 18 + 77
+    r = np.random.default_rng(43)
+    pos = [r.random(npart) for _ in range(3)]
+    vel = [r.standard_normal(npart) for _ in range(3)]
+    with ctx1(nyx, (32, 32, 32), resort_slack=slack) as c:
+        c.upload(0, pos, vel, m_const=1.0 / npart)
+        c.pm_init()
+        for moving in (False, True):
+            if moving:
+                c.move_kick_drift(1e-3)
+            out = torch.full((6, npart + 1), -7.0, dtype=torch.float64, device="cuda")
+            torch.cuda.synchronize()
+            # (8-byte aligned destinations)
+            c.download_device([out[k, 1:].data_ptr() if k in use else None for k in range(6)])
+            p, v = c.download()
+            got = out.cpu().numpy()
+            assert (got[:, 0] == -7.0).all()
+            for k, ref in enumerate(list(p) + list(v)):
+                assert np.array_equal(got[k, 1:], ref if k in use else np.full(npart, -7.0))
+
+
 @pytest.mark.parametrize("sweep2", [0, 9])
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("boxes", [
