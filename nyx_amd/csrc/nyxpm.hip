@@ -171,7 +171,14 @@ struct nyxpm_ctx {
     // first FP64 residual check (the correction carried over, phi updated once)
     int ir_first = kIrFirstDefault;
     int iters_seen = 0;  // most V-cycles of a box in the solves of the current call
-    int cycles_last = 0; // most V-cycles of a box in the last solve
+    // most V-cycles of a box in the last two solves that converged, from a guess [0] and
+    // from zero [1], of one tolerance and precision (how many cycles the next issues ahead)
+    struct SolveCounts {
+        double rel = 0.0, abs_tol = 0.0;
+        int precision = -1;
+        int last[2] = {0, 0};
+    };
+    SolveCounts solved[2];
     bool no_fused = false;  // force half-sweep smoothing (for comparisons)
     bool untiled_kick = false;  // force the thread-per-particle kick (for comparisons)
     bool separate_kicks = false;  // nyxpm_pm_steps without the kick / kick-drift pairing
@@ -1863,7 +1870,7 @@ int vcycle_group(nyxpm_ctx* c, int g, bool rs) {
 }
 
 template <typename T>
-int solve_impl(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int graph_cycles) {
+int solve_impl(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int graph_cycles, bool from_zero) {
     const int nbox = (int)c->boxes.size();
     int rc;
     // with the residual formed in the first sweep, every residual also starts the
@@ -1891,9 +1898,13 @@ int solve_impl(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int gr
     const int limit = fixed_iters > 0 ? fixed_iters : c->max_iter;
     // V-cycles issued before the host first waits for a check.  A wait empties the
     // stream: 10-15 us until the next cycle's first kernel, of ~45 us a cycle at 32^3.
-    // The previous solve's count less one: solves of one program differ little, and a
-    // cycle too many, with every box stopped, still costs its launches (~25 us).
-    const int ahead = fixed_iters > 0 ? fixed_iters : std::min(c->cycles_last - 1, limit);
+    // A cycle too many, with every box stopped, costs its launches (~25 us), so only as
+    // many as solves like this one (its tolerance and precision, from zero or from a
+    // guess) have needed: one less than the smaller of the last two counts, none without
+    // such a solve.
+    auto& h = c->solved[from_zero];
+    const bool like = h.precision == c->precision && h.rel == rel && h.abs_tol == abs_tol;
+    const int ahead = fixed_iters > 0 ? fixed_iters : like ? std::min({h.last[0] - 1, h.last[1] - 1, limit}) : 0;
     auto look = [&](int it, int g) { return it + g > ahead; };
     if ((rc = check(c, true, fixed_iters, rel, abs_tol, 0, look(0, g0)))) return rc;
     for (int it = 0, g = g0; it <= limit; it += g, g = 1) {
@@ -1908,21 +1919,26 @@ int solve_impl(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int gr
         if ((rc = check(c, false, fixed_iters, rel, abs_tol, g, look(it + g, 1)))) return rc;
     }
     if (c->results_ready && fixed_iters == 0) {
-        c->cycles_last = 0;
-        for (int b = 0; b < nbox; ++b) c->cycles_last = std::max(c->cycles_last, c->h_flags[nbox + b]);
+        int most = 0;
+        bool failed = false;
+        for (int b = 0; b < nbox; ++b) {
+            most = std::max(most, c->h_flags[nbox + b]);
+            failed = failed || c->h_flags[2 * nbox + b];
+        }
+        if (!failed) h = {rel, abs_tol, c->precision, {most, like ? h.last[0] : most}};
     }
     return NYXPM_OK;
 }
 
-int solve(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int graph_cycles) {
+int solve(nyxpm_ctx* c, double rel, double abs_tol, int fixed_iters, int graph_cycles, bool from_zero) {
     c->dt_valid = false;  // phi changes
     c->results_ready = false;
     if (c->precision == NYXPM_MIXED) {
         int rc = ensure_mixed_pools(c);
         if (rc) return rc;
-        return solve_impl<float>(c, rel, abs_tol, fixed_iters, graph_cycles);
+        return solve_impl<float>(c, rel, abs_tol, fixed_iters, graph_cycles, from_zero);
     }
-    return solve_impl<double>(c, rel, abs_tol, fixed_iters, graph_cycles);
+    return solve_impl<double>(c, rel, abs_tol, fixed_iters, graph_cycles, from_zero);
 }
 
 // Per-box results of the last solve; NYXPM_ERR_NOT_CONVERGED if any box failed.
@@ -2067,7 +2083,7 @@ int step_body(nyxpm_ctx* c, double dt, double a_old, double a_new, double four_p
         if ((rc = phase_rhs(c, a_old, four_pi_G))) return rc;
         hipLaunchKernelGGL(k_fill_dbl, dim3(nblocks(c->ncell_total)), dim3(kBlock), 0, c->stream, c->phi,
                            c->ncell_total, 0.0);
-        if ((rc = solve(c, rel, abs_tol, 0, graph_cycles))) return rc;
+        if ((rc = solve(c, rel, abs_tol, 0, graph_cycles, true))) return rc;
         if (graph_cycles == 0 && (rc = solve_results(c, nullptr, nullptr, false))) return rc;
     }
     if ((rc = phase_kick<kKickDrift>(c, dt, a_old, a_half))) return rc;
@@ -2078,7 +2094,7 @@ int step_body(nyxpm_ctx* c, double dt, double a_old, double a_new, double four_p
         invalidate_guess(c);  // Nyx's guess: the old phi just solved
     else if ((rc = prepare_guess(c)))
         return rc;
-    if ((rc = solve(c, rel, abs_tol, 0, graph_cycles))) return rc;
+    if ((rc = solve(c, rel, abs_tol, 0, graph_cycles, false))) return rc;
     if ((rc = phase_kick<kKick>(c, dt, a_half, a_new))) return rc;
     return NYXPM_OK;
 }
@@ -2096,7 +2112,7 @@ int step_tail(nyxpm_ctx* c, double dt, double a_old, double a_new, double four_p
     if ((rc = phase_deposit(c, false, mixed_deposit(c)))) return rc;
     if ((rc = phase_rhs(c, a_new, four_pi_G))) return rc;
     if ((rc = prepare_guess(c))) return rc;
-    if ((rc = solve(c, rel, abs_tol, 0, graph_cycles))) return rc;
+    if ((rc = solve(c, rel, abs_tol, 0, graph_cycles, false))) return rc;
     if (next_a_new > 0.0)
         return phase_kick<kKickPair>(c, dt, a_half, a_new, next_a_old, 0.5 * (next_a_old + next_a_new));
     return phase_kick<kKick>(c, dt, a_half, a_new);
@@ -3011,7 +3027,7 @@ int nyxpm_solve_for_phi(nyxpm_ctx* c, double a, double four_pi_G, double rel_tol
     if (!use_guess)
         hipLaunchKernelGGL(k_fill_dbl, dim3(nblocks(c->ncell_total)), dim3(kBlock), 0, c->stream, c->phi,
                            c->ncell_total, 0.0);
-    if ((rc = solve(c, rel_tol, abs_tol, 0, 0))) return rc;
+    if ((rc = solve(c, rel_tol, abs_tol, 0, 0, !use_guess))) return rc;
     if ((rc = solve_results(c, iters, final_resnorm, false))) return rc;
     c->phi_valid = true;
     invalidate_guess(c);
@@ -3029,7 +3045,7 @@ int nyxpm_solve_poisson(nyxpm_ctx* c, int box, const double* rhs, double* phi_io
     c->f_raw = false;  // the caller's f is final
     HIPCK(c, hipMemcpyAsync(c->phi + B.cell_off, phi_io, B.lev[0].nc * sizeof(double), hipMemcpyHostToDevice,
                             c->stream));
-    if ((rc = solve(c, rel_tol, abs_tol, fixed_iters, 0))) return rc;
+    if ((rc = solve(c, rel_tol, abs_tol, fixed_iters, 0, false))) return rc;
     int it = 0;
     double fin = 0;
     rc = solve_results(c, &it, &fin, false);
@@ -3207,7 +3223,7 @@ int nyxpm_pm_init(nyxpm_ctx* c, double a, double four_pi_G, double rel_tol, doub
     if ((rc = phase_rhs(c, a, four_pi_G))) return rc;
     hipLaunchKernelGGL(k_fill_dbl, dim3(nblocks(c->ncell_total)), dim3(kBlock), 0, c->stream, c->phi,
                        c->ncell_total, 0.0);
-    if ((rc = solve(c, rel_tol, abs_tol, 0, 0))) return rc;
+    if ((rc = solve(c, rel_tol, abs_tol, 0, 0, true))) return rc;
     if ((rc = solve_results(c, nullptr, nullptr, false))) return rc;
     c->phi_valid = true;
     invalidate_guess(c);

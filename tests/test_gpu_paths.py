@@ -380,3 +380,52 @@ def test_cycles_issued_ahead_up_to_the_limit(nyx):
             with pytest.raises(nyx.NyxPMError, match="after 4 cycles"):
                 c.solve_poisson(f, rel_tol=1e-14)
         assert c.solve_poisson(f, rel_tol=1e-2)[1] <= 4
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+def test_cycles_issued_ahead_fit_the_solve(nyx, precision):
+    # a solve that needs few cycles launches no more than it needs (one level-0 residual
+    # each, and the first) after one that failed, one from zero, one of another
+    # tolerance; alternating hard and easy guesses, at most one
+    n = (32, 32, 32)
+    f = mean_free(n, 93)
+    first = 5 if precision == "mixed" else 1
+
+    def residuals(c, solve):
+        c.timing_reset()
+        c.timing_enable(True)
+        try:
+            it = solve()
+        finally:
+            c.timing_enable(False)
+            got = c.timing("residual")[0]
+        need = 1 if it == 0 else 2 if it <= first else 2 + it - first
+        return got - need
+
+    with ctx1(nyx, n, precision=precision, max_iter=60) as c:
+        phi = c.solve_poisson(f, rel_tol=1e-13)[0]
+        with pytest.raises(nyx.NyxPMError):
+            c.solve_poisson(f, abs_tol=1e-300, rel_tol=0.0)
+        for rel in (0.0, 1e-9):
+            with pytest.raises(nyx.NyxPMError):
+                c.solve_poisson(f, rel_tol=rel / 1e300, abs_tol=0.0)
+            assert residuals(c, lambda: c.solve_poisson(0 * f, 0 * f, rel_tol=rel / 1e300)[1]) == 0
+        easy = lambda: c.solve_poisson(f, phi, rel_tol=1e-9)[1]
+        hard = lambda: c.solve_poisson(f, rel_tol=1e-9)[1]
+        assert easy() == 0
+        hard()
+        assert residuals(c, easy) <= 1
+        hard()
+        assert residuals(c, easy) <= 1
+    pos, vel, m = nyx.ics.lattice_gaussian(32, nyx.ics.SEED_BASE, sigma_cells=1.0)
+    with ctx1(nyx, n, precision=precision) as c:
+        c.upload(0, pos, vel, m_const=m)
+        c.assign_density(want=False)
+        solve = lambda guess, rel=1e-10: int(c.solve_for_phi(rel_tol=rel, use_guess=guess)[0][0])
+        for _ in range(3):
+            assert solve(False) > 3
+            assert residuals(c, lambda: solve(True, 1e-9)) == 0
+        for _ in range(2):
+            solve(False)
+        assert residuals(c, lambda: solve(False, 1e-2)) == 0
+        assert residuals(c, lambda: solve(False)) == 0
