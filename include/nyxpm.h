@@ -302,7 +302,8 @@ int nyxpm_pm_steps_comoving(nyxpm_ctx *ctx, int nsteps, double dt, double *a_io,
  * precision_mask bit 0 (FP64) and bit 1 (FP32): for every multigrid depth, the
  * fused smoother's column shape the level allows (128x8, 64x16, 64x8, 32x8,
  * 16x8) and z-chunk (2..256 planes), and the one-pass smoothing pair's column
- * (32x16, 64x16, 32x32, 16x16) and z-chunk (8..512), switched off at a level of
+ * (64x16, 32x32, 32x16, 16x16, 16x8) and z-chunk (8..512) against the untuned
+ * choice, switched off at a level of
  * 2^22 cells or more where two single sweeps are faster.  Bit 2, with
  * particles uploaded: the particle tile of the deposit and the kicks (16x8x8,
  * 12x8x8, 24x8x8, 16x16x8, 16x8x4, 32x8x4, 8x8x8), timed on a deposit, fold,

@@ -3714,8 +3714,8 @@ int nyxpm_autotune(nyxpm_ctx* c, int precision_mask, char* report, int report_le
         rep += buf;
         first_entry = false;
     }
-    // the two-sweep pass: column shape and z-chunk per precision and depth
-    static const int sw2_shapes[][2] = {{32, 16}, {64, 16}, {32, 32}, {16, 16}};
+    // the two-sweep pass: column shape and z-chunk per precision and depth, the present
+    // choice (the model's, whose list is longer) first
     static const int sw2_zcs[] = {8, 16, 32, 64, 128, 256, 512};
     for (int pr = 0; pr < 2; ++pr) {
         if (!(precision_mask & (1 << pr))) continue;
@@ -3725,43 +3725,48 @@ int nyxpm_autotune(nyxpm_ctx* c, int precision_mask, char* report, int report_le
             int maxnz = 0;
             for (int q = 0; q < s2.t.count; ++q)
                 maxnz = std::max(maxnz, c->boxes[c->seg_host[s2.t.first + q].box].lev[d].n[2]);
-            double best = 1e30;
-            int btx = s2.tx, bty = s2.ty, bzc = s2.zc;
-            for (auto& sh : sw2_shapes) {
+            struct Shape {
+                int tx, ty, zc;
+            };
+            std::vector<Shape> trials = {{s2.tx, s2.ty, s2.zc}};
+            for (auto& sh : kSw2Shapes) {
                 bool ok = true;
                 for (int q = 0; q < s2.t.count && ok; ++q)
                     ok = sw2_fits(c->boxes[c->seg_host[s2.t.first + q].box].lev[d], sh[0], sh[1]);
                 if (!ok) continue;
-                for (int zc : sw2_zcs) {
-                    if (zc != sw2_zcs[0] && zc >= 2 * maxnz) continue;
-                    s2.tx = sh[0];
-                    s2.ty = sh[1];
-                    s2.zc = zc;
-                    if ((rc = rebuild_sw2_table(c, pr, d))) return rc;
-                    float ms = 0.f;
-                    for (int rep_i = 0; rep_i < 2; ++rep_i) {  // warm-up, then a timed batch of 4
-                        HIPCK(c, hipEventRecord(e0, c->stream));
-                        for (int k = 0; k < (rep_i ? 4 : 1); ++k) {
-                            if (pr == 0)
-                                launch_sweep2<double, 0>(c, d, c->e64, c->e64b, c->r64, c->e64, c->e64b);
-                            else
-                                launch_sweep2<float, 0>(c, d, c->e32, c->e32b, c->r32, c->e32, c->e32b);
-                        }
-                        HIPCK(c, hipEventRecord(e1, c->stream));
-                        HIPCK(c, hipEventSynchronize(e1));
-                        HIPCK(c, hipEventElapsedTime(&ms, e0, e1));
+                for (int zc : sw2_zcs)
+                    if (zc == sw2_zcs[0] || zc < 2 * maxnz) trials.push_back({sh[0], sh[1], zc});
+            }
+            double best = 1e30;
+            int btx = s2.tx, bty = s2.ty, bzc = s2.zc;
+            for (const Shape& sh : trials) {
+                s2.tx = sh.tx;
+                s2.ty = sh.ty;
+                s2.zc = sh.zc;
+                if ((rc = rebuild_sw2_table(c, pr, d))) return rc;
+                float ms = 0.f;
+                for (int rep_i = 0; rep_i < 2; ++rep_i) {  // warm-up, then a timed batch of 4
+                    HIPCK(c, hipEventRecord(e0, c->stream));
+                    for (int k = 0; k < (rep_i ? 4 : 1); ++k) {
+                        if (pr == 0)
+                            launch_sweep2<double, 0>(c, d, c->e64, c->e64b, c->r64, c->e64, c->e64b);
+                        else
+                            launch_sweep2<float, 0>(c, d, c->e32, c->e32b, c->r32, c->e32, c->e32b);
                     }
-                    LAUNCHCK(c);
-                    const double us = ms * 1e3 / 4.0;
-                    if (c->verbose)
-                        std::fprintf(stderr, "nyxpm autotune: sweep2 %s.d%d %dx%d z-chunk %d: %.2f us\n",
-                                     pr == 0 ? "fp64" : "fp32", d, sh[0], sh[1], zc, us);
-                    if (us < best) {
-                        best = us;
-                        btx = sh[0];
-                        bty = sh[1];
-                        bzc = zc;
-                    }
+                    HIPCK(c, hipEventRecord(e1, c->stream));
+                    HIPCK(c, hipEventSynchronize(e1));
+                    HIPCK(c, hipEventElapsedTime(&ms, e0, e1));
+                }
+                LAUNCHCK(c);
+                const double us = ms * 1e3 / 4.0;
+                if (c->verbose)
+                    std::fprintf(stderr, "nyxpm autotune: sweep2 %s.d%d %dx%d z-chunk %d: %.2f us\n",
+                                 pr == 0 ? "fp64" : "fp32", d, sh.tx, sh.ty, sh.zc, us);
+                if (us < best) {
+                    best = us;
+                    btx = sh.tx;
+                    bty = sh.ty;
+                    bzc = sh.zc;
                 }
             }
             s2.tx = btx;

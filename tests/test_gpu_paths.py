@@ -429,3 +429,25 @@ def test_cycles_issued_ahead_fit_the_solve(nyx, precision):
             solve(False)
         assert residuals(c, lambda: solve(False, 1e-2)) == 0
         assert residuals(c, lambda: solve(False)) == 0
+
+
+def test_autotune_times_what_the_rule_chose(nyx):
+    # a level that only the narrowest column of the smoothing pair fits: it is timed, kept,
+    # and the solves keep their bits
+    geoms = [nyx.BoxGeom((64, 8, 512), (0, 0, 0), (2.0, 0.25, 16.0))] * 3
+    r = np.random.default_rng(95)
+    rho = [r.random((512, 8, 64)) for _ in geoms]
+    res = []
+    for precision in ("fp64", "mixed"):
+        with nyx.PMContext(geoms, precision=precision) as c:
+            for tune in (False, True):
+                if tune:
+                    rep = c.autotune()
+                    for key in ("sweep2.d0", "sweep2.fp64.d0"):
+                        assert rep[key]["shape"] == [16, 8] and 0 < rep[key]["us"] < 1e6 and rep[key]["on"]
+                for b in range(3):
+                    c.set_density(rho[b], b)
+                its = c.solve_for_phi(rel_tol=1e-8, use_guess=False)[0]
+                res.append((list(its), [c.get_phi(b) for b in range(3)]))
+    for a, b in (res[:2], res[2:]):
+        assert a[0] == b[0] and all(np.array_equal(p, q) for p, q in zip(a[1], b[1]))
