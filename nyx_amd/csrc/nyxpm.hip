@@ -234,6 +234,10 @@ struct nyxpm_ctx {
     int hole_num = 64;            // full sort once the emptied slots exceed np * hole_num / 1024
     bool moves_pending = false;
     bool capturing = false;       // a step is being recorded: nothing is read back
+    bool graph_call = false;      // in nyxpm_pm_steps with use_graph
+    bool full_sorts = false;      // its kick-drifts list no moves: full sorts (moves_many)
+    int full_calls = 0;           // further such calls that start so
+    bool recorded_inc = false;    // the recorded steps re-sort incrementally
     long long* resort = nullptr;  // a replay's re-sort state (Resort::state) and its pinned mirror
     long long* h_resort = nullptr;
     long long* hd_resort = nullptr;
@@ -1333,6 +1337,27 @@ int make_items(nyxpm_ctx* c, const int* mig = nullptr, const Resort& resort = {}
 // move into their new tile's slack.  Returns in *done whether the layout is
 // whole again (false: a tile ran out of slack, or the emptied slots passed
 // their limit; the caller then sorts in full).  Reads two flags back.
+// Whether the particles moved by `sorts` re-sorts (or a tile out of slack in all of them)
+// ask for recorded steps with plain full sorts: a migration writes each moved particle to
+// random lines, and a full sort behind it in a recorded step also scans all tiles in one
+// block and copies every slot back.  From 2^22 particles (below, the whole set lies in
+// the caches) and 6/1024 of them per step.  Captured steps of uniform particles, one per
+// cell, mixed precision, us, incremental / full sorts recorded: 512^3 and 0.75% moved 19.7 /
+// 17.2 ms, 1.2% 24.8 / 17.8, 11% 45.9 / 21.1 (0.5%, incremental: 16.6, and 19.0 before
+// captured steps re-sorted incrementally at all); 256^3 and 0.75% 2.86 / 2.51 ms, 11% 6.34 /
+// 3.10; 128^3, incremental, 1.2% 0.79 and 11% 1.23 ms (1.32 and 1.44 before).
+// The next kFullSortsCalls calls start with full sorts, then one looks again.
+constexpr long long kFullSortsMin = 1ll << 22;
+constexpr int kFullSortsNum = 6, kFullSortsCalls = 7;
+bool moves_many(const nyxpm_ctx* c, bool overflow, long long moved, int sorts) {
+    return c->npart_total >= kFullSortsMin && (overflow || moved * 1024 > sorts * c->npart_total * kFullSortsNum);
+}
+
+void set_full_sorts(nyxpm_ctx* c, bool on) {
+    c->full_sorts = on;
+    c->full_calls = on ? kFullSortsCalls : 0;
+}
+
 int phase_migrate(nyxpm_ctx* c, bool* done) {
     PartPtrs& A = c->P[c->cur];
     const long long* moves = reinterpret_cast<const long long*>(c->P[1 - c->cur].y);
@@ -1352,12 +1377,14 @@ int phase_migrate(nyxpm_ctx* c, bool* done) {
     *done = c->h_mig[0] == 0 && c->holes * 1024 <= c->npart_total * (long long)c->hole_num;
     if (*done) ++c->n_inc_sorts;
     c->items_valid = *done;
+    if (c->graph_call) set_full_sorts(c, moves_many(c, c->h_mig[0] != 0, c->h_mig[1], 1));
     return NYXPM_OK;
 }
 
 // The same in a captured step: the migration, and the full sort that it may ask for
 // decided on the device, in place (see Resort).
 int captured_resort(nyxpm_ctx* c) {
+    c->recorded_inc = true;
     PartPtrs& A = c->P[c->cur];
     PartPtrs& I = c->P[1 - c->cur];
     const long long* moves = reinterpret_cast<const long long*>(I.y);
@@ -1428,9 +1455,9 @@ int phase_sort(nyxpm_ctx* c) {
     c->cur = 1 - c->cur;
     c->holes = 0;
     if (c->capturing)
-        hipLaunchKernelGGL(k_fill_dbl, dim3(1), dim3(kBlock), 0, c->stream, reinterpret_cast<double*>(c->resort), 1LL,
-                           0.0);
-    ++c->n_full_sorts;
+        hipLaunchKernelGGL(k_resort_full, dim3(1), dim3(1), 0, c->stream, c->resort, c->hd_resort);
+    else
+        ++c->n_full_sorts;
     if ((rc = make_items(c))) return rc;
     c->sorted_valid = true;
     c->keys_valid = false;
@@ -1992,7 +2019,7 @@ int phase_kick_g(nyxpm_ctx* c, double dt, double a_prev, double a_cur, double a_
         Timed t(c, MODE == kKickPair ? "kick_pair" : MOVE ? "kick_drift" : "kick");
         // incremental re-sort: the kick-drift lists the particles that change tile
         // (the list lives in the idle buffer's y array, like the deferred list in x)
-        const int inc = MOVE && c->slack_num > 0 ? 1 : 0;
+        const int inc = MOVE && c->slack_num > 0 && !c->full_sorts ? 1 : 0;
         long long* moves = reinterpret_cast<long long*>(c->P[1 - c->cur].y);
         hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nmove, 4LL, 0);
         if (MOVE && !inc)
@@ -2513,6 +2540,7 @@ static int upload_impl(nyxpm_ctx* c, int box, int64_t np, const double* x, const
     }
     c->npart_total = tot;
     c->moves_pending = false;
+    c->full_calls = 0;
     invalidate_guess(c);
     // mass bookkeeping for the box (sumParticleMass and the fixed-point unit)
     Box& B = c->boxes[box];
@@ -3243,6 +3271,15 @@ int nyxpm_pm_steps(nyxpm_ctx* c, int nsteps, double dt, double a_old, double a_n
     const bool fused = !nyx_faithful && !c->separate_kicks;
     const double a_half = 0.5 * (a_old + a_new);
     if (use_graph && (rc = ensure_guess_buffer(c))) return rc;
+    struct GraphCall {
+        nyxpm_ctx* c;
+        ~GraphCall() { c->graph_call = c->full_sorts = false; }
+    } graph_call{c};
+    c->graph_call = use_graph != 0;
+    if (use_graph && c->full_calls > 0) {
+        c->full_sorts = true;
+        --c->full_calls;
+    }
     c->iters_seen = 0;
     if (fused && nsteps > 0 && (rc = phase_kick<kKickDrift>(c, dt, a_old, a_half))) return rc;
     auto one_step = [&](int s) -> int {
@@ -3254,8 +3291,11 @@ int nyxpm_pm_steps(nyxpm_ctx* c, int nsteps, double dt, double a_old, double a_n
     for (int s = 0; s < nsteps; ++s) {
         // a replay covers two steps; in the fused form both must end in a pair
         // kick.  The first step of a call runs eagerly: its V-cycle count sets
-        // the cycles recorded in the graph.
-        const bool replay = use_graph && s >= 1 && (fused ? s + 2 < nsteps : s + 1 < nsteps);
+        // the cycles recorded in the graph, and the particles that change tile in it how
+        // the recorded steps sort (full sorts start behind an eager step, which uses up
+        // the list of moves).
+        const bool replay = use_graph && s >= 1 && (fused ? s + 2 < nsteps : s + 1 < nsteps) &&
+                            !(c->full_sorts && c->moves_pending);
         if (!replay) {
             if ((rc = one_step(s))) return rc;
             if ((rc = solve_results(c, iters, nullptr, false))) return rc;
@@ -3266,7 +3306,7 @@ int nyxpm_pm_steps(nyxpm_ctx* c, int nsteps, double dt, double a_old, double a_n
         // the launches a capture records depend on which particle buffer is live
         // and on the binning flags; a replay is valid only from the same state
         const int state = c->cur | (c->keys_valid ? 2 : 0) | (c->items_valid ? 4 : 0) | (c->sorted_valid ? 8 : 0) |
-                          (c->moves_pending ? 16 : 0);
+                          (c->moves_pending ? 16 : 0) | (c->full_sorts ? 32 : 0);
         const int cycles = c->graph_cycles > 0 ? c->graph_cycles
                                                : std::min(c->max_iter, std::max(2, c->iters_seen + kGraphMargin));
         bool same = c->gexec && c->g_prec == c->precision && c->g_mode == mode && c->g_state == state &&
@@ -3284,6 +3324,7 @@ int nyxpm_pm_steps(nyxpm_ctx* c, int nsteps, double dt, double a_old, double a_n
             int cur0 = c->cur;
             const long long holes0 = c->holes;
             c->capturing = true;
+            c->recorded_inc = false;
             for (int r = 0; r < 2 && !rc; ++r)
                 rc = fused ? step_tail(c, dt, a_old, a_new, four_pi_G, rel_tol, abs_tol, cycles, a_old, a_new)
                            : step_body(c, dt, a_old, a_new, four_pi_G, rel_tol, abs_tol, nyx_faithful, cycles);
@@ -3318,6 +3359,7 @@ int nyxpm_pm_steps(nyxpm_ctx* c, int nsteps, double dt, double a_old, double a_n
         c->n_full_sorts += c->h_resort[1];
         c->n_inc_sorts += c->h_resort[2];
         c->n_moved += c->h_resort[3];
+        if (c->recorded_inc) set_full_sorts(c, moves_many(c, c->h_resort[2] == 0, c->h_resort[3], 2));
         if (rc) return rc;
         for (int b = 0; b < nbox; ++b) {
             c->iters_seen = std::max(c->iters_seen, c->h_gstat[nbox + b]);

@@ -385,6 +385,14 @@ __global__ void __launch_bounds__(kBlock) k_resort_copy(Resort r, long long slot
     }
 }
 
+// A recorded full sort that is not k_resort_*'s: no emptied slots, counted.
+__global__ void k_resort_full(long long* state, long long* h_state) {
+    state[0] = 0;
+    state[1] += 1;
+    for (int q = 0; q < 4; ++q)
+        __hip_atomic_store(&h_state[q], state[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // The state a replay starts from.
 __global__ void k_resort_state(long long* state, long long holes) {
     state[0] = holes;

@@ -347,6 +347,37 @@ def test_captured_resort_equals_eager(nyx, precision, slack, speed):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("kind", ["pair", "separate", "faithful"])
+def test_captured_full_sorts_of_many_moves(nyx, kind):
+    # from 2^22 particles, captured steps record plain full sorts while more than 6/1024 of
+    # the particles change tile per step (0.02 cells: not; 0.1: they do; 2: tiles overflow),
+    # over calls that change between these, against eager steps bit for bit
+    n, npart = (64, 64, 64), 2 ** 22 + 3
+    r = np.random.default_rng(97)
+    pos = [r.random(npart) for _ in range(3)]
+    vel = [r.standard_normal(npart) for _ in range(3)]
+    m = (0.5 + r.random(npart)) / npart
+    res = []
+    for graph in (False, True):
+        with ctx1(nyx, n, precision="mixed", pair_kicks=kind != "separate") as c:
+            c.upload(0, pos, vel, m=m)
+            c.pm_init(four_pi_G=1e-3)
+            states = []
+            for cells, nsteps in ((0.02, 6), (0.1, 8), (0.1, 7), (2.0, 7), (0.02, 6)):
+                st0 = c.sort_stats()
+                c.pm_steps(nsteps, cells / 64, four_pi_G=1e-3, use_graph=graph, nyx_faithful=kind == "faithful")
+                st = {k: v - st0[k] for k, v in c.sort_stats().items()}
+                print(kind, graph, cells, nsteps, st, flush=True)
+                assert st["full"] + st["incremental"] >= nsteps
+                if graph and cells > 0.05:  # all but the first, which looks
+                    assert st["incremental"] <= 1
+                p, v = c.download()
+                states += list(p) + list(v) + [c.get_phi()]
+            res.append(states)
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 def test_cycles_issued_ahead(nyx, precision):
     # V-cycles issued before the host looks at a check (one fewer than the last solve
