@@ -248,8 +248,9 @@ struct nyxpm_ctx {
     int* h_mig = nullptr;         // pinned mirror
     int* hd_mig = nullptr;        // its device address
     long long* bsum = nullptr;
-    // AssignDensityAndVels: halo slots of the three momentum deposits (allocated by the
-    // first call, with the tile's size) and the per-box maxima
+    // AssignDensityAndVels: halo slots of the three momentum deposits where the idle buffer
+    // is too small for them (allocated by the first such call, with the tile's size) and the
+    // per-box maxima
     double* mom_halo = nullptr;
     unsigned long long* mom_max = nullptr;
     int scan_blocks = 0;
@@ -259,8 +260,13 @@ struct nyxpm_ctx {
     int* nheavy = nullptr;      // nitems + 1
     int* nsplit = nullptr;      // nitems + 2: tiles deposited in parts
     int heavy_cap = 0;
-    unsigned long long* split_acc = nullptr;  // their accumulators (zero between deposits)
-    int* split_done = nullptr;                // parts arrived
+    // their accumulators and the parts arrived: zero between deposits, and touched in a
+    // deposit by device-scope atomics alone, never by plain loads or stores (split_combine)
+    unsigned long long* split_acc = nullptr;
+    int* split_done = nullptr;
+    // the same for the three momentum deposits (allocated by the first that needs them)
+    unsigned long long* mom_acc = nullptr;
+    int* mom_done = nullptr;
     int split_cap = 0;
     long long split_min = 0;  // tiles above are cut into parts of split_part slots
     int split_part = 0;
@@ -1185,7 +1191,7 @@ void free_particles(nyxpm_ctx* c) {
     dfree(c->items);
     dfree(c->heavy);
     dfree(c->split_acc);
-    dfree(c->split_done);
+    dfree(c->mom_acc);
 }
 
 // A particle buffer of n slots: one allocation, each array 256-byte aligned in it.
@@ -1275,6 +1281,19 @@ int choose_chunk(const nyxpm_ctx* c, long long slots) {
     return chunk;
 }
 
+// Accumulators of n split tiles and their counters behind them, one allocation, zeroed
+// (2 u64 words per LDS cell: 22 KB a tile of 16x8x8).
+int alloc_split(nyxpm_ctx* c, long long n, unsigned long long** acc, int** done) {
+    const size_t words = (size_t)n * split_words(c), all = words + (size_t)(n + 1) / 2;
+    int rc = dalloc(c, acc, all);
+    if (rc || !n) return rc;
+    *done = reinterpret_cast<int*>(*acc + words);
+    hipLaunchKernelGGL(k_fill_dbl, dim3(nblocks((long long)all)), dim3(kBlock), 0, c->stream,
+                       reinterpret_cast<double*>(*acc), (long long)all, 0.0);
+    LAUNCHCK(c);
+    return NYXPM_OK;
+}
+
 // New tables for `slots` slots of `np` particles (the context's stay until set_items).
 int alloc_items(nyxpm_ctx* c, long long slots, long long np, ItemTables* t) {
     t->chunk = choose_chunk(c, slots);
@@ -1288,24 +1307,14 @@ int alloc_items(nyxpm_ctx* c, long long slots, long long np, ItemTables* t) {
     // more than one part make fewer parts than that, the last included
     t->heavy_cap = slots / kHeavyTile + 1;
     if (std::min<long long>(t->split_part, t->split_min) < 2 * kHeavyTile) t->heavy_cap += t->split_cap;
-    // (three accumulators per split tile: the momentum deposit's components)
-    const size_t words = (size_t)t->split_cap * 3 * split_words(c);
     int rc = dalloc(c, &t->items, t->items_cap);
     if (!rc) rc = dalloc(c, &t->heavy, t->heavy_cap);
-    if (!rc) rc = dalloc(c, &t->split_acc, words);
-    if (!rc) rc = dalloc(c, &t->split_done, 3 * t->split_cap);
+    if (!rc) rc = alloc_split(c, t->split_cap, &t->split_acc, &t->split_done);
     if (rc) {
         dfree(t->items);
         dfree(t->heavy);
-        dfree(t->split_acc);
-        dfree(t->split_done);
-        return rc;
     }
-    if (t->split_cap) {
-        HIPCK(c, hipMemsetAsync(t->split_acc, 0, words * 8, c->stream));
-        HIPCK(c, hipMemsetAsync(t->split_done, 0, 3 * t->split_cap * sizeof(int), c->stream));
-    }
-    return NYXPM_OK;
+    return rc;
 }
 
 // Into the context, which holds none (free_particles).
@@ -2971,7 +2980,12 @@ static int density_and_vels_impl(nyxpm_ctx* c, int box, double* dst) {
     const int nbox = (int)c->boxes.size();
     const long long H = (long long)c->ntiles_total * c->halo_stride;
     int rc;
-    if (!c->mom_halo && (rc = dalloc(c, &c->mom_halo, 3 * H))) return rc;
+    // the halo slots in the idle buffer where they fit (it holds no list of moves behind a sort)
+    PartPtrs& I = c->P[1 - c->cur];
+    double* halo = !c->moves_pending && I.bytes >= (size_t)(3 * H) * sizeof(double) ? I.x : nullptr;
+    if (!halo && !c->mom_halo && (rc = dalloc(c, &c->mom_halo, 3 * H))) return rc;
+    if (!halo) halo = c->mom_halo;
+    if (c->split_cap && !c->mom_acc && (rc = alloc_split(c, 3LL * c->split_cap, &c->mom_acc, &c->mom_done))) return rc;
     const size_t lds = 2 * sizeof(unsigned long long) * (c->tile[0] + 1) * (c->tile[1] + 1) * (c->tile[2] + 1);
     const dim3 grid(c->heavy_cap + c->tseg_blocks);
     hipLaunchKernelGGL(k_deposit<false>, grid, dim3(kBlock), lds, c->stream, c->tseg, c->tseg_n, c->dboxes,
@@ -2984,10 +2998,10 @@ static int density_and_vels_impl(nyxpm_ctx* c, int box, double* dst) {
         hipLaunchKernelGGL(k_max_mom, dim3(c->pseg_blocks), dim3(kBlock), 0, c->stream, c->pseg, c->pseg_n,
                            c->dboxes, A.x, A.m, A.vx, A.vy, A.vz, c->mom_max);
     const DepositMom mom{{A.vx, A.vy, A.vz}, c->mom_max, {c->r64, c->e64, c->e64b},
-                         {c->mom_halo, c->mom_halo + H, c->mom_halo + 2 * H}};
+                         {halo, halo + H, halo + 2 * H}};
     hipLaunchKernelGGL((k_deposit<false, true>), dim3(grid.x, 3), dim3(kBlock), lds, c->stream, c->tseg, c->tseg_n,
-                       c->dboxes, c->tbase, c->cursor, c->heavy, c->nheavy, c->heavy_cap, c->split_acc,
-                       split_words(c), c->split_done, c->split_cap, A.x, A.y, A.z, A.m, c->own, c->halo,
+                       c->dboxes, c->tbase, c->cursor, c->heavy, c->nheavy, c->heavy_cap, c->mom_acc,
+                       split_words(c), c->mom_done, c->split_cap, A.x, A.y, A.z, A.m, c->own, c->halo,
                        c->err_flag, mom);
     const FoldFields<4> fields{{c->own, mom.own[0], mom.own[1], mom.own[2]},
                                {c->halo, mom.halo[0], mom.halo[1], mom.halo[2]}};

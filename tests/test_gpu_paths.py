@@ -252,6 +252,48 @@ def test_density_and_vels_second_box_of_a_batch(nyx, orc, clump):
         assert np.array_equal(out[d + 1] == 0, out[0] == 0)
 
 
+@pytest.mark.parametrize("per_tile,clump", [(40, 0), (3400, 0), (3400, 30001)])
+def test_density_and_vels_scratch(nyx, orc, per_tile, clump):
+    # the momentum deposits' halo slots in the idle buffer (60 B a slot) or their own where
+    # those are more, and the accumulators of split tiles, which only this call allocates:
+    # what the context holds after it, the oracle's fields, and the steps go on as without
+    n = (64, 32, 40)
+    hi = (1.6, 0.8, 1.0)
+    tiles = 4 * 4 * 5
+    npart = per_tile * tiles
+    r = np.random.default_rng(73)
+    pos = [np.concatenate([r.random(npart) * h, 0.41 + 0.02 * r.random(clump)]) for h in hi]
+    vel = [r.standard_normal(npart + clump) for _ in range(3)]
+    m = (0.5 + r.random(npart + clump)) / npart
+    halo = 3 * tiles * (17 * 9 * 9 - 16 * 8 * 8) * 8
+    res = []
+    for call in (False, True):
+        with ctx1(nyx, n, hi=hi) as c:
+            c.upload(0, pos, vel, m=m)
+            c.pm_init()
+            c.pm_steps(2, 1e-4)
+            c.assign_density(want=False)
+            if call:
+                ref = orc.deposit_vels(n, (0, 0, 0), hi, *c.download(), m=m)
+                held = c.device_bytes()
+                out = c.assign_density_and_vels()
+                more = c.device_bytes() - held
+                assert np.array_equal(c.assign_density_and_vels(), out)
+                assert c.device_bytes() - held == more
+                slots = npart + clump + ((npart + clump) * 256 + 1023 >> 10) + 16 * tiles
+                split = 8 * (slots // 4096 * 3 * 2 * 17 * 9 * 9 + (slots // 4096 * 3 + 1) // 2)
+                assert more == split + (halo if slots * 60 < halo else 0)
+                assert np.abs(out[0] - ref[0]).max() <= 1e-13 * ref[0].max()
+                big = ref[0] > 1e-3 * ref[0].max()
+                for d in range(3):
+                    assert np.abs(out[d + 1] - ref[d + 1])[big].max() <= 1e-11
+            c.pm_steps(2, 1e-4)
+            p, v = c.download()
+            res.append(list(p) + list(v) + [c.get_phi()])
+    for a, b in zip(*res):
+        assert np.array_equal(a, b)
+
+
 @pytest.mark.parametrize("precision", ["fp64", "mixed"])
 @pytest.mark.parametrize("npart", [3000, 2 ** 18 + 5])
 def test_tiled_gather_equals_thread_per_particle(nyx, npart, precision):
