@@ -252,8 +252,8 @@ __global__ void __launch_bounds__(kBlock) k_scan_down(const int* __restrict__ co
     if (blockIdx.x == 0 && threadIdx.x == 0) start[n] = bsum[gridDim.x];
 }
 
-// One particle buffer: arrays of one allocation that starts at x (`bytes` long, 0
-// for a buffer not allocated).
+// One particle buffer: arrays of one allocation that starts at x (`bytes` long), or, with
+// bytes = 0, of their own (or none).
 struct PartPtrs {
     double *x, *y, *z, *vx, *vy, *vz, *m;
     int* id;

@@ -524,3 +524,29 @@ def test_autotune_times_what_the_rule_chose(nyx):
                 res.append((list(its), [c.get_phi(b) for b in range(3)]))
     for a, b in (res[:2], res[2:]):
         assert a[0] == b[0] and all(np.array_equal(p, q) for p, q in zip(a[1], b[1]))
+
+
+def test_uploads_across_the_particle_buffers_kinds(nyx):
+    # particle buffers of an allocation per array (below 2^18 slots) and of one for all, with
+    # and without masses, replaced by each other in one context: as in a context of its own
+    n = (32, 32, 32)
+
+    def steps(c, npart, mass, seed):
+        r = np.random.default_rng(seed)
+        pos = [r.random(npart) for _ in range(3)]
+        vel = [r.standard_normal(npart) for _ in range(3)]
+        m = (0.5 + r.random(npart)) / npart if mass else None
+        c.upload(0, pos, vel, m=m, m_const=1.0 / npart)
+        c.pm_init()
+        c.pm_steps(2, 1e-3)
+        p, v = c.download()
+        return list(p) + list(v) + [c.get_phi()]
+
+    runs = [(5000, False), (300000, False), (5000, True), (300000, True), (209000, True), (7000, True)]
+    with ctx1(nyx, n) as c:
+        together = [steps(c, npart, mass, 100 + i) for i, (npart, mass) in enumerate(runs)]
+    for i, (npart, mass) in enumerate(runs):
+        with ctx1(nyx, n) as c:
+            alone = steps(c, npart, mass, 100 + i)
+        for a, b in zip(together[i], alone):
+            assert np.array_equal(a, b)
