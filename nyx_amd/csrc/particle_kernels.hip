@@ -1153,6 +1153,11 @@ __global__ void __launch_bounds__(kBlock) k_kick(const BoxSeg* segs, int nseg, c
 // item is processed independently, so results do not.
 constexpr int kChunk = 16 * kBlock;  // default particles per work item (fewer items: less phi staging)
 
+// Entries of a tile above which a wave writes them together: one thread takes ~50 ns an
+// entry, and a clump's tile has up to 2048 parts and np / chunk items (4 10^6 particles in
+// one cell of 64^3: 146 -> 12 us, half of 2^24 in one cell of 256^3: 149 -> 15 us).
+constexpr int kItemsByThread = 8;
+
 struct TileItem {
     long long p0;   // first particle
     int np;         // particles in this chunk
@@ -1183,7 +1188,7 @@ __global__ void __launch_bounds__(kBlock) k_make_items(const long long* __restri
     // thw, whose sum then passes the slots that the lists are sized for: no lists (the
     // full sort that follows makes them)
     const bool overflow = mig && mig[0] != 0;
-    int nc = 0;
+    int nc = 0, parts = 0, len = 0, split = -1, h = 0;
     long long p0 = 0, cnt = 0;
     if (t < ntiles && !overflow) {
         p0 = tbase[t];
@@ -1191,17 +1196,15 @@ __global__ void __launch_bounds__(kBlock) k_make_items(const long long* __restri
         nc = (int)((cnt + chunk - 1) / chunk);
         // tiles the deposit starts first (the longest blocks), the heaviest in parts
         if (cnt > kHeavyTile) {
-            int split = -1, parts = 1, len = (int)cnt;
+            parts = 1;
+            len = (int)cnt;
             if (cnt > split_min) split = atomicAdd(nsplit, 1);
             if (split >= split_cap) split = -1;
             if (split >= 0) {
                 len = split_part;
                 parts = (int)((cnt + len - 1) / len);
             }
-            const int h = atomicAdd(nheavy, parts);
-            for (int q = 0; q < parts; ++q)
-                heavy[h + q] = HeavyItem{(int)t, q * len, (int)min((long long)len, cnt - (long long)q * len), parts,
-                                         split};
+            h = atomicAdd(nheavy, parts);
         }
     }
     // wave-inclusive prefix of nc, one atomic per wave
@@ -1216,12 +1219,29 @@ __global__ void __launch_bounds__(kBlock) k_make_items(const long long* __restri
     if (lane == kWave - 1 && total > 0) base = atomicAdd(nitems, total);
     base = __shfl(base, kWave - 1);
     int slot = base + incl - nc;
-    for (int c = 0; c < nc; ++c) {
+    auto put_item = [&](int at, int c, long long p, long long n, int tile) {
         TileItem it;
-        it.p0 = p0 + (long long)c * chunk;
-        it.np = (int)min((long long)chunk, cnt - (long long)c * chunk);
-        it.tile = (int)t;
-        items[slot + c] = it;
+        it.p0 = p + (long long)c * chunk;
+        it.np = (int)min((long long)chunk, n - (long long)c * chunk);
+        it.tile = tile;
+        items[at + c] = it;
+    };
+    auto put_heavy = [&](int at, int q, int l, long long n, int np, int sp, int tile) {
+        heavy[at + q] = HeavyItem{tile, q * l, (int)min((long long)l, n - (long long)q * l), np, sp};
+    };
+    // a tile of few entries by its thread, one of many by the whole wave
+    const bool wide = max(nc, parts) > kItemsByThread;
+    if (!wide) {
+        for (int c = 0; c < nc; ++c) put_item(slot, c, p0, cnt, (int)t);
+        for (int q = 0; q < parts; ++q) put_heavy(h, q, len, cnt, parts, split, (int)t);
+    }
+    for (unsigned long long m = __ballot(wide); m; m &= m - 1) {
+        const int src = __ffsll((long long)m) - 1;
+        const long long wp = __shfl(p0, src), wn = __shfl(cnt, src);
+        const int wt = __shfl((int)t, src), wc = __shfl(nc, src), ws = __shfl(slot, src);
+        const int wparts = __shfl(parts, src), wh = __shfl(h, src), wl = __shfl(len, src), wsp = __shfl(split, src);
+        for (int c = lane; c < wc; c += kWave) put_item(ws, c, wp, wn, wt);
+        for (int q = lane; q < wparts; q += kWave) put_heavy(wh, q, wl, wn, wparts, wsp, wt);
     }
 }
 

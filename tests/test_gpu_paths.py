@@ -550,3 +550,29 @@ def test_uploads_across_the_particle_buffers_kinds(nyx):
             alone = steps(c, npart, mass, 100 + i)
         for a, b in zip(together[i], alone):
             assert np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("precision", ["fp64", "mixed"])
+@pytest.mark.parametrize("share", [0.3, 1.0])
+def test_items_of_a_clump_by_a_wave(nyx, precision, share):
+    # tiles of more items and deposit parts than one thread writes, next to tiles of few:
+    # steps with the default kick items and with items of 256 particles, against the
+    # thread-per-particle kick
+    r = np.random.default_rng(103)
+    n, npart = (48, 32, 32), 60000
+    clump = int(share * npart)
+    pos = [r.random(npart) * 1.5 if d == 0 else r.random(npart) for d in range(3)]
+    for d in range(3):
+        pos[d][:clump] = (0.4, 0.61, 0.27)[d] + r.random(clump) / 64
+    vel = [0.1 * r.standard_normal(npart) for _ in range(3)]
+    res = []
+    for kw in (dict(kick="global"), {}, dict(kick_chunk=256)):
+        with ctx1(nyx, n, hi=(1.5, 1, 1), precision=precision, **kw) as c:
+            c.upload(0, pos, vel, m_const=1.0 / npart)
+            c.pm_init(four_pi_G=1e-3)
+            c.pm_steps(3, 1e-3, four_pi_G=1e-3)
+            p, v = c.download()
+            res.append(list(p) + list(v) + [c.get_phi(), c.assign_density()])
+    for other in res[1:]:
+        for a, b in zip(res[0], other):
+            assert np.array_equal(a, b)
