@@ -485,10 +485,14 @@ struct DepositMom {
     double* own[3];                     // per component
     double* halo[3];
 };
-// FP64: held to the SGPRs of eight waves per SIMD (seven without: 64 10^6 particles on
-// 448x448x320, density, 1163 us instead of 1156).
+// FP64: compiled for the seven waves per SIMD that the LDS of seven 16x8x8 tiles admits.
+// Without a bound / for eight / for seven waves, deposit, us: 512^3 cells with 2 10^7
+// particles 567 / 538 / 523, with 10^6 555 / 527 / 521, with 2^27 1200 / 1190 / 1170, 256^3
+// with 2 10^6 78 / 74.5 / 72.6 (517, 515, 1150 and 71.2 before tiles were deposited in
+// parts); the momenta, whole call, 512^3 with 2 10^7, none / seven: 4860 / 4680.  FP32: no
+// difference.
 template <bool F32, bool MOM = false>
-__global__ void __launch_bounds__(kBlock, F32 || MOM ? 1 : 8)
+__global__ void __launch_bounds__(kBlock, F32 ? 1 : 7)
     k_deposit(const BoxSeg* segs, int nseg, const BoxDev* boxes, const long long* __restrict__ tbase,
               const int* __restrict__ thw, const HeavyItem* __restrict__ heavy, const int* nheavy, int heavy_cap,
               unsigned long long* split_acc, int split_words, int* split_done, int split_cap,
