@@ -258,10 +258,10 @@ struct nyxpm_ctx {
     unsigned long long* mom_max = nullptr;
     int scan_blocks = 0;
     TileItem* items = nullptr;  // tile chunks of the last sort (tile-staged kernels)
-    int* nitems = nullptr;
+    int* nitems = nullptr;      // counters on a 256-byte line each, cleared together
     HeavyItem* heavy = nullptr; // tiles of more than kHeavyTile slots, or their parts (deposit order)
-    int* nheavy = nullptr;      // nitems + 1
-    int* nsplit = nullptr;      // nitems + 2: tiles deposited in parts
+    int* nheavy = nullptr;      // nitems + 64
+    int* nsplit = nullptr;      // nitems + 128: tiles deposited in parts
     int heavy_cap = 0;
     // their accumulators and the parts arrived: zero between deposits, and touched in a
     // deposit by device-scope atomics alone, never by plain loads or stores (split_combine)
@@ -1143,10 +1143,10 @@ int alloc_fields(nyxpm_ctx* c) {
     if ((rc = dalloc(c, &c->active, nbox))) return rc;
     if ((rc = dalloc(c, &c->iters, nbox))) return rc;
     if ((rc = dalloc(c, &c->failed, nbox))) return rc;
-    if ((rc = dalloc(c, &c->nitems, 3))) return rc;
-    c->nheavy = c->nitems + 1;
-    c->nsplit = c->nitems + 2;
-    HIPCK(c, hipMemset(c->nitems, 0, 3 * sizeof(int)));
+    if ((rc = dalloc(c, &c->nitems, kBlock))) return rc;
+    c->nheavy = c->nitems + 64;
+    c->nsplit = c->nitems + 128;
+    HIPCK(c, hipMemset(c->nitems, 0, kBlock * sizeof(int)));
     if ((rc = dalloc(c, &c->dtmin, nbox))) return rc;
     if ((rc = dalloc(c, &c->mom_max, 3 * nbox))) return rc;
     if ((rc = dalloc(c, &c->nr, (size_t)nbox * kNormSlots))) return rc;
@@ -1354,7 +1354,7 @@ void set_items(nyxpm_ctx* c, const ItemTables& t) {
 
 int make_items(nyxpm_ctx* c, const int* mig = nullptr, const Resort& resort = {}) {
     Timed t(c, "items");
-    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nitems, 3LL, 0);
+    hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(kBlock), 0, c->stream, c->nitems, (long long)kBlock, 0);
     hipLaunchKernelGGL(k_make_items, dim3(nblocks(c->ntiles_total)), dim3(kBlock), 0, c->stream, c->tbase,
                        c->cursor, c->ntiles_total, c->items, c->nitems, c->kick_chunk, c->heavy, c->nheavy,
                        c->nsplit, c->split_min, c->split_part, c->split_cap, mig, c->hd_mig, resort, c->hd_resort);

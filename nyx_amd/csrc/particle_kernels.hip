@@ -1200,20 +1200,11 @@ __global__ void __launch_bounds__(kBlock) k_make_items(const long long* __restri
         p0 = tbase[t];
         cnt = thw[t];
         nc = (int)((cnt + chunk - 1) / chunk);
-        // tiles the deposit starts first (the longest blocks), the heaviest in parts
-        if (cnt > kHeavyTile) {
-            parts = 1;
-            len = (int)cnt;
-            if (cnt > split_min) split = atomicAdd(nsplit, 1);
-            if (split >= split_cap) split = -1;
-            if (split >= 0) {
-                len = split_part;
-                parts = (int)((cnt + len - 1) / len);
-            }
-            h = atomicAdd(nheavy, parts);
-        }
     }
-    // wave-inclusive prefix of nc, one atomic per wave
+    // wave-inclusive prefix of nc, one atomic per wave, before the atomics of the heavy
+    // tiles: the kicks want the items in tile order (each XCD a run of neighbouring tiles),
+    // and waves that reach it a round trip or two late scatter their items (512^3 particles,
+    // half of them in clumps, FP64: kick 2.72 -> 2.51 ms, paired kick 6.97 -> 6.77)
     const int lane = threadIdx.x & (kWave - 1);
     int incl = nc;
     for (int o = 1; o < kWave; o <<= 1) {
@@ -1225,6 +1216,18 @@ __global__ void __launch_bounds__(kBlock) k_make_items(const long long* __restri
     if (lane == kWave - 1 && total > 0) base = atomicAdd(nitems, total);
     base = __shfl(base, kWave - 1);
     int slot = base + incl - nc;
+    // tiles the deposit starts first (the longest blocks), the heaviest in parts
+    if (cnt > kHeavyTile) {
+        parts = 1;
+        len = (int)cnt;
+        if (cnt > split_min) split = atomicAdd(nsplit, 1);
+        if (split >= split_cap) split = -1;
+        if (split >= 0) {
+            len = split_part;
+            parts = (int)((cnt + len - 1) / len);
+        }
+        h = atomicAdd(nheavy, parts);
+    }
     auto put_item = [&](int at, int c, long long p, long long n, int tile) {
         TileItem it;
         it.p0 = p + (long long)c * chunk;
