@@ -681,8 +681,9 @@ int rrz_tile(int pr, const Level& L) {
 
 // Coarse planes per block of k_resid_restrict_z for a depth's levels `lev` (one per box),
 // or 0 where the thread-per-coarse-cell kernel takes them: 16, halved down to 2 while the
-// launch has fewer than 2048 blocks; at least 2^20 cells and one block per CU.  Against
-// that kernel, us: 160x192x224 FP64 34.4 -> 23.5, 112x96x144 FP32 6.9 -> 6.7,
+// launch has fewer than 2048 blocks (FP32, whose tile is twice as high: 1024; us, 2048 ->
+// 1024: 160x192x224 20.3 -> 17.8, 256^3 29.8 -> 28.9); at least 2^20 cells and one block
+// per CU.  Against that kernel, us: 160x192x224 FP64 34.4 -> 23.5, 112x96x144 FP32 6.9 -> 6.7,
 // 80x96x112 FP64 7.1 -> 8.1.
 int rrz_zchunk(int pr, const std::vector<const Level*>& lev) {
     long long cells = 0;
@@ -695,7 +696,7 @@ int rrz_zchunk(int pr, const std::vector<const Level*>& lev) {
         return n;
     };
     int zc = 16;
-    while (zc > 2 && blocks(zc) < 2048) zc /= 2;
+    while (zc > 2 && blocks(zc) < (pr == 0 ? 2048 : 1024)) zc /= 2;
     return blocks(zc) >= 256 ? zc : 0;
 }
 
