@@ -850,12 +850,16 @@ def pmc_summary(fetch_csv, write_csv, copy_fetch_csv, copy_write_csv, fetch_json
         sz = 4 if "float" in nm else 8
         key = stage + ".d0" if stage and (stage.startswith("sweep") or stage == "resid_restrict") else stage
         alg = kernel_bytes(key, N, N, halo, sz) if key else None
+        if alg and gb * 1e9 < 0.9 * alg:
+            # less than the finest level's bytes: a mode that only coarser levels run
+            # with the same grid (FP64's post-smoothing pair there ends in phi)
+            continue
         tail = f"{alg / 1e9:.3f} | {gb / (alg / 1e9):.2f} |" if alg else " | |"
         print(f"| `{nm}` | {len(fv)} | {fk:.4g} | {wk:.4g} | {gb:.3f} | " + tail)
         # the mixed-precision step's kernels (FP32 multigrid, FP32-weight deposit
         # and interpolation) for roofline.traffic
-        mixed_kernel = {"fold": nm.startswith("k_fold<false>"),
-                        "deposit": nm.startswith("k_deposit<true>")}.get(key, "double" not in nm)
+        mixed_kernel = {"fold": nm.startswith("k_fold<false"),
+                        "deposit": nm.startswith("k_deposit<true")}.get(key, "double" not in nm)
         if key and alg:
             # the mixed step's kernels under the stage name, the FP64 step's
             # under "fp64:" + the stage name
