@@ -78,12 +78,20 @@ struct DevBuf {
 };
 
 // Largest double below hi whose cell index stays < n (upper end kept by the
-// periodic shift).
+// periodic shift).  Found by bisection: where hi lies next to zero the doubles below
+// it are so dense that stepping down through them one by one would not end.
 double domain_rhi(double lo, double hi, int n) {
     const double dxi = 1.0 / ((hi - lo) / (double)n);
+    const auto inside = [&](double r) { return (int)std::floor((r - lo) * dxi) < n; };
     double r = std::nextafter(hi, -INFINITY);
-    while ((int)std::floor((r - lo) * dxi) >= n) r = std::nextafter(r, -INFINITY);
-    return r;
+    if (inside(r)) return r;
+    double in = lo, out = r;  // the index grows with r
+    while ((r = std::nextafter(in, INFINITY)) < out) {
+        const double mid = in + 0.5 * (out - in);
+        if (mid > in && mid < out) r = mid;
+        (inside(r) ? in : out) = r;
+    }
+    return in;
 }
 
 // Coarsening chain: halve all dimensions while all are even and stay >= 2.

@@ -747,13 +747,23 @@ void orc_update_particles(const int n[3], const double plo[3], const double phi_
 
 /*
  * Largest double below hi whose cell index (x-lo)*dxi stays < n: the upper end
- * of the particle domain used by the periodic shift.
+ * of the particle domain used by the periodic shift.  Stepped down to where that
+ * is a few doubles away; bisected where hi is next to zero and it is not.
  */
 double orc_domain_rhi(double lo, double hi, int n) {
     double dxi = 1.0 / ((hi - lo) / (double)n);
     double r = nextafter(hi, -INFINITY);
-    while ((int)floor((r - lo) * dxi) >= n) r = nextafter(r, -INFINITY);
-    return r;
+    for (int k = 0; k < 64; ++k) {
+        if ((int)floor((r - lo) * dxi) < n) return r;
+        r = nextafter(r, -INFINITY);
+    }
+    double in = lo;
+    while (nextafter(in, r) < r) {
+        double mid = 0.5 * in + 0.5 * r;
+        if (!(mid > in && mid < r)) mid = nextafter(in, r);
+        if ((int)floor((mid - lo) * dxi) < n) in = mid; else r = mid;
+    }
+    return in;
 }
 
 /*

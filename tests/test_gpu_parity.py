@@ -267,6 +267,39 @@ def test_kick_wraps_like_redistribute(nyx, orc, golden):
         assert np.array_equal(vel[d], v2[d])
 
 
+# boxes that end at zero, or within round-off of it: the doubles below the upper end
+# are too dense there to step through
+@pytest.mark.parametrize("plo,phi_hi", [((-1.0,) * 3, (0.0,) * 3), ((-0.3, 0.0, -2.0), (-0.3 + 24 * 0.0125, 1.0, 0.0))])
+def test_box_that_ends_at_zero(nyx, orc, plo, phi_hi):
+    n = (24, 16, 16)
+    r = np.random.default_rng(12)
+    NP = 3000
+    ext = [phi_hi[d] - plo[d] for d in range(3)]
+    rhi = [orc.domain_rhi(plo[d], phi_hi[d], n[d]) for d in range(3)]
+    pos = [np.minimum(plo[d] + ext[d] * r.random(NP), rhi[d]) for d in range(3)]
+    for d in range(3):
+        pos[d][d] = rhi[d]
+        pos[d][3 + d] = plo[d]
+    vel = [ext[d] * r.standard_normal(NP) for d in range(3)]
+    m = r.uniform(0.5, 1.5, NP)
+    pot = r.standard_normal((n[2], n[1], n[0]))
+    with ctx1(nyx, n, plo, phi_hi) as c:
+        c.upload(0, pos, vel, m=m)
+        rho = c.assign_density()
+        c.set_phi(pot)
+        c.move_kick_drift(0.01, 1.0, 1.0)
+        c.redistribute()
+        gpos, gvel = c.download()
+    assert relmax(rho, orc.deposit(n, plo, phi_hi, *pos, m=m)) <= 1e-13
+    p2 = [a.copy() for a in pos]
+    v2 = [a.copy() for a in vel]
+    orc.update_particles(n, plo, phi_hi, p2, v2, orc.grav_vector(n, plo, phi_hi, pot), 0.01, 1.0, 1.0, 1)
+    orc.enforce_periodic(n, plo, phi_hi, p2)
+    for d in range(3):
+        assert np.array_equal(gpos[d], p2[d])
+        assert np.array_equal(gvel[d], v2[d])
+
+
 @pytest.mark.parametrize("tile", [(8, 8, 8), (16, 8, 4)])
 def test_tiled_kick_equals_global_kick(nyx, tile):
     # clustered particles (heavy tiles split into chunks), several steps so that

@@ -54,6 +54,20 @@ def test_periodic_wrap(orc):
     assert x[5] == 0.999999999
 
 
+# The upper end kept by the periodic shift is the last double whose cell index is
+# inside; a box that ends at zero or within round-off of it has its neighbours
+# 1e-33 or less apart there.
+@pytest.mark.parametrize("lo,hi,n", [(0.0, 1.0, 8), (-1.0, 0.0, 16), (-0.3, -0.3 + 24 * 0.0125, 24), (-0.3, 0.05, 28),
+                                     (2.0, 2.5, 10), (-3.0, 1e-300, 12), (-7.0, -5e-324, 6)])
+def test_domain_end_is_the_last_inside(orc, lo, hi, n):
+    dxi = 1.0 / ((hi - lo) / n)
+    rhi = orc.domain_rhi(lo, hi, n)
+    up = np.nextafter(rhi, np.inf)
+    assert lo < rhi < hi
+    assert np.floor((rhi - lo) * dxi) < n
+    assert up == hi or np.floor((up - lo) * dxi) >= n
+
+
 def _two_body(orc):
     # two equal masses, mirror symmetric about the box centre
     n = (16, 16, 16)
