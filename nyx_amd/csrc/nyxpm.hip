@@ -1312,7 +1312,9 @@ int choose_chunk(const nyxpm_ctx* c, long long slots) {
 }
 
 // Accumulators of n split tiles and their counters behind them, one allocation, zeroed
-// (2 u64 words per LDS cell: 22 KB a tile of 16x8x8).
+// (2 u64 words per LDS cell: 22 KB a tile of 16x8x8).  These zeros are the only plain
+// stores to them, a launch of its own before any deposit: from then on split_combine()
+// touches them by device-scope atomics alone, which needs no fence and leaves them zero.
 int alloc_split(nyxpm_ctx* c, long long n, unsigned long long** acc, int** done) {
     const size_t words = (size_t)n * split_words(c), all = words + (size_t)(n + 1) / 2;
     int rc = dalloc(c, acc, all);
